@@ -182,6 +182,7 @@ extern "C" int vsc_pipeline_create(int width, int height, const vsc_pipeline_cfg
         vsc_pipeline_destroy(p);
         return rc;
     }
+    if (cfg->overlap) stream_set_shared(p->stab);
     const size_t lo_b = (size_t)p->Wd * p->Hd * 2 * 4, hi_b = (size_t)width * height * 2 * 4;
     for (int i = 0; i < 2 * p->sets && !rc; ++i) rc = dalloc(reinterpret_cast<void**>(&p->lo[i / 2][i % 2]), lo_b);
     if (here)

@@ -408,6 +408,11 @@ extern "C" int vsc_server_open(vsc_server* sv, int width, int height, int* id)
     st = Stream();
     st.W = width; st.H = height;
     int rc = vsc_pipeline_create(width, height, &sv->cfg.form, &st.pipe);
+    if (!rc) {
+        vsc_stream* stab = nullptr;
+        rc = vsc_pipeline_stream(st.pipe, &stab);
+        stream_set_shared(stab);   // many streams' frames run side by side
+    }
     if (!rc && !sv->ups_params.empty() && sv->cfg.form.upsample == 1 && sv->cfg.form.downscale > 1)
         rc = vsc_pipeline_set_upsampler_params(st.pipe, sv->ups_params.data());
     if (!rc) {

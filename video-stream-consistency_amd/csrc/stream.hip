@@ -6,6 +6,8 @@
 #include "vsc_internal.h"
 
 #include <algorithm>
+#include <cmath>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -27,6 +29,13 @@ struct vsc_stream {
     bool has_last = false;
     void* block = nullptr;
     size_t bytes = 0;
+    // resident solver (resident.hip): control words, the host word that tells
+    // of a launch the device could not hold at once, and how many frames the
+    // blocked solver takes after one
+    unsigned* ctl = nullptr;
+    volatile unsigned* note = nullptr;
+    int cus = 0, skip = 0, backoff = 0;
+    bool shared = false;
     // staged (per-stage reference sequence) images, allocated on first use
     void* staged_block = nullptr;
     float* st[32] = {};
@@ -65,6 +74,37 @@ size_t footprint(int W, int H, int fw, int fh, int* nlev_out = nullptr)
 
 inline View pl(float* d, int w, int h) { return planar(d, w, h, 3); }
 
+// Pinned host words for the streams' notes: one page for the process, 16 words
+// apart; a stream that finds none left does without the resident solver.
+struct Notes {
+    static constexpr int N = 256, STRIDE = 16;
+    std::mutex m;
+    unsigned* page = nullptr;
+    bool used[N] = {};
+    volatile unsigned* take()
+    {
+        std::lock_guard<std::mutex> hold(m);
+        if (!page && hipHostMalloc(reinterpret_cast<void**>(&page), N * STRIDE * 4, hipHostMallocPortable) != hipSuccess) {
+            page = nullptr;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        for (int i = 0; i < N; ++i)
+            if (!used[i]) {
+                used[i] = true;
+                page[i * STRIDE] = 0u;
+                return page + i * STRIDE;
+            }
+        return nullptr;
+    }
+    void give(volatile unsigned* w)
+    {
+        std::lock_guard<std::mutex> hold(m);
+        used[(w - page) / STRIDE] = false;
+    }
+};
+Notes notes;
+
 }  // namespace
 
 extern "C" size_t vsc_stream_footprint(int width, int height, int flow_width, int flow_height)
@@ -89,7 +129,8 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
     s->fh = flow_height;
     s->bytes = footprint(width, height, flow_width, flow_height, &s->nlev);
     level_dims(width, height, s->lw, s->lh);
-    int rc = check_hip(hipMalloc(&s->block, s->bytes), "vsc_stream_create");
+    // (the solver's control words stand behind the carved pieces)
+    int rc = check_hip(hipMalloc(&s->block, s->bytes + RESIDENT_CTL_BYTES), "vsc_stream_create");
     if (rc) {
         delete s;
         return rc;
@@ -120,6 +161,18 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
         delete s;
         return set_error(VSC_E_INVALID, "vsc_stream_create: internal error: carve does not match the footprint");
     }
+    // without these the blocked solver runs alone
+    int dev = 0;
+    static const std::vector<unsigned> zeros(RESIDENT_CTL_BYTES / 4, 0u);
+    unsigned* ctl = reinterpret_cast<unsigned*>(static_cast<char*>(s->block) + s->bytes);
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+        hipMemcpy(ctl, zeros.data(), RESIDENT_CTL_BYTES, hipMemcpyHostToDevice) == hipSuccess) {
+        s->ctl = ctl;
+        s->note = notes.take();
+    } else {
+        (void)hipGetLastError();
+    }
     *out = s;
     return VSC_OK;
 }
@@ -133,6 +186,7 @@ extern "C" int vsc_stream_destroy(vsc_stream* s)
         int rc2 = check_hip(hipFree(s->block), "vsc_stream_destroy");
         if (!rc) rc = rc2;
     }
+    if (s->note) notes.give(s->note);   // hipFree has waited for the device
     delete s;
     return rc;
 }
@@ -201,6 +255,11 @@ int check_params(const vsc_stream* s, const vsc_params& p)
 // (NULL = defaults) valid for this stream, and a previous frame set.
 namespace vsc {
 
+void stream_set_shared(vsc_stream* s)
+{
+    if (s) s->shared = true;
+}
+
 int stream_params_check(const vsc_stream* s, const vsc_params* params)
 {
     if (!s) return set_error(VSC_E_INVALID, "vsc_stab_frame: null stream");
@@ -243,21 +302,65 @@ int prepare_flows(vsc_stream* s, const vsc_frame_in* in, View* fwd, View* bwd, h
     return rc;
 }
 
-// Pyramid solve, levels L-1 .. 0 (videostabilizer.cpp:219-227) with the
-// temporally blocked solver.  Level j initial solution: O[j][0] (level L-1)
-// or bilinear(up) of the level above.  Returns the index of O[0] holding the
-// result.
-int solve_pyramid(vsc_stream* s, int L, const vsc_params& p, int fma, hipStream_t st, int* final_idx)
+// Whether this frame's levels may use the resident solver: not beside other
+// work on purpose, not under capture (its launches take turns across streams),
+// not on a stream that leaves CUs out, and not for some frames after the device
+// could not hold a launch at once (64, doubled each time up to 4096).
+bool resident_frame(vsc_stream* s, const vsc_params& p, hipStream_t st)
 {
-    int cur = 0;
+    if (!s->note || s->shared || !std::isfinite(p.mom_fac)) return false;
+    if (*s->note) {
+        *s->note = 0u;
+        s->backoff = std::min(4096, std::max(64, 2 * s->backoff));
+        s->skip = s->backoff;
+    }
+    if (s->skip > 0) {
+        --s->skip;
+        return false;
+    }
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+    uint32_t mask[32] = {};
+    if (st && hipExtStreamGetCUMask(st, 32, mask) == hipSuccess) {
+        int n = 0;
+        for (uint32_t m : mask) n += __builtin_popcount(m);
+        if (n > 0 && n < s->cus) return false;
+    }
+    return true;
+}
+
+// The buffer of O[j] in which level j starts.  The blocked solver starts in 0
+// and swaps at every launch; a resident level 0 starts where its one swap ends
+// in the same buffer, so that the two forms may alternate between frames and
+// in captured graphs.
+int level_start(const vsc_stream* s, int j, int iters, int fma, bool resident)
+{
+    if (!resident || j > 0) return 0;
+    const int halo = plan_consist_blocked(s->lw[0], s->lh[0], iters, fma).halo;
+    return ((iters + halo - 1) / halo & 1) ^ 1;
+}
+
+// Pyramid solve, levels L-1 .. 0 (videostabilizer.cpp:219-227): a level that
+// fits the chip with the resident solver, others with the temporally blocked
+// one.  Level j initial solution: O[j][level_start] (level L-1) or bilinear(up)
+// of the level above.  Returns the index of O[0] holding the result.
+int solve_pyramid(vsc_stream* s, int L, const vsc_params& p, int fma, const ResidentPlan* res, const bool* resident,
+                  hipStream_t st, int* final_idx)
+{
     for (int j = L - 1; j >= 0; --j) {
         const int w = s->lw[j], h = s->lh[j];
         const int iters = p.num_iter / (j + 1);
-        int rc;
+        int rc, cur = level_start(s, j, iters, fma, resident[j]);
         if (j != L - 1) {
-            cur = 0;
-            rc = launch_bilinear(pl(s->O[j + 1][*final_idx], s->lw[j + 1], s->lh[j + 1]), pl(s->O[j][0], w, h), st);
+            rc = launch_bilinear(pl(s->O[j + 1][*final_idx], s->lw[j + 1], s->lh[j + 1]), pl(s->O[j][cur], w, h), st);
             if (rc) return rc;
+        }
+        if (resident[j]) {
+            ResidentLevel l{s->L[j], s->Wt[j], s->A[j], {s->O[j][cur], s->O[j][cur ^ 1]}, {s->U[j][0], s->U[j][1]},
+                            s->P[j], w, h, iters, p.step_size, p.mom_fac, s->ctl, const_cast<unsigned*>(s->note)};
+            if ((rc = launch_resident(l, res[j], st))) return rc;
+            *final_idx = cur ^ 1;
+            continue;
         }
         const BlockedPlan plan = plan_consist_blocked(w, h, iters, fma);
         int ucur = 0;
@@ -338,12 +441,17 @@ int frame_fused(vsc_stream* s, const vsc_frame_in* in, const vsc_params& p, uint
     if (fma && !direct)
         for (int j = 0; j < L; ++j)
             if ((rc = launch_fma_consts(s->L[j], s->A[j], s->Wt[j], s->lw[j], s->lh[j], p.step_size, st))) return rc;
+    ResidentPlan rplan[VSC_MAX_LEVELS];
+    bool resident[VSC_MAX_LEVELS] = {};
+    if (resident_frame(s, p, st))
+        for (int j = 0; j < L; ++j) resident[j] = plan_resident(s->lw[j], s->lh[j], p.num_iter / (j + 1), s->cus, fma, &rplan[j]);
     if (L == 1) {
         // single level: the solution starts at the processed frame (videostabilizer.cpp:209)
-        if ((rc = launch_copy_view(pl(s->P[0], W, H), pl(s->O[0][0], W, H), st))) return rc;
+        const int start = level_start(s, 0, p.num_iter, fma, resident[0]);
+        if ((rc = launch_copy_view(pl(s->P[0], W, H), pl(s->O[0][start], W, H), st))) return rc;
     }
     int fin = 0;
-    if ((rc = solve_pyramid(s, L, p, fma, st, &fin))) return rc;
+    if ((rc = solve_pyramid(s, L, p, fma, rplan, resident, st, &fin))) return rc;
     const View res = pl(s->O[0][fin], W, H);
     if (out_rgba && (rc = launch_to_rgba(res, out_rgba, st))) return rc;
     if (out_float && (rc = launch_copy_view(res, View{out_float, W, H, 3, 1, 3}, st))) return rc;
@@ -529,6 +637,17 @@ int stream_batch_frame(vsc_stream* s, const vsc_frame_in* in, const vsc_params* 
 }
 
 }  // namespace vsc
+
+// Diagnostic (no declaration in vsc.h): the stream's next resident launch is
+// given up as if the device could not hold it, so that the ticket form
+// computes its level.  Returns whether the stream has a resident solver.
+extern "C" int vsct_resident_give_up(vsc_stream* s, vsc_hip_stream stream)
+{
+    if (!s || !s->note) return 0;
+    static const unsigned one = 1u;
+    if (check_hip(hipMemcpyAsync(s->ctl, &one, 4, hipMemcpyHostToDevice, as_stream(stream)), "vsct_resident_give_up")) return 0;
+    return check_hip(hipStreamSynchronize(as_stream(stream)), "vsct_resident_give_up") ? 0 : 1;
+}
 
 extern "C" int vsc_stab_frame(vsc_stream* s, const vsc_frame_in* in, const vsc_params* params, uint8_t* out_rgba,
                               float* out_float, int mode, vsc_hip_stream stream)

@@ -238,6 +238,33 @@ int launch_consist_blocked(const float* lapP, const float* A, const float* Wt, c
                            float mom, int fma, const BlockedPlan& plan, hipStream_t s, int store_u = 1);
 // in place: Wt <- cnt + Wt, L <- step*fma(-Wt, A, L) (the FMA-form constants of a planar level)
 int launch_fma_consts(float* L, const float* A, float* Wt, int W, int H, float step, hipStream_t s);
+// One pyramid level solved with its tiles resident on the chip (resident.hip);
+// K, Q, A: k, q and unused (FMA form) or lapP, w, A (reference order).  O[0]
+// holds the initial solution, O[1] receives the result; U and P are scratch of
+// a level's size; ctl: RESIDENT_CTL_BYTES of device memory of the stream's
+// own, zero at rest.
+constexpr size_t RESIDENT_CTL_BYTES = 66 << 10;
+struct ResidentPlan {
+    int variant, h, nx, ny;
+};
+struct ResidentLevel {
+    const float* K;
+    const float* Q;
+    const float* A;
+    float* O[2];
+    float* U[2];
+    float* P;
+    int W, H, iters;
+    float step, mom;
+    unsigned* ctl;
+    unsigned* note;   // pinned host word, set when the device could not hold the launch at once
+};
+// false when no tiling of the level fits `cus` compute units at once
+bool plan_resident(int W, int H, int iters, int cus, int fma, ResidentPlan* out);
+int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_t s);
+// a stream whose frames run beside other work on purpose (overlapped pipelines,
+// the server): its solver leaves CUs free between launches (blocked form only)
+void stream_set_shared(vsc_stream* s);
 int launch_to_rgba(View in, uint8_t* out, hipStream_t s);
 int launch_rgba_to_view(const uint8_t* in, View out, hipStream_t s);
 int launch_copy_view(View in, View out, hipStream_t s);
