@@ -24,6 +24,14 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t fo_u32x4
 // displacement on its diagonals.  Block: 4 rows x 32 pixels, 8 waves (row,
 // 16-pixel half); channel chunks of KC stream through LDS as straight 16-byte
 // copies (the tensors are already channels-last).
+//
+// A block computes DG of the 9 vertical displacements (blockIdx.z = item *
+// 9/DG + group): the channel chunks are a serial chain of loads and products,
+// and with all nine a block of the coarse levels (1 to 36 blocks) walks it with
+// 18 products a chunk.  Groups of three cut the products, the staged rows (12 to
+// 6) and the registers by a third, so that chunks are fetched two ahead.
+// (Mean of the four levels, two pairs: BF16 960x576 12.7 us a launch with whole
+// blocks, 9.0 in thirds; FP32 640x384 28.7 and 15.5.)
 // ---------------------------------------------------------------------------
 template <int EK> struct CorrK;
 template <> struct CorrK<EK_F32> { static constexpr int KC = 16; };
@@ -54,9 +62,10 @@ __device__ inline fo_f32x4 corr_mma(const fo_u32x4& a, const fo_u32x4& b, fo_f32
 // BFMM (FP32 storage only): the FP32 features are rounded to BF16 as they are
 // staged and multiplied on the BF16 MFMA (FP32 accumulation): the BF16 cost
 // volume of an otherwise FP32 network.
-template <int EK, bool BFMM>
+template <int EK, bool BFMM, int DG>
 __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
 {
+    static_assert(DG == 9 || DG == 3, "all displacements, or a third of them");
     static_assert(!BFMM || EK == EK_F32, "BF16 products of FP32 storage only");
     using E = Elem<EK>;
     using T = typename E::T;
@@ -64,10 +73,10 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
     using M = typename Elem<MK>::T;
     constexpr int VEC = E::VEC, KC = CorrK<MK>::KC, KV = KC / VEC;
     constexpr int MVEC = Elem<MK>::VEC, ROW = KC + MVEC;
-    constexpr int RR = 4, RP = 32, HALO = 4, BR = RR + 2 * HALO, BP = RP + 2 * HALO;
+    constexpr int RR = 4, RP = 32, HALO = 4, BR = RR + DG - 1, BP = RP + 2 * HALO;
     constexpr int NA = RR * RP * KV, NB = BR * BP * KV, NU = NA + NB, RU = (NU + 511) / 512;
     constexpr int OPX = 88 / VEC;                       // output vectors per pixel (81 + 7 zeros)
-    constexpr int SROW = 89;                            // stage floats per pixel (odd: fewer conflicts)
+    constexpr int SROW = 9 * DG + (DG == 9 ? 8 : 0);   // stage floats per pixel (odd: fewer conflicts)
     constexpr int OPER_BYTES = (RR * RP + BR * BP) * ROW * (int)sizeof(M);
     constexpr int STAGE_BYTES = RR * RP * SROW * 4;
     constexpr int LDS = OPER_BYTES > STAGE_BYTES ? OPER_BYTES : STAGE_BYTES;
@@ -76,20 +85,23 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
     M* sB = sA + RR * RP * ROW;
     float* stage = reinterpret_cast<float*>(lds);
 
-    const int n = blockIdx.z, h0 = blockIdx.y * RR, w0 = blockIdx.x * RP;
+    const int n = blockIdx.z / (9 / DG), d0 = blockIdx.z % (9 / DG) * DG;   // displacement rows d0 .. d0+DG-1
+    const int h0 = blockIdx.y * RR, w0 = blockIdx.x * RP;
+    const bool copy_f1 = a.f1_c0 >= 0 && d0 == 0;
     const T* f1 = static_cast<const T*>(a.f1[n]);
     const T* f2 = static_cast<const T*>(a.f2[n]);
     const int tid = threadIdx.x, q = tid / 64, lane = tid % 64;
     const int qr = q >> 1, seg = q & 1, l16 = lane % 16, lg = lane / 16;
 
-    fo_f32x4 acc[9][2];
+    fo_f32x4 acc[DG][2];
 #pragma unroll
-    for (int d = 0; d < 9; ++d)
+    for (int d = 0; d < DG; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t) acc[d][t] = fo_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    fo_u32x4 rg[RU];
-    auto fetch = [&](int c0) {
+    constexpr int DEPTH = DG == 9 ? 1 : 2;
+    fo_u32x4 regs[DEPTH][RU];
+    auto fetch = [&](int c0, fo_u32x4 (&rg)[RU]) {
 #pragma unroll
         for (int k = 0; k < RU; ++k) {
             const int u = tid + 512 * k;
@@ -101,13 +113,13 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
                     v = *reinterpret_cast<const fo_u32x4*>(f1 + ((long long)gh * a.W + gw) * a.cs1 + ch);
                     // the decoder's concatenation takes f1 beside the cost volume
                     // (pwcnet.py:578): every block stages its own pixels' f1 once
-                    if (a.f1_c0 >= 0)
+                    if (copy_f1)
                         *reinterpret_cast<fo_u32x4*>(static_cast<T*>(a.out) +
                                                      (((long long)n * a.H + gh) * a.W + gw) * a.ocs + a.f1_c0 + ch) = v;
                 }
             } else if (u < NU) {
                 const int ub = u - NA, p = ub / KV, cv = ub % KV, r = p / BP, x = p % BP;
-                const int gh = h0 - HALO + r, gw = w0 - HALO + x, ch = c0 + cv * VEC;
+                const int gh = h0 - HALO + d0 + r, gw = w0 - HALO + x, ch = c0 + cv * VEC;
                 if (gh >= 0 && gh < a.H && gw >= 0 && gw < a.W && ch < a.C)
                     v = *reinterpret_cast<const fo_u32x4*>(f2 + ((long long)gh * a.W + gw) * a.cs2 + ch);
             }
@@ -115,8 +127,7 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
         }
     };
 
-    fetch(0);
-    for (int c0 = 0; c0 < a.C; c0 += KC) {
+    auto chunk = [&](int c0, fo_u32x4 (&rg)[RU]) {
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < RU; ++k) {
@@ -135,10 +146,10 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
             }
         }
         __syncthreads();
-        if (c0 + KC < a.C) fetch(c0 + KC);
+        if (c0 + DEPTH * KC < a.C) fetch(c0 + DEPTH * KC, rg);
         const fo_u32x4 fa = *reinterpret_cast<const fo_u32x4*>(&sA[(qr * RP + 16 * seg + l16) * ROW + lg * (KC / 4)]);
 #pragma unroll
-        for (int d = 0; d < 9; ++d) {
+        for (int d = 0; d < DG; ++d) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const fo_u32x4 fb = *reinterpret_cast<const fo_u32x4*>(
@@ -146,12 +157,20 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
                 acc[d][t] = corr_mma<MK>(fa, fb, acc[d][t]);
             }
         }
+    };
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i)
+        if (i * KC < a.C) fetch(i * KC, regs[i]);
+    for (int c0 = 0; c0 < a.C; c0 += DEPTH * KC) {
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i)
+            if (c0 + i * KC < a.C) chunk(c0 + i * KC, regs[i]);
     }
 
     // diagonals -> stage[row*32 + px][plane]
     __syncthreads();
 #pragma unroll
-    for (int d = 0; d < 9; ++d)
+    for (int d = 0; d < DG; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -162,6 +181,18 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
             }
     __syncthreads();
     T* out = static_cast<T*>(a.out) + (long long)n * a.H * a.W * a.ocs;
+    if constexpr (DG != 9) {
+        // this group's channels, and the zero channels 81 .. 87 with the last group
+        const int nc = 9 * DG + (d0 + DG == 9 ? 7 : 0);
+        for (int e = tid; e < RR * RP * nc; e += 512) {
+            const int p = e / nc, pl = e - p * nc, r = p / RP, x = p % RP;
+            const int h = h0 + r, w = w0 + x;
+            if (h >= a.H || w >= a.W) continue;
+            const float g = pl < 9 * DG ? stage[p * SROW + pl] : 0.0f;
+            out[((long long)h * a.W + w) * a.ocs + d0 * 9 + pl] = E::st(g > 0.0f ? g : g * 0.1f);
+        }
+        return;
+    }
     for (int e = tid; e < RR * RP * OPX; e += 512) {
         const int p = e / OPX, v = e % OPX, r = p / RP, x = p % RP;
         const int h = h0 + r, w = w0 + x;
@@ -194,10 +225,13 @@ int launch_corr_nhwc(int ek, const void* const* f1, const void* const* f2, int c
     a.cs1 = cs1; a.cs2 = cs2; a.C = C; a.H = H; a.W = W; a.out = out; a.ocs = ocs;
     a.f1_c0 = f1_c0;
     if (f1_c0 >= 0 && f1_c0 + C > ocs) return set_error(VSC_E_INVALID, "corr nhwc: f1 copy outside the pixel");
-    dim3 grid((W + 31) / 32, (H + 3) / 4, N);
-    if (ek == EK_BF16) hipLaunchKernelGGL((k_corr_nhwc<EK_BF16, false>), grid, dim3(512), 0, s, a);
-    else if (bf16_products) hipLaunchKernelGGL((k_corr_nhwc<EK_F32, true>), grid, dim3(512), 0, s, a);
-    else hipLaunchKernelGGL((k_corr_nhwc<EK_F32, false>), grid, dim3(512), 0, s, a);
+    // thirds of the displacements while whole blocks would not give every CU two
+    const bool thirds = (long long)((W + 31) / 32) * ((H + 3) / 4) * N < 512;
+    dim3 grid((W + 31) / 32, (H + 3) / 4, thirds ? 3 * N : N);
+    auto go = [&](auto whole, auto third) { hipLaunchKernelGGL(thirds ? third : whole, grid, dim3(512), 0, s, a); };
+    if (ek == EK_BF16) go(k_corr_nhwc<EK_BF16, false, 9>, k_corr_nhwc<EK_BF16, false, 3>);
+    else if (bf16_products) go(k_corr_nhwc<EK_F32, true, 9>, k_corr_nhwc<EK_F32, true, 3>);
+    else go(k_corr_nhwc<EK_F32, false, 9>, k_corr_nhwc<EK_F32, false, 3>);
     return check_launch("corr nhwc");
 }
 
