@@ -307,8 +307,27 @@ __global__ void k_conv_finalize(ConvArgs a, int parts)
     if (a.out2) static_cast<typename Elem<EK>::T*>(a.out2)[pix * a.out2_cs + a.out2_c0 + co] = Elem<EK>::st(x);
 }
 
+// Parts a layer's channel loop is split into (1: unsplit), given its blocks per
+// batch item: when the grid leaves most CUs idle (FP32: under 128 blocks per
+// item; 16-bit: under 32, where the partial-sum traffic and the finalize launch
+// cost more than idle CUs down to that size, as measured on 1080p frames) and
+// the caller provided room for the partial sums.  The split depends on one batch
+// item's geometry and the room per item only, so an item's result has the same
+// bits alone and in a batch of any size.
+template <int EK>
+static int conv_parts(const ConvArgs& a, long long item_blocks, int chunks)
+{
+    if (!a.partial || chunks < 2 || item_blocks >= (EK == EK_F32 ? 128 : 32)) return 1;
+    const long long item_stride = (long long)a.Ho * a.Wo * a.Cout;
+    int parts = (int)std::min<long long>(chunks, (256 + item_blocks - 1) / item_blocks);
+    parts = (int)std::min<long long>(parts, a.part_stride / std::max<long long>(item_stride, 1));
+    if (parts < 2) return 1;
+    const int cpp = (chunks + parts - 1) / parts;
+    return (chunks + cpp - 1) / cpp;
+}
+
 template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
-static void conv_go(const ConvArgs& a, hipStream_t s)
+static void conv_go(const ConvArgs& a, int split_nt, hipStream_t s)
 {
     constexpr int KC = KCX;
     const int ps = a.pstep;
@@ -318,24 +337,10 @@ static void conv_go(const ConvArgs& a, hipStream_t s)
     b.tiles_x = (ws + 15) / 16;
     b.ctiles = (a.Cout + NT - 1) / NT;
     const int chunks = (a.Cin + KC - 1) / KC;
-    // split the channel loop when the grid leaves most CUs idle (FP32: under
-    // 128 blocks per item; 16-bit: under 32, where the partial-sum traffic
-    // and the finalize launch cost more than idle CUs down to that size, as
-    // measured on 1080p frames) and the caller provided room for the partial
-    // sums.  The split depends on one batch item's geometry and the room per
-    // item only, so an item's result has the same bits alone and in a batch
-    // of any size.
-    const long long item_blocks = (long long)b.tiles_x * b.tiles_y * ps * ps * b.ctiles;
-    const long long item_stride = (long long)a.Ho * a.Wo * a.Cout;
-    const long long stride = item_stride * a.N;
-    int parts = 1;
-    if (a.partial && chunks > 1 && item_blocks < (EK == EK_F32 ? 128 : 32)) {
-        parts = (int)std::min<long long>(chunks, (256 + item_blocks - 1) / item_blocks);
-        parts = (int)std::min<long long>(parts, a.part_stride / std::max<long long>(item_stride, 1));
-        if (parts < 2) parts = 1;
-    }
+    const long long item_px = (long long)b.tiles_x * b.tiles_y * ps * ps;
+    const long long stride = (long long)a.Ho * a.Wo * a.Cout * a.N;
+    int parts = conv_parts<EK>(a, item_px * ((a.Cout + split_nt - 1) / split_nt), chunks);
     b.cpp = (chunks + parts - 1) / parts;
-    parts = (chunks + b.cpp - 1) / b.cpp;
     b.partial = parts > 1 ? a.partial : nullptr;
     b.part_stride = stride;
     dim3 grid(b.tiles_x * b.tiles_y * ps * ps, b.ctiles * parts, a.N);
@@ -345,11 +350,11 @@ static void conv_go(const ConvArgs& a, hipStream_t s)
 }
 
 template <int EK, int EKO, int S, int NT, int KCX>
-static void conv_mr(const ConvArgs& a, int mr, hipStream_t s)
+static void conv_mr(const ConvArgs& a, int mr, int split_nt, hipStream_t s)
 {
-    if (mr == 4) conv_go<EK, EKO, S, NT, (S == 1 ? 4 : 2), 4, KCX>(a, s);
-    else if (mr == 2) conv_go<EK, EKO, S, NT, 2, 4, KCX>(a, s);
-    else conv_go<EK, EKO, S, NT, 1, 4, KCX>(a, s);
+    if (mr == 4) conv_go<EK, EKO, S, NT, (S == 1 ? 4 : 2), 4, KCX>(a, split_nt, s);
+    else if (mr == 2) conv_go<EK, EKO, S, NT, 2, 4, KCX>(a, split_nt, s);
+    else conv_go<EK, EKO, S, NT, 1, 4, KCX>(a, split_nt, s);
 }
 
 // Tile choice.  Channel tile: FP32 layers take the widest tile they fill (64,
@@ -373,20 +378,40 @@ static void conv_pick(const ConvArgs& a, hipStream_t s)
     if (S == 2 && mr > 2) mr = 2;
     constexpr int KC = ConvK<EK>::KC;
     if constexpr (EK == EK_F32) {
-        if (NTsel == 64) conv_mr<EK, EKO, S, 64, KC>(a, mr, s);
-        else if (NTsel == 32) conv_mr<EK, EKO, S, 32, KC>(a, mr, s);
-        else conv_mr<EK, EKO, S, 16, KC>(a, mr, s);
+        // Layers of 64-pixel tiles that would take 64-channel tiles: those are the
+        // cheapest a channel, but on a grid of a few blocks per CU the fullest
+        // CU decides (288 blocks are two on 32 of the 256 CUs), and 96 channels
+        // leave a quarter of two tiles empty.  So the width of least
+        // blocks-on-the-fullest-CU * (channels + 4).  (80x48 pixels, 2 items,
+        // 128 -> 128 channels: 46 us with 64 channels, 35 with 32; 256 -> 96: @F96@.)
+        // The split stays that of 64 channels, so the width leaves the bits alone.
+        int nt = NTsel;
+        if (NTsel == 64 && mr == 1) {
+            const long long item = (((a.Ho + ps - 1) / ps + 3) / 4) * (((a.Wo + ps - 1) / ps + 15) / 16) * (long long)ps * ps;
+            const long long parts = conv_parts<EK>(a, item * ntiles, (a.Cin + KC - 1) / KC);
+            long long best = 1LL << 60;
+            for (int w = 64; w >= 16; w /= 2) {
+                const long long blocks = item * ((a.Cout + w - 1) / w) * parts * a.N, cost = (blocks + 255) / 256 * (w + 4);
+                if (cost < best) {
+                    best = cost;
+                    nt = w;
+                }
+            }
+        }
+        if (nt == 64) conv_mr<EK, EKO, S, 64, KC>(a, mr, NTsel, s);
+        else if (nt == 32) conv_mr<EK, EKO, S, 32, KC>(a, mr, NTsel, s);
+        else conv_mr<EK, EKO, S, 16, KC>(a, mr, NTsel, s);
     } else {
         // layers with 8 or 16 input channels (the image and the first feature
         // level) stage chunks of that width
         if (NTsel == 32) {
-            if (a.Cin <= 8) conv_mr<EK, EKO, S, 32, 8>(a, mr, s);
-            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 32, 16>(a, mr, s);
-            else conv_mr<EK, EKO, S, 32, KC>(a, mr, s);
+            if (a.Cin <= 8) conv_mr<EK, EKO, S, 32, 8>(a, mr, NTsel, s);
+            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 32, 16>(a, mr, NTsel, s);
+            else conv_mr<EK, EKO, S, 32, KC>(a, mr, NTsel, s);
         } else {
-            if (a.Cin <= 8) conv_mr<EK, EKO, S, 16, 8>(a, mr, s);
-            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 16, 16>(a, mr, s);
-            else conv_mr<EK, EKO, S, 16, KC>(a, mr, s);
+            if (a.Cin <= 8) conv_mr<EK, EKO, S, 16, 8>(a, mr, NTsel, s);
+            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 16, 16>(a, mr, NTsel, s);
+            else conv_mr<EK, EKO, S, 16, KC>(a, mr, NTsel, s);
         }
     }
 }
