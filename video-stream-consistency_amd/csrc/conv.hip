@@ -383,7 +383,8 @@ static void conv_pick(const ConvArgs& a, hipStream_t s)
         // CU decides (288 blocks are two on 32 of the 256 CUs), and 96 channels
         // leave a quarter of two tiles empty.  So the width of least
         // blocks-on-the-fullest-CU * (channels + 4).  (80x48 pixels, 2 items,
-        // 128 -> 128 channels: 46 us with 64 channels, 35 with 32; 256 -> 96: @F96@.)
+        // 128 -> 128 channels: 46 us with 64 channels, 35 with 32;
+        // 256 -> 96: 52 us with 64, 40 with 32.)
         // The split stays that of 64 channels, so the width leaves the bits alone.
         int nt = NTsel;
         if (NTsel == 64 && mr == 1) {
