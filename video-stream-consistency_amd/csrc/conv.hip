@@ -49,7 +49,9 @@ struct ConvArgs {
     // split over input channels: blockIdx.y = part * ctiles + channel tile; part p
     // covers chunks [p*cpp, (p+1)*cpp) and writes raw FP32 sums to
     // partial + p*part_stride (k_conv_finalize adds them in part order)
-    int ctiles, cpp;
+    // flush > 0 (FP32, 64-pixel tiles): an unsplit layer that keeps a split's order
+    // of sums: every `flush` chunks the accumulators are added to the total
+    int ctiles, cpp, flush;
     float* partial;
     long long part_stride;
 };
@@ -99,7 +101,7 @@ __device__ inline void conv_load4(const void* src, long long off, float v[4], in
     for (int r = 0; r < 4; ++r) v[r] += (r < nvalid) ? E::ld(p[r]) : 0.0f;
 }
 
-template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
+template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX, bool FLUSH>
 __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 {
     using E = Elem<EK>;
@@ -241,6 +243,23 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d)
         if (cbeg + d * KC < cend) fetch(cbeg + d * KC, rp[d], rw[d]);
+    [[maybe_unused]] cv_f32x4 total[NT / 16][MR];
+    [[maybe_unused]] int left = a.flush;
+    auto add_up = [&]() {
+#pragma unroll
+        for (int i = 0; i < NT / 16; ++i)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                total[i][m] += acc[i][m];
+                acc[i][m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
+    if constexpr (FLUSH) {
+#pragma unroll
+        for (int i = 0; i < NT / 16; ++i)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) total[i][m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     for (int c0 = cbeg; c0 < cend; c0 += DEPTH * KC) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
@@ -249,7 +268,19 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
             stage(rp[d], rw[d]);
             if (cc + DEPTH * KC < cend) fetch(cc + DEPTH * KC, rp[d], rw[d]);
             compute();
+            if constexpr (FLUSH) {
+                if (--left == 0 || cc + KC >= cend) {
+                    add_up();
+                    left = a.flush;
+                }
+            }
         }
+    }
+    if constexpr (FLUSH) {
+#pragma unroll
+        for (int i = 0; i < NT / 16; ++i)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) acc[i][m] = total[i][m];
     }
 
     // epilogue: lane holds output channels nt0 + 16i + 4lg + r of pixel l16 of row q*MR+m
@@ -326,6 +357,17 @@ static int conv_parts(const ConvArgs& a, long long item_blocks, int chunks)
     return (chunks + cpp - 1) / cpp;
 }
 
+// Modelled time (us) of an FP32 layer of 64-pixel tiles, `blocks` blocks of `w`
+// channels before the split, `chunks` chunks in `parts` parts: a chunk costs
+// 0.042 us per channel + 4 of the fullest CU's blocks (its MFMAs) but at least
+// 0.8 us (its way through LDS), a split 5.5 us for the launch that adds the parts
+// (fitted on the layers of a 640x360 frame).
+static double conv_split_cost(long long blocks, int w, int chunks, int parts)
+{
+    const long long full = (blocks * parts + 255) / 256;
+    return ((chunks + parts - 1) / parts) * std::max(0.8, 0.042 * full * (w + 4)) + (parts > 1 ? 5.5 : 0.0);
+}
+
 template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
 static void conv_go(const ConvArgs& a, int split_nt, hipStream_t s)
 {
@@ -339,12 +381,22 @@ static void conv_go(const ConvArgs& a, int split_nt, hipStream_t s)
     const int chunks = (a.Cin + KC - 1) / KC;
     const long long item_px = (long long)b.tiles_x * b.tiles_y * ps * ps;
     const long long stride = (long long)a.Ho * a.Wo * a.Cout * a.N;
-    int parts = conv_parts<EK>(a, item_px * ((a.Cout + split_nt - 1) / split_nt), chunks);
+    const int parts = conv_parts<EK>(a, item_px * ((a.Cout + split_nt - 1) / split_nt), chunks);
     b.cpp = (chunks + parts - 1) / parts;
+    if constexpr (EK == EK_F32 && MR == 1) {
+        if (parts > 1 && conv_split_cost(item_px * b.ctiles * a.N, NT, chunks, 1) < conv_split_cost(item_px * b.ctiles * a.N, NT, chunks, parts)) {
+            b.flush = b.cpp;
+            b.cpp = chunks;
+            b.partial = nullptr;
+            dim3 grid(b.tiles_x * b.tiles_y * ps * ps, b.ctiles, a.N);
+            hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, true>), grid, dim3(64 * NW), 0, s, b);
+            return;
+        }
+    }
     b.partial = parts > 1 ? a.partial : nullptr;
     b.part_stride = stride;
     dim3 grid(b.tiles_x * b.tiles_y * ps * ps, b.ctiles * parts, a.N);
-    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX>), grid, dim3(64 * NW), 0, s, b);
+    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, false>), grid, dim3(64 * NW), 0, s, b);
     if (parts > 1)
         hipLaunchKernelGGL((k_conv_finalize<EK, EKO>), dim3((unsigned)((stride + 255) / 256)), dim3(256), 0, s, b, parts);
 }
@@ -378,22 +430,23 @@ static void conv_pick(const ConvArgs& a, hipStream_t s)
     if (S == 2 && mr > 2) mr = 2;
     constexpr int KC = ConvK<EK>::KC;
     if constexpr (EK == EK_F32) {
-        // Layers of 64-pixel tiles that would take 64-channel tiles: those are the
-        // cheapest a channel, but on a grid of a few blocks per CU the fullest
-        // CU decides (288 blocks are two on 32 of the 256 CUs), and 96 channels
-        // leave a quarter of two tiles empty.  So the width of least
-        // blocks-on-the-fullest-CU * (channels + 4).  (80x48 pixels, 2 items,
-        // 128 -> 128 channels: 46 us with 64 channels, 35 with 32;
-        // 256 -> 96: 52 us with 64, 40 with 32.)
-        // The split stays that of 64 channels, so the width leaves the bits alone.
+        // Layers of 64-pixel tiles: the widest channel tiles are the cheapest a
+        // channel, but on a grid of a few blocks per CU the fullest CU decides
+        // (288 blocks are two on 32 of the 256 CUs), 96 channels leave a quarter
+        // of two 64-channel tiles empty, and narrow tiles can do without a split.
+        // So the width of least modelled time, split or not.  (80x48 pixels, 2
+        // items, 128 -> 128 channels: 46 us with 64 channels, 31 with 16; 256 -> 96:
+        // 52 + 5 with 64 split, 37 with 16 unsplit.)  The order of sums is the
+        // widest tiles' split in every case, so the choice leaves the bits alone.
         int nt = NTsel;
-        if (NTsel == 64 && mr == 1) {
+        if (mr == 1) {
             const long long item = (((a.Ho + ps - 1) / ps + 3) / 4) * (((a.Wo + ps - 1) / ps + 15) / 16) * (long long)ps * ps;
-            const long long parts = conv_parts<EK>(a, item * ntiles, (a.Cin + KC - 1) / KC);
-            long long best = 1LL << 60;
-            for (int w = 64; w >= 16; w /= 2) {
-                const long long blocks = item * ((a.Cout + w - 1) / w) * parts * a.N, cost = (blocks + 255) / 256 * (w + 4);
-                if (cost < best) {
+            const int chunks = (a.Cin + KC - 1) / KC, parts = conv_parts<EK>(a, item * ntiles, chunks);
+            double best = 1e300;
+            for (int w = NTsel; w >= 16; w /= 2) {
+                const long long blocks = item * ((a.Cout + w - 1) / w) * a.N;
+                const double cost = std::min(conv_split_cost(blocks, w, chunks, 1), conv_split_cost(blocks, w, chunks, parts));
+                if (cost < best - 1e-9) {
                     best = cost;
                     nt = w;
                 }
