@@ -13,150 +13,141 @@ namespace vsc {
 // CPU op, correlation.cc:163-177: *dst = 0; *dst += v1*v2 for c = 0..C-1).
 //
 // A block owns a tile of 8 rows x 8*QX pixels of one image and DG of the
-// vertical displacements (a 576-thread block all 9; the small levels' tiles
-// spread them over 3 blocks of 3 waves).  Wave d handles vertical
-// displacement dy = d - MD; its lane (row, quad)
-// keeps QX pixels x (2*MD+1) horizontal displacements in registers (QX = 4
-// for large images: 12 f2 loads from LDS feed 36 multiply-adds; QX = 1 for
-// small pyramid levels, where parallelism matters more than reuse).  Channels
-// stream through LDS in chunks (8 channels for QX = 4, 32 for QX = 1): the f1 tile and the f2 tile (a
-// 4-pixel halo in x, the rows the block's displacements reach), zeros
-// outside the image (an out-of-range term of the
-// reference contributes nothing, and acc + (+-0) == acc for the accumulator
-// values that occur, so zero terms leave every bit unchanged).  Every thread
-// issues all its global loads of the next chunk before computing the current
-// one, so the chunk loop overlaps memory and arithmetic.  This staging replaces the reference's
-// channels-last rearrange kernels and their per-call cudaMalloc
-// (correlation_cuda.cu:32-95,365-370).  Each (dy, dx) output row segment of
-// 8*QX pixels is written contiguously.
+// vertical displacements (blockIdx.z = item * (P / DG) + group).  A wave takes
+// one vertical displacement and one of XS groups of horizontal ones; its lane
+// (row, group of QX pixels) keeps QX x P/XS sums in registers (QX = 4: 12 f2
+// values from LDS feed 36 multiply-adds).  Channels stream through LDS CC at a
+// time: the f1 tile and the f2 rows that the block's displacements reach (a
+// 4-pixel halo in x), zeros outside the image (acc + (+-0) == acc for the
+// values that occur, so zero terms leave every bit unchanged).
+//
+// Staging.  A thread owns one 4-pixel slot of the tiles for the whole call and
+// every CPT-th channel of it: its addresses are one pointer plus multiples of a
+// plane, and all loads of the next chunk are in flight during this one's sums.
+// The loads are 16 bytes wide whatever the alignment; a slot over the right edge
+// is read further left and shifted.  (One pixel a load with its own index
+// arithmetic took 4 us a chunk: 17x30x196 28.4 us, now 12.9; 480x272x32 34.9 us,
+// now 24.1, its multiplications and additions alone about 20.)  This staging
+// replaces the reference's channels-last rearrange kernels and their per-call
+// cudaMalloc (correlation_cuda.cu:32-95,365-370).  Output rows are written 4*QX
+// bytes a lane, again whatever the alignment (479x271x32: 115 us with 4-byte
+// stores where rows are not aligned, now 44).
 // ---------------------------------------------------------------------------
 static constexpr int CF_TH = 8, CF_HALO = 4;
-// vertical displacements per block of the 1-pixel tile (md = 4: three blocks
-// of 3 waves per tile; 1920x1088 pyramid 134.0 us against 141.3 us for one
-// block of 9 waves and 162.7 us for nine blocks of one wave)
-static constexpr int CF_DG1 = 3;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
-// DG: vertical displacements (waves) per block; the P of them are split over
-// P / DG blocks (blockIdx.z = item * (P / DG) + group), each staging only the
-// CF_TH + DG - 1 f2 rows its displacements read.
-template <int MD, bool LEGACY, int QX, int CC, int DG>
-__global__ __launch_bounds__(64 * DG) void k_corr_f32(const float* __restrict__ f1, const float* __restrict__ f2,
-                                                      float* __restrict__ out, int C, int H, int W)
+// CCT: channels of a chunk, rounded to what the threads take in whole passes.
+// Needs W >= 4.
+template <int MD, bool LEGACY, int QX, int DG, int XS, int CCT>
+__global__ __launch_bounds__(64 * DG * XS) void k_corr_f32(const float* __restrict__ f1, const float* __restrict__ f2,
+                                                           float* __restrict__ out, int C, int H, int W)
 {
-    constexpr int P = 2 * MD + 1;
-    constexpr int NTH = 64 * DG, G = DG >= P ? 1 : P / DG;
-    static_assert(DG >= P || P % DG == 0, "displacement groups of equal size");
-    constexpr int TW = 8 * QX;
-    constexpr int SW = TW + 2 * CF_HALO, SH = CF_TH + DG - 1;
-    // f2 row pitch: the 1-pixel tile's lanes read 8 rows x 8 consecutive
-    // pixels at once; a pitch of 24 floats puts those rows on distinct banks
-    // (16 would stack them on the same 16)
-    constexpr int SWP = QX == 1 ? 24 : SW;
-    constexpr int N1 = CC * CF_TH * TW, N2 = CC * SH * SW;
-    constexpr int L1 = (N1 + NTH - 1) / NTH, L2 = (N2 + NTH - 1) / NTH;
-    __shared__ __attribute__((aligned(16))) float s1[CC][CF_TH][TW];
-    __shared__ __attribute__((aligned(16))) float s2[CC][SH][SWP];
+    constexpr int P = 2 * MD + 1, XG = P / XS, G = DG > P ? 1 : P / DG;
+    static_assert(P % XS == 0 && (DG > P || P % DG == 0), "displacement groups of equal size");
+    constexpr int TW = 8 * QX, NTH = 64 * DG * XS, SH = CF_TH + (DG > P ? P : DG) - 1;
+    // f2 row pitch: the 1-pixel tile's lanes read 8 rows x 8 neighbouring
+    // pixels at once; 24 floats put those rows on distinct banks (16 would not)
+    constexpr int PITCH = QX == 1 ? 24 : TW + 2 * CF_HALO;
+    constexpr int S1 = TW / 4, S2 = S1 + 2 * CF_HALO / 4;
+    constexpr int N1 = CF_TH * S1, NS = N1 + S2 * SH;   // 4-pixel slots of a channel: f1 tile, both tiles
+    static_assert(NS <= NTH, "a slot each");
+    // channels of one pass of the threads, passes and channels of a chunk
+    constexpr int CPT = NTH / NS, K = CCT / CPT > 1 ? CCT / CPT : 1, CC = CPT * K;
+    __shared__ __attribute__((aligned(16))) float s1[CC][CF_TH * TW];
+    __shared__ __attribute__((aligned(16))) float s2[CC][SH * PITCH];
 
     const int n = blockIdx.z / G, dg = blockIdx.z % G;
     const int tid = threadIdx.x;
-    const int dl = tid / 64, d = dg * DG + dl, rem = tid % 64;   // local and global displacement row
-    const int row = rem / 8, quad = rem % 8;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
+    const int dl = wave / XS, x0 = (wave % XS) * XG;
+    const int d = dg * DG + dl;
+    const int row = lane / 8, px = lane % 8 * QX;
     const int w0 = blockIdx.x * TW, h0 = blockIdx.y * CF_TH;
     const long long HW = (long long)H * W;
-    const float* a = f1 + (long long)n * C * HW;
-    const float* b = f2 + (long long)n * C * HW;
 
-    float acc[QX][P];
+    const int slot = tid % NS, cl = tid / NS;
+    const bool in1 = slot < N1;
+    const int sr = in1 ? slot / S1 : (slot - N1) / S2, sq = in1 ? slot % S1 : (slot - N1) % S2;
+    const int gy = in1 ? h0 + sr : h0 - MD + dg * DG + sr;
+    const int gx = in1 ? w0 + 4 * sq : w0 - CF_HALO + 4 * sq;
+    const bool ok = cl < CPT && gy >= 0 && gy < H && gx >= 0 && gx < W;
+    const int xs = min(gx, W - 4), shift = gx - xs;     // a slot over the right edge is read further left and shifted
+    const float* src = (in1 ? f1 : f2) + ((long long)n * C + cl) * HW + (ok ? (long long)gy * W + xs : 0);
+    float* dst = in1 ? &s1[0][0] + cl * (CF_TH * TW) + sr * TW + 4 * sq
+                     : &s2[0][0] + cl * (SH * PITCH) + sr * PITCH + 4 * sq;
+    const int dpitch = CPT * (in1 ? CF_TH * TW : SH * PITCH);
+
+    f32x4u_t rg[K];
+    auto fetch = [&](int c0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            f32x4u_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (ok && c0 + cl + CPT * k < C)
+                v = *reinterpret_cast<const f32x4u_t*>(src + (long long)(c0 + CPT * k) * HW);
+            rg[k] = v;
+        }
+    };
+    float acc[QX][XG];
 #pragma unroll
     for (int x = 0; x < QX; ++x)
 #pragma unroll
-        for (int k = 0; k < P; ++k) acc[x][k] = 0.0f;
-
-    // chunk staging: global loads from clamped addresses into registers (all
-    // in flight together), LDS stores after the previous chunk's compute
-    float r1[L1], r2[L2];
-    auto load_chunk = [&](int c0) {
-#pragma unroll
-        for (int k = 0; k < L1; ++k) {
-            const int e = tid + NTH * k;
-            const int x = e % TW, r = (e / TW) % CF_TH, c = e / (TW * CF_TH);
-            const int gh = min(h0 + r, H - 1), gw = min(w0 + x, W - 1), gc = min(c0 + c, C - 1);
-            const bool ok = e < N1 && c0 + c < C && h0 + r < H && w0 + x < W;
-            const float v = a[gc * HW + (long long)gh * W + gw];
-            r1[k] = ok ? v : 0.0f;
-        }
-#pragma unroll
-        for (int k = 0; k < L2; ++k) {
-            const int e = tid + NTH * k;
-            const int x = e % SW, r = (e / SW) % SH, c = e / (SW * SH);
-            const int ghr = h0 - MD + dg * DG + r, gwr = w0 - CF_HALO + x;
-            const int gh = min(max(ghr, 0), H - 1), gw = min(max(gwr, 0), W - 1), gc = min(c0 + c, C - 1);
-            const bool ok = e < N2 && c0 + c < C && ghr >= 0 && ghr < H && gwr >= 0 && gwr < W;
-            const float v = b[gc * HW + (long long)gh * W + gw];
-            r2[k] = ok ? v : 0.0f;
-        }
-    };
-    load_chunk(0);
+        for (int k = 0; k < XG; ++k) acc[x][k] = 0.0f;
+    fetch(0);
     for (int c0 = 0; c0 < C; c0 += CC) {
         __syncthreads();
+        if (cl < CPT) {
 #pragma unroll
-        for (int k = 0; k < L1; ++k) {
-            const int e = tid + NTH * k;
-            if (e < N1) (&s1[0][0][0])[e] = r1[k];
-        }
-#pragma unroll
-        for (int k = 0; k < L2; ++k) {
-            const int e = tid + NTH * k;
-            if (e < N2) {
-                if constexpr (SWP == SW) (&s2[0][0][0])[e] = r2[k];
-                else s2[e / (SW * SH)][(e / SW) % SH][e % SW] = r2[k];
+            for (int k = 0; k < K; ++k) {
+                f32x4u_t v = rg[k];
+                if (shift & 1) v = f32x4u_t{v.y, v.z, v.w, 0.0f};
+                if (shift & 2) v = f32x4u_t{v.z, v.w, 0.0f, 0.0f};
+                *reinterpret_cast<f32x4_t*>(dst + k * dpitch) = __builtin_bit_cast(f32x4_t, v);
             }
         }
         __syncthreads();
-        if (c0 + CC < C) load_chunk(c0 + CC);   // next chunk in flight during the compute
-        if (d < P) {
-            const int cn = min(CC, C - c0);
-            const int br = row + dl;
-            for (int cc = 0; cc < cn; ++cc) {
-                float va[QX], vb[QX + 2 * MD];
+        if (c0 + CC < C) fetch(c0 + CC);
+        if (DG > P && dl >= P) continue;   // a wave that only stages
+        const int cn = min(CC, C - c0);
+        const float* pa = &s1[0][row * TW + px];
+        const float* pb = &s2[0][(row + dl) * PITCH + px + CF_HALO - MD + x0];
+#pragma unroll 8
+        for (int cc = 0; cc < cn; ++cc) {
+            float va[QX], vb[QX + XG - 1];
 #pragma unroll
-                for (int x = 0; x < QX; ++x) va[x] = s1[cc][row][quad * QX + x];
+            for (int x = 0; x < QX; ++x) va[x] = pa[cc * (CF_TH * TW) + x];
 #pragma unroll
-                for (int x = 0; x < QX + 2 * MD; ++x) vb[x] = s2[cc][br][quad * QX + CF_HALO - MD + x];
+            for (int x = 0; x < QX + XG - 1; ++x) vb[x] = pb[cc * (SH * PITCH) + x];
 #pragma unroll
-                for (int x = 0; x < QX; ++x)
+            for (int x = 0; x < QX; ++x)
 #pragma unroll
-                    for (int k = 0; k < P; ++k) acc[x][k] += va[x] * vb[x + k];
-            }
+                for (int k = 0; k < XG; ++k) acc[x][k] += va[x] * vb[x + k];
         }
     }
-    const int h = h0 + row;
-    if (d >= P || h >= H) return;
-    float* o = out + ((long long)n * P * P + (long long)d * P) * HW + (long long)h * W + w0 + quad * QX;
-    // four pixels of a plane row as one 16-byte store when they are in the
-    // image and 16-byte aligned (a 16-byte aligned output and W a multiple of
-    // 4: every plane row then starts aligned)
-    if (QX == 4 && (W & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && w0 + quad * QX + 3 < W) {
+    const int h = h0 + row, w = w0 + px;
+    if (h >= H || (DG > P && dl >= P)) return;
+    float* o = out + ((long long)n * P * P + (long long)d * P + x0) * HW + (long long)h * W + w;
+    if (QX > 1 && w + QX <= W) {
+        typedef float V __attribute__((ext_vector_type(QX), aligned(4)));
 #pragma unroll
-        for (int k = 0; k < P; ++k) {
-            float v[4];
+        for (int k = 0; k < XG; ++k) {
+            V v;
 #pragma unroll
-            for (int x = 0; x < 4; ++x) v[x] = LEGACY ? acc[x % QX][k] / (float)C : acc[x % QX][k];
-            __builtin_nontemporal_store(*reinterpret_cast<const f32x4_t*>(v), reinterpret_cast<f32x4_t*>(o + k * HW));
+            for (int x = 0; x < QX; ++x) v[x] = LEGACY ? acc[x][k] / (float)C : acc[x][k];
+            __builtin_nontemporal_store(v, reinterpret_cast<V*>(o + k * HW));
         }
         return;
     }
 #pragma unroll
-    for (int k = 0; k < P; ++k)
+    for (int k = 0; k < XG; ++k)
 #pragma unroll
         for (int x = 0; x < QX; ++x)
-            if (w0 + quad * QX + x < W)
-                __builtin_nontemporal_store(LEGACY ? acc[x][k] / (float)C : acc[x][k], o + k * HW + x);
+            if (w + x < W) __builtin_nontemporal_store(LEGACY ? acc[x][k] / (float)C : acc[x][k], o + k * HW + x);
 }
 
 // Any displacement, FP32 or FP64: one thread per output element, sequential
-// in c (correlation.cc:147-182).  Used for max_displacement > 4 and FP64.
+// in c (correlation.cc:147-182).  Used for max_displacement > 4, FP64 and
+// images less than 4 pixels wide.
 template <typename T, bool LEGACY>
 __global__ __launch_bounds__(256) void k_corr_generic(const T* __restrict__ f1, const T* __restrict__ f2,
                                                       T* __restrict__ out, int N, int C, int H, int W, int md)
@@ -182,30 +173,52 @@ __global__ __launch_bounds__(256) void k_corr_generic(const T* __restrict__ f1, 
     out[i] = LEGACY ? acc / (T)C : acc;
 }
 
-template <int MD, int QX, int CC, int DG>
+template <int MD, int QX, int DG, int XS, int CCT>
 static void launch_corr_f32_q(const float* f1, const float* f2, float* out, int N, int C, int H, int W, bool legacy,
                               hipStream_t s)
 {
-    constexpr int P = 2 * MD + 1, G = DG >= P ? 1 : P / DG;
-    dim3 grid((W + 8 * QX - 1) / (8 * QX), (H + CF_TH - 1) / CF_TH, N * G);
+    dim3 grid((W + 8 * QX - 1) / (8 * QX), (H + CF_TH - 1) / CF_TH, N * (DG > 2 * MD + 1 ? 1 : (2 * MD + 1) / DG));
+    const dim3 block(64 * DG * XS);
     if (legacy)
-        hipLaunchKernelGGL((k_corr_f32<MD, true, QX, CC, DG>), grid, dim3(64 * DG), 0, s, f1, f2, out, C, H, W);
+        hipLaunchKernelGGL((k_corr_f32<MD, true, QX, DG, XS, CCT>), grid, block, 0, s, f1, f2, out, C, H, W);
     else
-        hipLaunchKernelGGL((k_corr_f32<MD, false, QX, CC, DG>), grid, dim3(64 * DG), 0, s, f1, f2, out, C, H, W);
+        hipLaunchKernelGGL((k_corr_f32<MD, false, QX, DG, XS, CCT>), grid, block, 0, s, f1, f2, out, C, H, W);
 }
 
-// 4 pixels per thread when that gives at least half a machine of blocks
-// (1920x1088 pyramid, with the 16-byte stores: at 240x136, 136 blocks of the
-// 4-pixel tile take 29.8 us against 40.2 us for 510 of the 1-pixel tile; at
-// 120x68, 36 against 135 blocks, 40 against 24 us)
+// The form by the number of 32x8 tiles, T.  Small levels are bound by the chain
+// of their chunks, so they are cut into as many waves as there are CUs for, each
+// with few sums and long chunks; large ones by LDS reads and the vector units,
+// so a lane takes 4 pixels with all horizontal displacements and a block all
+// vertical ones.  md = 4, us of the chosen form and of its two neighbours
+// (pixels x channels, T):
+//   30x17x196, 3      12.9 | 14.1 of the next
+//   60x34x128, 10     10.9 of the one before | 10.9 | 11.9
+//   120x68x96, 36     14.3 | 13.7 | 17.4
+//   200x90x64, 84     25.1 | 16.3 | 20.0
+//   240x150x32, 152   16.8 | 11.2 | 13.8
+//   480x272x32, 510   39.4 | 24.1
+// Other displacements: one small form and one large one (md = 0 with two waves
+// that only stage).
 template <int MD>
 static void launch_corr_f32(const float* f1, const float* f2, float* out, int N, int C, int H, int W, bool legacy,
                             hipStream_t s)
 {
-    const long long blocks4 = (long long)((W + 31) / 32) * ((H + CF_TH - 1) / CF_TH) * N;
-    if (blocks4 >= 128) launch_corr_f32_q<MD, 4, 8, 9>(f1, f2, out, N, C, H, W, legacy, s);
-    else launch_corr_f32_q<MD, 1, 32, ((2 * MD + 1) % CF_DG1 == 0 ? CF_DG1 : 2 * MD + 1)>(f1, f2, out, N, C, H, W,
-                                                                                           legacy, s);
+    constexpr int P = 2 * MD + 1;
+    const long long T = (long long)((W + 31) / 32) * ((H + CF_TH - 1) / CF_TH) * N;
+    if constexpr (MD == 4) {
+        if (36 * T <= 256) launch_corr_f32_q<MD, 1, 1, 3, 64>(f1, f2, out, N, C, H, W, legacy, s);
+        else if (12 * T <= 256) launch_corr_f32_q<MD, 1, 3, 3, 40>(f1, f2, out, N, C, H, W, legacy, s);
+        else if (T <= 55) launch_corr_f32_q<MD, 1, 3, 3, 20>(f1, f2, out, N, C, H, W, legacy, s);
+        else if (T <= 120) launch_corr_f32_q<MD, 2, 3, 1, 16>(f1, f2, out, N, C, H, W, legacy, s);
+        else if (T < 256) launch_corr_f32_q<MD, 4, 3, 1, 16>(f1, f2, out, N, C, H, W, legacy, s);
+        else launch_corr_f32_q<MD, 4, 9, 1, 4>(f1, f2, out, N, C, H, W, legacy, s);
+    } else if constexpr (MD == 0) {
+        if (T < 128) launch_corr_f32_q<MD, 1, 3, 1, 32>(f1, f2, out, N, C, H, W, legacy, s);
+        else launch_corr_f32_q<MD, 4, 3, 1, 8>(f1, f2, out, N, C, H, W, legacy, s);
+    } else {
+        if (T < 128) launch_corr_f32_q<MD, 1, P % 3 == 0 ? 3 : P, 1, 32>(f1, f2, out, N, C, H, W, legacy, s);
+        else launch_corr_f32_q<MD, 4, P, 1, 8>(f1, f2, out, N, C, H, W, legacy, s);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -312,7 +325,7 @@ int correlation_forward(const void* f1, const void* f2, void* out, int N, int C,
         const float* a = static_cast<const float*>(f1);
         const float* b = static_cast<const float*>(f2);
         float* o = static_cast<float*>(out);
-        switch (md) {
+        switch (W >= 4 ? md : -1) {   // (narrower images: one thread per output)
             case 0: launch_corr_f32<0>(a, b, o, N, C, H, W, legacy, s); break;
             case 1: launch_corr_f32<1>(a, b, o, N, C, H, W, legacy, s); break;
             case 2: launch_corr_f32<2>(a, b, o, N, C, H, W, legacy, s); break;
@@ -320,8 +333,9 @@ int correlation_forward(const void* f1, const void* f2, void* out, int N, int C,
             case 4: launch_corr_f32<4>(a, b, o, N, C, H, W, legacy, s); break;
             default: {
                 const long long total = (long long)N * (2 * md + 1) * (2 * md + 1) * H * W;
-                hipLaunchKernelGGL((k_corr_generic<float, false>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                                   s, a, b, o, N, C, H, W, md);
+                const dim3 g((unsigned)((total + 255) / 256));
+                if (legacy) hipLaunchKernelGGL((k_corr_generic<float, true>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
+                else hipLaunchKernelGGL((k_corr_generic<float, false>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
             }
         }
         return check_launch("correlation f32");
