@@ -1,4 +1,4 @@
-"""Every form of the FP32 Correlation at the edges of its range:
+"""Every form of the FP32 Correlation and of Warp at the edges of its range:
 the smallest and largest grids of each tile, remainders of tiles, slots that
 hang over the right edge, chunk remainders, images too narrow for wide loads."""
 import numpy as np
@@ -24,3 +24,20 @@ def test_correlation_f32_forms_bit_exact(vsc, orc, cuda, md, shape):
     print(f"corr f32 md={md} {shape}", flush=True)
     got = vsc.correlation(_t(f1, cuda), _t(f2, cuda), md, 0).cpu().numpy()
     assert np.array_equal(got, orc.correlation(f1, f2, md))
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 6, 2), (2, 4, 3, 65), (1, 3, 5, 1), (1, 9, 2, 128)])
+def test_warp_corners_at_the_edges(vsc, orc, cuda, shape):
+    """Positions a hair outside each edge (mass inside above 0.999, so the pixel
+    is kept with a corner missing), on the last column and row, and not finite.
+    FP32 weights against the oracle's double ones: a few roundings of values
+    of order 1."""
+    N, C, H, W = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.uniform(-1, 1, shape).astype(np.float32)
+    ys, xs = np.mgrid[0:H, 0:W].astype(np.float32)
+    for tx, ty in ((-0.0005, 0), (W - 1 + 0.0005, 0), (0, -0.0005), (0, H - 1 + 0.0005), (W - 1, H - 1), (W - 1.5, 0),
+                   (-1, 0), (W, 0), (np.inf, 0), (np.nan, 0)):
+        fl = np.stack([np.stack([tx - xs, ty - ys])] * N).astype(np.float32)
+        got = vsc.warp(_t(x, cuda), _t(fl, cuda)).cpu().numpy()
+        assert np.max(np.abs(got - orc.warp(x, fl))) < 1e-5, (tx, ty)
