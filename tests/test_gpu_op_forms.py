@@ -41,3 +41,43 @@ def test_warp_corners_at_the_edges(vsc, orc, cuda, shape):
         fl = np.stack([np.stack([tx - xs, ty - ys])] * N).astype(np.float32)
         got = vsc.warp(_t(x, cuda), _t(fl, cuda)).cpu().numpy()
         assert np.max(np.abs(got - orc.warp(x, fl))) < 1e-5, (tx, ty)
+
+
+# widths and alignments that used to be copied first, both sides of the line between one and three
+# displacements a block, hanging slots of 1 to 3 pixels, images too narrow for wide loads
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("shape", [(1, 33, 16, 225), (1, 32, 20, 193), (1, 31, 29, 222), (2, 64, 9, 67), (1, 5, 3, 1),
+                                   (1, 40, 5, 2), (2, 37, 6, 3), (1, 8, 2, 4), (1, 65, 37, 31)])
+def test_correlation_lowp_reads_any_width(vsc, orc, cuda, kind, shape):
+    """The bits of the same values in rows of a multiple of 4 (zeros to the
+    right, as outside the image), and of operands one element off their
+    alignment.  16-bit values also against the oracle: their products are exact
+    in FP32, so only the FP32 sums of C terms round, and 2 C ulps of the sum of
+    magnitudes bounds any order."""
+    import torch
+    N, C, H, W = shape
+    rng = np.random.default_rng(sum(shape))
+    f1, f2 = rng.standard_normal(shape).astype(np.float32), rng.standard_normal(shape).astype(np.float32)
+    if kind == "fp8":
+        q = [_t(rng.integers(0, 0x78, shape).astype(np.uint8), cuda) for _ in range(2)]
+        one = torch.ones(1, device=cuda)
+        call = lambda a, b: vsc.correlation_fp8(a, b, one, 4, 0)
+    else:
+        dt = torch.bfloat16 if kind == "bf16" else torch.float16
+        q = [_t(x, cuda).to(dt) for x in (f1, f2)]
+        call = lambda a, b: vsc.correlation(a, b, 4, 0)
+    print(f"corr {kind} {shape}", flush=True)
+    got = call(*q)
+    off, wide = [], []
+    for x in q:
+        buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=cuda)
+        off.append(buf[1:].view(x.shape))
+        off[-1].copy_(x)
+        wide.append(torch.zeros((N, C, H, (W + 7) // 4 * 4), dtype=x.dtype, device=cuda))
+        wide[-1][..., :W] = x
+    assert torch.equal(call(*off), got)
+    assert torch.equal(call(*wide)[..., :W], got)
+    if kind != "fp8":
+        f1, f2 = (x.float().cpu().numpy() for x in q)
+        bound = orc.correlation(np.abs(f1), np.abs(f2), 4)
+        assert np.all(np.abs(got.cpu().numpy() - orc.correlation(f1, f2, 4)) <= 2 * C * 2.0 ** -24 * bound + 1e-30)

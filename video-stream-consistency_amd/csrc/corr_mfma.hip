@@ -12,13 +12,15 @@
 // bound by the 81 output planes it writes, not by the products.
 //
 // Block: 8 waves; wave q computes one 16-pixel segment (q & 1) of output row
-// h0 + q/2 for all (2*MD+1)^2 displacements, 72 FP32 accumulators per lane.  The
-// NCHW operands are first copied channels-last (channels padded to 32, zeros)
-// by a bandwidth-bound conversion kernel; channels then stream through LDS in
-// chunks of 32 as straight 8-byte copies: the f1 tile (4 rows x 32 px) and the
-// f2 tile (12 rows x 40 px, MD-pixel halo, zeros outside the image), with a
-// padded pixel stride, so that each lane's 8-channel MFMA operand is one
-// 16-byte (8-byte for FP8) LDS read and 8 lanes cover all banks.
+// h0 + q/2 for DG vertical displacements and all horizontal ones, 8*DG FP32
+// accumulators per lane.  Channels stream through LDS in chunks of 32: the f1
+// tile (4 rows x 32 px) and the f2 rows that the displacements reach (40 px,
+// zeros outside the image), read from the NCHW operands 4 pixels at a time and
+// turned channels-last with byte permutes, with a padded pixel stride, so that
+// each lane's 8-channel MFMA operand is one 16-byte (8-byte for FP8) LDS read
+// and 8 lanes cover all banks.  (Widths that are not a multiple of 4 used to be
+// copied channels-last first, into memory allocated for the call: 213x119x64 in
+// BF16 45.6 us with the two copies, 13.9 without.)
 // After the channel loop, each wave moves the diagonals of its tiles through a
 // small LDS stage and writes every (dy, dx) output row as 32 consecutive floats.
 #include "vsc_internal.h"
@@ -32,7 +34,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
-static constexpr int CM_ROWS = 4;    // output rows per block (one per wave)
+static constexpr int CM_ROWS = 4;    // output rows per block (one per two waves)
 static constexpr int CM_PX = 32;     // output pixels per row per block
 static constexpr int CM_HALO = 4;    // f2 halo (max displacement supported)
 static constexpr int CM_KC = 32;     // channels per chunk (one MFMA K step)
@@ -78,156 +80,143 @@ __device__ inline uint2 nchw_px8(const uint32_t (&raw)[8], int j)
     return make_uint2(__builtin_amdgcn_perm(t23, t01, 0x05040100u), __builtin_amdgcn_perm(t67, t45, 0x05040100u));
 }
 
-// NCHW: the operands are read in their NCHW layout (width a multiple of 4,
-// 8-byte (16-bit) or 4-byte (FP8) aligned): each staging unit loads 4 pixels
-// of GC channel planes and writes them channels-last into LDS, so no
-// conversion pass runs before the kernel.  Otherwise the operands are
-// channels-last copies [n][y][x][CP].
-template <int KIND, int MD, bool LEGACY, bool NCHW>
+template <int KIND, int MD, bool LEGACY, int DG>
 __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, const void* __restrict__ f2v,
-                                               float* __restrict__ out, int C, int CP, int H, int W,
-                                               const float* scale)
+                                               float* __restrict__ out, int C, int H, int W, const float* scale)
 {
     constexpr int EB = (KIND == CM_FP8) ? 1 : 2;          // bytes per element
     constexpr int ST = CmLayout<EB>::STRIDE;              // LDS pixel stride in elements
-    constexpr int P = 2 * MD + 1;
-    constexpr int BR = CM_ROWS + 2 * CM_HALO, BC = CM_PX + 2 * CM_HALO;
+    constexpr int P = 2 * MD + 1, G = P / DG;
+    static_assert(P % DG == 0, "displacement groups of equal size");
+    constexpr int BR = CM_ROWS + DG - 1, BC = CM_PX + 2 * CM_HALO;
     using E = typename std::conditional<EB == 2, uint16_t, uint8_t>::type;
     // LDS: the operand tiles during the channel loop, then the whole output
     // tile [row][plane][32 px] at a plane pitch of 36 floats (the operand
     // tiles are dead by then): the 16 lanes of a K group write 16 planes at
     // once, which a 32-float pitch puts on the same banks
-    constexpr int SP = CM_PX + 4;
+    constexpr int SP = CM_PX + 4, PL = DG * P;
     constexpr int A_BYTES = CM_ROWS * CM_PX * ST * EB, B_BYTES = BR * BC * ST * EB;
-    constexpr int OUT_BYTES = CM_ROWS * P * P * SP * 4;
+    constexpr int OUT_BYTES = CM_ROWS * PL * SP * 4;
     constexpr int LDS_BYTES = (A_BYTES + B_BYTES) > OUT_BYTES ? (A_BYTES + B_BYTES) : OUT_BYTES;
     __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
     E (*sA)[CM_PX][ST] = reinterpret_cast<E (*)[CM_PX][ST]>(lds);
     E (*sB)[BC][ST] = reinterpret_cast<E (*)[BC][ST]>(lds + A_BYTES);
-    float (*stage)[P * P][SP] = reinterpret_cast<float (*)[P * P][SP]>(lds);
+    float (*stage)[PL][SP] = reinterpret_cast<float (*)[PL][SP]>(lds);
 
-    // operands are channels-last copies [n][y][x][CP] (CP: C padded to a
-    // multiple of 32 with zeros), so a chunk of 32 channels of one pixel is
-    // contiguous: staged with 8-byte vectors (VPP per pixel), no transpose
-    constexpr int VPP = CM_KC * EB / 8;
-    const E* f1 = static_cast<const E*>(f1v);
-    const E* f2 = static_cast<const E*>(f2v);
-    const int n = blockIdx.z;
-    const int h0 = blockIdx.y * CM_ROWS, w0 = blockIdx.x * CM_PX;
+    const int tiles = gridDim.x / G, dg = blockIdx.x / tiles;
+    const int n = blockIdx.z, h0 = blockIdx.y * CM_ROWS, w0 = blockIdx.x % tiles * CM_PX;
     const long long HW = (long long)H * W;
-    const E* a = f1 + (long long)n * HW * CP;
-    const E* b = f2 + (long long)n * HW * CP;
+    const E* f1 = static_cast<const E*>(f1v) + (long long)n * C * HW;
+    const E* f2 = static_cast<const E*>(f2v) + (long long)n * C * HW;
     const int tid = threadIdx.x;
     const int q = tid / 64, lane = tid % 64;
     const int qr = q >> 1, seg = q & 1;         // output row in the block, 16-pixel segment
     const int lr = lane % 16, lg = lane / 16;   // operand row/column, K group
 
-    f32x4 acc[P][2];
+    f32x4 acc[DG][2];
 #pragma unroll
-    for (int d = 0; d < P; ++d)
+    for (int d = 0; d < DG; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t) acc[d][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // NCHW staging units: (channel group of GC, row, group of 4 pixels)
+    // Staging units: GC channels x 4 pixels of a row of one of the tiles.  A unit
+    // loads its 4 pixels of GC channel planes, whatever their alignment, and
+    // writes them channels-last into LDS.  One that hangs over the right edge is
+    // read further left and shifted (zeros come in); images less than 4 pixels
+    // wide are read pixel by pixel.
     constexpr int GC = 8 / EB, CG = CM_KC / GC;
     constexpr int NA4 = CG * CM_ROWS * (CM_PX / 4), NB4 = CG * BR * (BC / 4), NU4 = NA4 + NB4;
     constexpr int RU4 = (NU4 + 511) / 512;
     using Raw = typename std::conditional<EB == 2, uint2, uint32_t>::type;
-    Raw raw[NCHW ? RU4 : 1][GC];
-    auto fetch4 = [&](int c0) {
-        const E* fa = f1 + (long long)n * C * HW;
-        const E* fb = f2 + (long long)n * C * HW;
+    typedef uint32_t U2 __attribute__((ext_vector_type(2), aligned(2)));
+    typedef uint32_t U1 __attribute__((aligned(1)));
+    Raw raw[RU4][GC];
+    const E* src[RU4];
+    int cfirst[RU4], shift[RU4];
+    E* dst[RU4];
+#pragma unroll
+    for (int k = 0; k < RU4; ++k) {
+        const int u = tid + 512 * k;
+        const bool inA = u < NA4;
+        const int ul = inA ? u : u - NA4;
+        const int rows = inA ? CM_ROWS : BR, groups = inA ? CM_PX / 4 : BC / 4;
+        const int g = ul % groups, r = (ul / groups) % rows, cg = ul / (groups * rows);
+        const int gh = inA ? h0 + r : h0 - MD + dg * DG + r;
+        const int gw = inA ? w0 + 4 * g : w0 - CM_HALO + 4 * g;
+        const bool ok = u < NU4 && gh >= 0 && gh < H && gw >= 0 && gw < W;
+        const int xs = W >= 4 ? min(gw, W - 4) : gw;
+        src[k] = (inA ? f1 : f2) + (ok ? (long long)cg * GC * HW + (long long)gh * W + xs : 0);
+        shift[k] = W >= 4 ? gw - xs : W - gw;         // (narrow images: pixels left)
+        cfirst[k] = ok ? cg * GC : 1 << 30;           // nothing to load
+        dst[k] = u >= NU4 ? nullptr : inA ? &sA[r][4 * g][cg * GC] : &sB[r][4 * g][cg * GC];
+    }
+    auto fetch = [&](int c0) {
 #pragma unroll
         for (int k = 0; k < RU4; ++k) {
-            const int u = tid + 512 * k;
-            const bool inA = u < NA4;
-            const int ul = inA ? u : u - NA4;
-            const int rows = inA ? CM_ROWS : BR, groups = inA ? CM_PX / 4 : BC / 4;
-            const int g = ul % groups, r = (ul / groups) % rows, cg = ul / (groups * rows);
-            const int gh = inA ? h0 + r : h0 - CM_HALO + r;
-            const int gw = inA ? w0 + 4 * g : w0 - CM_HALO + 4 * g;
-            const bool ok = u < NU4 && gh >= 0 && gh < H && gw >= 0 && gw < W;
-            const E* src = (inA ? fa : fb) + (long long)gh * W + gw;
+            const E* s = src[k] + (long long)c0 * HW;
 #pragma unroll
             for (int j = 0; j < GC; ++j) {
-                const int c = c0 + cg * GC + j;
                 Raw v{};
-                if (ok && c < C) v = *reinterpret_cast<const Raw*>(src + (long long)c * HW);
+                if (c0 + j + cfirst[k] < C) {
+                    const E* p = s + j * HW;
+                    if (W >= 4) {
+                        if constexpr (EB == 2) {
+                            const U2 t = *reinterpret_cast<const U2*>(p);
+                            v = make_uint2(t.x, t.y);
+                        } else {
+                            v = *reinterpret_cast<const U1*>(p);
+                        }
+                    } else {
+                        if constexpr (EB == 2) {
+                            v.x = p[0] | (shift[k] > 1 ? (uint32_t)p[1] << 16 : 0u);
+                            v.y = shift[k] > 2 ? p[2] : 0u;
+                        } else {
+                            v = p[0] | (shift[k] > 1 ? (uint32_t)p[1] << 8 : 0u) | (shift[k] > 2 ? (uint32_t)p[2] << 16 : 0u);
+                        }
+                    }
+                }
                 raw[k][j] = v;
             }
         }
     };
-    auto stage4 = [&]() {
+    auto stage_chunk = [&]() {
 #pragma unroll
         for (int k = 0; k < RU4; ++k) {
-            const int u = tid + 512 * k;
-            if (u >= NU4) continue;
-            const bool inA = u < NA4;
-            const int ul = inA ? u : u - NA4;
-            const int rows = inA ? CM_ROWS : BR, groups = inA ? CM_PX / 4 : BC / 4;
-            const int g = ul % groups, r = (ul / groups) % rows, cg = ul / (groups * rows);
+            if (!dst[k]) continue;
+            if (W >= 4 && shift[k] > 0 && shift[k] < 4) {
+#pragma unroll
+                for (int j = 0; j < GC; ++j) {
+                    if constexpr (EB == 2) {
+                        const uint64_t t = ((uint64_t)raw[k][j].y << 32 | raw[k][j].x) >> (16 * shift[k]);
+                        raw[k][j] = make_uint2((uint32_t)t, (uint32_t)(t >> 32));
+                    } else {
+                        raw[k][j] >>= 8 * shift[k];
+                    }
+                }
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 uint2 v;
                 if constexpr (EB == 2) v = nchw_px16(raw[k], j);
                 else v = nchw_px8(raw[k], j);
-                E* dst = inA ? &sA[r][4 * g + j][cg * GC] : &sB[r][4 * g + j][cg * GC];
-                *reinterpret_cast<uint2*>(dst) = v;
-            }
-        }
-    };
-
-    constexpr int NA = CM_ROWS * CM_PX * VPP, NB = BR * BC * VPP, NU = NA + NB, RU = (NU + 511) / 512;
-    uint2 rg[NCHW ? 1 : RU];
-    auto fetch = [&](int c0) {
-        if constexpr (NCHW) {
-            fetch4(c0);
-        } else {
-#pragma unroll
-            for (int k = 0; k < RU; ++k) {
-                const int u = tid + 512 * k;
-                uint2 v = make_uint2(0u, 0u);
-                if (u < NA) {
-                    const int p = u / VPP, cv = u % VPP, r = p / CM_PX, x = p % CM_PX;
-                    const int gh = h0 + r, gw = w0 + x;
-                    if (gh < H && gw < W)
-                        v = *reinterpret_cast<const uint2*>(a + ((long long)gh * W + gw) * CP + c0 + cv * (8 / EB));
-                } else if (u < NU) {
-                    const int ub = u - NA, p = ub / VPP, cv = ub % VPP, r = p / BC, x = p % BC;
-                    const int gh = h0 - CM_HALO + r, gw = w0 - CM_HALO + x;
-                    if (gh >= 0 && gh < H && gw >= 0 && gw < W)
-                        v = *reinterpret_cast<const uint2*>(b + ((long long)gh * W + gw) * CP + c0 + cv * (8 / EB));
-                }
-                rg[k] = v;
+                *reinterpret_cast<uint2*>(dst[k] + j * ST) = v;
             }
         }
     };
 
     fetch(0);
-    for (int c0 = 0; c0 < CP; c0 += CM_KC) {
+    for (int c0 = 0; c0 < C; c0 += CM_KC) {
         __syncthreads();
-        if constexpr (NCHW) stage4();
-#pragma unroll
-        for (int k = 0; k < (NCHW ? 0 : RU); ++k) {
-            const int u = tid + 512 * k;
-            if (u < NA) {
-                const int p = u / VPP, cv = u % VPP;
-                *reinterpret_cast<uint2*>(&sA[p / CM_PX][p % CM_PX][cv * (8 / EB)]) = rg[k];
-            } else if (u < NU) {
-                const int ub = u - NA, p = ub / VPP, cv = ub % VPP;
-                *reinterpret_cast<uint2*>(&sB[p / BC][p % BC][cv * (8 / EB)]) = rg[k];
-            }
-        }
+        stage_chunk();
         __syncthreads();
-        if (c0 + CM_KC < CP) fetch(c0 + CM_KC);
+        if (c0 + CM_KC < C) fetch(c0 + CM_KC);
         // A operand: pixel lr of this wave's segment, channels 8*lg .. 8*lg+7
         const E* pa = &sA[qr][16 * seg + lr][8 * lg];
 #pragma unroll
-        for (int d = 0; d < P; ++d) {
-            const int br = qr + CM_HALO + d - MD;   // f2 row of displacement dy = d - MD
+        for (int d = 0; d < DG; ++d) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const E* pb = &sB[br][16 * seg + 8 * t + lr][8 * lg];
+                const E* pb = &sB[qr + d][16 * seg + 8 * t + lr][8 * lg];
                 acc[d][t] = cm_mfma<KIND>(pa, pb, acc[d][t]);
             }
         }
@@ -239,7 +228,7 @@ __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, con
     // diagonals -> stage[row][plane][pixel]: lane holds G[4*lg + r][lr + 8*t]
     __syncthreads();
 #pragma unroll
-    for (int d = 0; d < P; ++d)
+    for (int d = 0; d < DG; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -255,17 +244,18 @@ __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, con
             }
     __syncthreads();
     // each group of 8 lanes writes one 128-byte row segment of one plane, 16
-    // bytes per lane where the 4 pixels are in the image and the output rows
-    // are 16-byte aligned (a 16-byte aligned output, W a multiple of 4);
-    // the cost volume is not re-read by this kernel: non-temporal stores
-    const bool vec = (W & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    for (int e = tid; e < CM_ROWS * P * P * CM_PX / 4; e += 512) {
-        const int x = 4 * (e % (CM_PX / 4)), pl = (e / (CM_PX / 4)) % (P * P), r = e / (CM_PX / 4 * P * P);
+    // bytes a lane whatever the alignment (the tail of a row pixel by pixel); the
+    // cost volume is not re-read by this kernel: non-temporal stores
+    float* o0 = out + ((long long)n * P * P + dg * PL) * HW;
+    for (int e = tid; e < CM_ROWS * PL * CM_PX / 4; e += 512) {
+        const int x = 4 * (e % (CM_PX / 4)), pl = (e / (CM_PX / 4)) % PL, r = e / (CM_PX / 4 * PL);
         const int h = h0 + r, w = w0 + x;
         if (h >= H) continue;
-        float* o = out + ((long long)n * P * P + pl) * HW + (long long)h * W + w;
-        if (vec && w + 3 < W) {
-            __builtin_nontemporal_store(*reinterpret_cast<const f32x4*>(&stage[r][pl][x]), reinterpret_cast<f32x4*>(o));
+        float* o = o0 + pl * HW + (long long)h * W + w;
+        if (w + 3 < W) {
+            typedef float F4U __attribute__((ext_vector_type(4), aligned(4)));
+            __builtin_nontemporal_store(__builtin_bit_cast(F4U, *reinterpret_cast<const f32x4*>(&stage[r][pl][x])),
+                                        reinterpret_cast<F4U*>(o));
         } else {
             for (int j = 0; j < 4; ++j)
                 if (w + j < W) __builtin_nontemporal_store(stage[r][pl][x + j], o + j);
@@ -273,135 +263,58 @@ __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, con
     }
 }
 
-// The kernel as is (152 VGPRs for md = 4: one 512-thread block per CU), and
-// the same tile capped at 128 VGPRs for two blocks per CU (13 of them spill
-// to scratch at md = 4).  Grids of at least 256 blocks take the capped form
-// (1920x1088 pyramid, BF16: 32.9 vs 38.4 us at 480x272, 19.7 vs 21.5 us at
-// 240x136); smaller grids lose to the spills (120x68: 15.7 vs 13.9 us).
-template <int KIND, int MD, bool LEGACY, bool NCHW>
-__global__ __launch_bounds__(512) void k_corr_mfma(const void* __restrict__ f1v, const void* __restrict__ f2v,
-                                                   float* __restrict__ out, int C, int CP, int H, int W,
-                                                   const float* scale)
+// Waves per SIMD the registers are capped for: three blocks per CU (four in
+// FP8, whose staging holds less) with 3 or fewer vertical displacements a
+// block, two with more (480x272x32, FP8: 24.6 us at 4, 21.2 at 6, 19.5 at 8;
+// BF16: 32.6, 26.0, 35.0 with spills).
+template <int KIND, int MD, bool LEGACY, int DG>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DG > 3 ? 4 : KIND == CM_FP8 ? 8 : 6)))
+void k_corr_mfma(const void* __restrict__ f1, const void* __restrict__ f2, float* __restrict__ out, int C, int H, int W,
+                 const float* scale)
 {
-    corr_mfma_tile<KIND, MD, LEGACY, NCHW>(f1v, f2v, out, C, CP, H, W, scale);
+    corr_mfma_tile<KIND, MD, LEGACY, DG>(f1, f2, out, C, H, W, scale);
 }
 
-template <int KIND, int MD, bool LEGACY, bool NCHW>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_corr_mfma2(
-    const void* __restrict__ f1v, const void* __restrict__ f2v, float* __restrict__ out, int C, int CP, int H, int W,
-    const float* scale)
+template <int KIND, int MD, int DG>
+static void launch_mfma_dg(const void* f1, const void* f2, float* out, int N, int C, int H, int W, bool legacy,
+                           const float* scale, hipStream_t s)
 {
-    corr_mfma_tile<KIND, MD, LEGACY, NCHW>(f1v, f2v, out, C, CP, H, W, scale);
+    dim3 grid((W + CM_PX - 1) / CM_PX * ((2 * MD + 1) / DG), (H + CM_ROWS - 1) / CM_ROWS, N);
+    if (legacy) hipLaunchKernelGGL((k_corr_mfma<KIND, MD, true, DG>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale);
+    else hipLaunchKernelGGL((k_corr_mfma<KIND, MD, false, DG>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale);
 }
 
+// Vertical displacements per block: all nine need 72 sums a lane, so one or two
+// blocks stood on a CU, each a chain of loads, products, staging and stores;
+// thirds stage half as much again but overlap three or four blocks (BF16,
+// 240x136x64: 16.7 us with nine, 13.3 with three; 213x119x64: 15.9, 13.9).  One
+// a block while all of them still fit the chip at once (30x17x196: 10.6 us with
+// one, 13.1 with three, 25.1 with nine; 121x68x96, 612 blocks of one: 10.5, 8.4, 15.2).
 template <int KIND, int MD>
-static void launch_mfma(const void* f1, const void* f2, float* out, int N, int C, int CP, int H, int W, bool legacy,
-                        bool nchw, const float* scale, hipStream_t s)
+static void launch_mfma(const void* f1, const void* f2, float* out, int N, int C, int H, int W, bool legacy,
+                        const float* scale, hipStream_t s)
 {
-    dim3 grid((W + CM_PX - 1) / CM_PX, (H + CM_ROWS - 1) / CM_ROWS, N);
-    const bool two = (long long)grid.x * grid.y * grid.z >= 256;
-    if (legacy && nchw)
-        hipLaunchKernelGGL(two ? (k_corr_mfma2<KIND, MD, true, true>) : (k_corr_mfma<KIND, MD, true, true>), grid,
-                           dim3(512), 0, s, f1, f2, out, C, CP, H, W, scale);
-    else if (legacy)
-        hipLaunchKernelGGL(two ? (k_corr_mfma2<KIND, MD, true, false>) : (k_corr_mfma<KIND, MD, true, false>), grid,
-                           dim3(512), 0, s, f1, f2, out, C, CP, H, W, scale);
-    else if (nchw)
-        hipLaunchKernelGGL(two ? (k_corr_mfma2<KIND, MD, false, true>) : (k_corr_mfma<KIND, MD, false, true>), grid,
-                           dim3(512), 0, s, f1, f2, out, C, CP, H, W, scale);
-    else
-        hipLaunchKernelGGL(two ? (k_corr_mfma2<KIND, MD, false, false>) : (k_corr_mfma<KIND, MD, false, false>), grid,
-                           dim3(512), 0, s, f1, f2, out, C, CP, H, W, scale);
+    constexpr int P = 2 * MD + 1;
+    const long long tiles = (long long)((W + CM_PX - 1) / CM_PX) * ((H + CM_ROWS - 1) / CM_ROWS) * N;
+    if (MD == 4 && tiles * P <= 256) launch_mfma_dg<KIND, MD, MD == 4 ? 1 : P>(f1, f2, out, N, C, H, W, legacy, scale, s);
+    else launch_mfma_dg<KIND, MD, P % 3 == 0 ? 3 : P>(f1, f2, out, N, C, H, W, legacy, scale, s);
 }
 
 template <int KIND>
-static int dispatch_md(const void* f1, const void* f2, float* out, int N, int C, int CP, int H, int W, int md,
-                       bool legacy, bool nchw, const float* scale, hipStream_t s)
+static int dispatch_md(const void* f1, const void* f2, float* out, int N, int C, int H, int W, int md, bool legacy,
+                       const float* scale, hipStream_t s)
 {
     switch (md) {
-        case 0: launch_mfma<KIND, 0>(f1, f2, out, N, C, CP, H, W, legacy, nchw, scale, s); break;
-        case 1: launch_mfma<KIND, 1>(f1, f2, out, N, C, CP, H, W, legacy, nchw, scale, s); break;
-        case 2: launch_mfma<KIND, 2>(f1, f2, out, N, C, CP, H, W, legacy, nchw, scale, s); break;
-        case 3: launch_mfma<KIND, 3>(f1, f2, out, N, C, CP, H, W, legacy, nchw, scale, s); break;
-        case 4: launch_mfma<KIND, 4>(f1, f2, out, N, C, CP, H, W, legacy, nchw, scale, s); break;
+        case 0: launch_mfma<KIND, 0>(f1, f2, out, N, C, H, W, legacy, scale, s); break;
+        case 1: launch_mfma<KIND, 1>(f1, f2, out, N, C, H, W, legacy, scale, s); break;
+        case 2: launch_mfma<KIND, 2>(f1, f2, out, N, C, H, W, legacy, scale, s); break;
+        case 3: launch_mfma<KIND, 3>(f1, f2, out, N, C, H, W, legacy, scale, s); break;
+        case 4: launch_mfma<KIND, 4>(f1, f2, out, N, C, H, W, legacy, scale, s); break;
         default:
             return set_error(VSC_E_UNSUPPORTED,
                              "vsc_correlation_forward: reduced-precision correlation supports max_displacement <= 4");
     }
     return check_launch("correlation mfma");
-}
-
-// NCHW -> channels-last [n][y][x][CP], channels >= C zero.  One thread per
-// 4 consecutive pixels and 8-byte channel group (G = 4 BF16/F16 or 8 FP8
-// channels): G vector loads of 4 pixels of one channel (coalesced along x
-// across the wave), a register transpose, 4 vector stores of G channels.
-// Needs H*W % 4 == 0 for the vector loads; k_to_nhwc1 is the general form.
-template <typename E>
-__global__ void k_to_nhwc4(const E* __restrict__ in, E* __restrict__ out, int C, int CP, long long HW, int N)
-{
-    constexpr int G = 8 / sizeof(E);
-    using V4 = typename std::conditional<sizeof(E) == 2, uint2, uint32_t>::type;   // 4 pixels of one channel
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long quads = HW / 4;
-    const int groups = CP / G;
-    const long long p4 = e % quads;
-    const long long rest = e / quads;
-    if (rest >= (long long)groups * N) return;
-    const int g = (int)(rest % groups), n = (int)(rest / groups);
-    E v[G][4];
-#pragma unroll
-    for (int k = 0; k < G; ++k) {
-        const int c = g * G + k;
-        V4 x;
-        if (c < C) x = *reinterpret_cast<const V4*>(in + ((long long)n * C + c) * HW + p4 * 4);
-        else __builtin_memset(&x, 0, sizeof(x));
-        __builtin_memcpy(v[k], &x, sizeof(x));
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        E w[G];
-#pragma unroll
-        for (int k = 0; k < G; ++k) w[k] = v[k][j];
-        uint2 pk;
-        __builtin_memcpy(&pk, w, 8);
-        *reinterpret_cast<uint2*>(out + ((long long)n * HW + p4 * 4 + j) * CP + g * G) = pk;
-    }
-}
-
-template <typename E>
-__global__ void k_to_nhwc1(const E* __restrict__ in, E* __restrict__ out, int C, int CP, long long HW, int N)
-{
-    constexpr int G = 8 / sizeof(E);
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int groups = CP / G;
-    const long long p = e % HW;
-    const long long rest = e / HW;
-    if (rest >= (long long)groups * N) return;
-    const int g = (int)(rest % groups), n = (int)(rest / groups);
-    E v[G];
-#pragma unroll
-    for (int k = 0; k < G; ++k) {
-        const int c = g * G + k;
-        v[k] = c < C ? in[((long long)n * C + c) * HW + p] : (E)0;
-    }
-    uint2 pk;
-    __builtin_memcpy(&pk, v, 8);
-    *reinterpret_cast<uint2*>(out + ((long long)n * HW + p) * CP + g * G) = pk;
-}
-
-template <typename E>
-static void to_nhwc(const void* in, void* out, int C, int CP, long long HW, int N, hipStream_t s)
-{
-    constexpr int G = 8 / sizeof(E);
-    if (HW % 4 == 0) {
-        const long long units = (HW / 4) * (CP / G) * N;
-        hipLaunchKernelGGL(k_to_nhwc4<E>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s,
-                           static_cast<const E*>(in), static_cast<E*>(out), C, CP, HW, N);
-    } else {
-        const long long units = HW * (CP / G) * N;
-        hipLaunchKernelGGL(k_to_nhwc1<E>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s,
-                           static_cast<const E*>(in), static_cast<E*>(out), C, CP, HW, N);
-    }
 }
 
 size_t corr_mfma_workspace_bytes(int N, int C, int H, int W, int in_dtype)
@@ -413,55 +326,25 @@ size_t corr_mfma_workspace_bytes(int N, int C, int H, int W, int in_dtype)
     return 2 * one;
 }
 
-// widths that are multiples of 4 with aligned operands: the kernel reads the
-// NCHW operands itself, with no channels-last copy and no workspace
-bool corr_mfma_reads_nchw(const void* f1, const void* f2, int W, int in_dtype)
+// Whether the entry points that take or hold a workspace ask for one.  The
+// kernel reads its operands in place at any width and alignment; the requirement
+// for other widths and alignments is the entry points' contract.
+bool corr_mfma_asks_workspace(const void* f1, const void* f2, int W, int in_dtype)
 {
     const uintptr_t align = in_dtype == VSC_FP8E4M3 ? 4 : 8;
-    return W % 4 == 0 && reinterpret_cast<uintptr_t>(f1) % align == 0 && reinterpret_cast<uintptr_t>(f2) % align == 0;
+    return W % 4 != 0 || reinterpret_cast<uintptr_t>(f1) % align != 0 || reinterpret_cast<uintptr_t>(f2) % align != 0;
 }
 
-// workspace: corr_mfma_workspace_bytes() bytes of device memory, or NULL to
-// allocate it stream-ordered for this call (unused when the kernel reads the
-// NCHW operands directly)
 int corr_mfma_dispatch(const void* f1, const void* f2, float* out, int N, int C, int H, int W, int md, int legacy,
-                       int in_dtype, const float* chan_scale, void* workspace, hipStream_t s)
+                       int in_dtype, const float* chan_scale, hipStream_t s)
 {
-    if (in_dtype != VSC_BF16 && in_dtype != VSC_F16 && in_dtype != VSC_FP8E4M3)
-        return set_error(VSC_E_DTYPE, "vsc_correlation_forward: unsupported input type");
     if (md > 4)
         return set_error(VSC_E_UNSUPPORTED,
                          "vsc_correlation_forward: reduced-precision correlation supports max_displacement <= 4");
-    const int eb = in_dtype == VSC_FP8E4M3 ? 1 : 2;
-    const int CP = (C + CM_KC - 1) / CM_KC * CM_KC;
-    const long long HW = (long long)H * W;
-    if (corr_mfma_reads_nchw(f1, f2, W, in_dtype)) {
-        if (in_dtype == VSC_BF16) return dispatch_md<CM_BF16>(f1, f2, out, N, C, CP, H, W, md, legacy, true, nullptr, s);
-        if (in_dtype == VSC_F16) return dispatch_md<CM_F16>(f1, f2, out, N, C, CP, H, W, md, legacy, true, nullptr, s);
-        return dispatch_md<CM_FP8>(f1, f2, out, N, C, CP, H, W, md, legacy, true, chan_scale, s);
-    }
-    const size_t bytes = corr_mfma_workspace_bytes(N, C, H, W, in_dtype);
-    void* ws = workspace;
-    int rc;
-    if (!ws && (rc = check_hip(hipMallocAsync(&ws, bytes, s), "vsc_correlation_forward workspace"))) return rc;
-    void* t1 = ws;
-    void* t2 = static_cast<char*>(ws) + bytes / 2;
-    if (eb == 2) {
-        to_nhwc<uint16_t>(f1, t1, C, CP, HW, N, s);
-        to_nhwc<uint16_t>(f2, t2, C, CP, HW, N, s);
-    } else {
-        to_nhwc<uint8_t>(f1, t1, C, CP, HW, N, s);
-        to_nhwc<uint8_t>(f2, t2, C, CP, HW, N, s);
-    }
-    rc = check_launch("correlation to channels-last");
-    if (!rc) {
-        if (in_dtype == VSC_BF16) rc = dispatch_md<CM_BF16>(t1, t2, out, N, C, CP, H, W, md, legacy, false, nullptr, s);
-        else if (in_dtype == VSC_F16) rc = dispatch_md<CM_F16>(t1, t2, out, N, C, CP, H, W, md, legacy, false, nullptr, s);
-        else rc = dispatch_md<CM_FP8>(t1, t2, out, N, C, CP, H, W, md, legacy, false, chan_scale, s);
-    }
-    if (workspace) return rc;
-    const int rc2 = check_hip(hipFreeAsync(ws, s), "vsc_correlation_forward workspace free");
-    return rc ? rc : rc2;
+    if (in_dtype == VSC_BF16) return dispatch_md<CM_BF16>(f1, f2, out, N, C, H, W, md, legacy, nullptr, s);
+    if (in_dtype == VSC_F16) return dispatch_md<CM_F16>(f1, f2, out, N, C, H, W, md, legacy, nullptr, s);
+    if (in_dtype == VSC_FP8E4M3) return dispatch_md<CM_FP8>(f1, f2, out, N, C, H, W, md, legacy, chan_scale, s);
+    return set_error(VSC_E_DTYPE, "vsc_correlation_forward: unsupported input type");
 }
 
 // ---------------------------------------------------------------------------
