@@ -81,3 +81,23 @@ def test_correlation_lowp_reads_any_width(vsc, orc, cuda, kind, shape):
         f1, f2 = (x.float().cpu().numpy() for x in q)
         bound = orc.correlation(np.abs(f1), np.abs(f2), 4)
         assert np.all(np.abs(got.cpu().numpy() - orc.correlation(f1, f2, 4)) <= 2 * C * 2.0 ** -24 * bound + 1e-30)
+
+
+@pytest.mark.parametrize("shape", [(2, 5, 3, 1), (1, 300, 7, 9), (1, 3, 67, 61), (3, 257, 4, 8), (1, 2, 257, 256)])
+def test_fp8_quantiser_planes(vsc, cuda, shape):
+    """Plane sizes around the quantiser's 4-pixel groups and 1024- and
+    4096-pixel blocks, more channels than threads: the bits of the same
+    formulas in FP32 (numpy), a channel of zeros among them."""
+    import torch
+    rng = np.random.default_rng(sum(shape))
+    f1 = rng.standard_normal(shape).astype(np.float32)
+    f2 = (rng.standard_normal(shape) * np.exp(rng.uniform(-2, 2, (1, shape[1], 1, 1)))).astype(np.float32)
+    f1[:, 1] = 0
+    m1, m2 = np.abs(f1).max(axis=(0, 2, 3)), np.abs(f2).max(axis=(0, 2, 3))
+    r = np.where((m1 > 0) & (m2 > 0), np.sqrt(m2 / np.where(m1 > 0, m1, 1), dtype=np.float32), np.float32(1))
+    s1, s2 = (m1 * r).max() / np.float32(448), (m2 / r).max() / np.float32(448)
+    e = [(f1 * r[None, :, None, None]) / s1, (f2 / r[None, :, None, None]) / s2]
+    q1, q2, sc = vsc.quantize_fp8_pair(_t(f1, cuda), _t(f2, cuda))
+    for q, x in zip((q1, q2), e):
+        assert torch.equal(q.cpu(), torch.from_numpy(x.astype(np.float32)).to(torch.float8_e4m3fn).view(torch.uint8))
+    assert abs(float(sc.cpu()[0]) - float(s1 * s2)) <= 1e-6 * float(s1 * s2)

@@ -554,12 +554,11 @@ def quantize_fp8_pair(f1, f2, workspace=None):
     q1 = torch.empty(a.shape, dtype=torch.uint8, device=a.device)
     q2 = torch.empty(a.shape, dtype=torch.uint8, device=a.device)
     sc = torch.empty(1, dtype=torch.float32, device=a.device)
-    if workspace is not None:
-        check(lib().vsc_quantize_fp8_pair_ws(_ptr(a), _ptr(b), _ptr(q1), _ptr(q2), _ptr(sc), N, C, H, W,
-                                             _ptr(workspace), workspace.numel() * workspace.element_size(),
-                                             _stream()))
-        return q1, q2, sc
-    check(lib().vsc_quantize_fp8_pair(_ptr(a), _ptr(b), _ptr(q1), _ptr(q2), _ptr(sc), N, C, H, W, _stream()))
+    if workspace is None:
+        # from torch's allocator: the stream-ordered allocation of the form without a workspace costs 25 us a call
+        workspace = torch.empty(lib().vsc_quantize_fp8_pair_workspace_size(C), dtype=torch.uint8, device=a.device)
+    check(lib().vsc_quantize_fp8_pair_ws(_ptr(a), _ptr(b), _ptr(q1), _ptr(q2), _ptr(sc), N, C, H, W,
+                                         _ptr(workspace), workspace.numel() * workspace.element_size(), _stream()))
     return q1, q2, sc
 
 

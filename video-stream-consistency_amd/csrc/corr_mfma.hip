@@ -399,15 +399,35 @@ __global__ void k_to_e4m3(const float* in, uint8_t* out, long long n)
 // ---------------------------------------------------------------------------
 // per-channel max |f| over N, H, W, as ordered float bits (non-negative floats
 // order like their bit patterns), accumulated with atomicMax
-__global__ void k_chan_absmax(const float* f, uint32_t* mx, int N, int C, long long HW)
+// mx[t*C + c] = largest magnitude of channel c of tensor t (0: f1, 1: f2);
+// blockIdx.x = t * blocks of a plane + block.  4096 pixels and more a block and
+// one atomic each: with 256 blocks' waves all updating a channel's word the
+// updates alone took 60 us.
+__global__ __launch_bounds__(256) void k_chan_absmax(const float* f1, const float* f2, uint32_t* mx, int C,
+                                                     long long HW)
 {
-    const int c = blockIdx.y, n = blockIdx.z;
-    const float* p = f + ((long long)n * C + c) * HW;
+    const int gx = gridDim.x / 2, t = (int)blockIdx.x >= gx;
+    const int c = blockIdx.y, n = blockIdx.z, bx = blockIdx.x - t * gx;
+    const float* p = (t ? f2 : f1) + ((long long)n * C + c) * HW;
+    typedef float F4U __attribute__((ext_vector_type(4), aligned(4)));
     float m = 0.0f;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < HW; i += (long long)gridDim.x * blockDim.x)
-        m = fmaxf(m, fabsf(p[i]));
+    const long long step = (long long)gx * 1024;
+    for (long long i = (long long)bx * 1024 + threadIdx.x * 4; i < HW; i += step) {
+        if (i + 4 <= HW) {
+            const F4U v = *reinterpret_cast<const F4U*>(p + i);
+            m = fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
+        } else {
+            for (long long j = i; j < HW; ++j) m = fmaxf(m, fabsf(p[j]));
+        }
+    }
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(&mx[c], __builtin_bit_cast(uint32_t, m));
+    __shared__ float s_m[4];
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x / 64] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+        atomicMax(&mx[t * C + c], __builtin_bit_cast(uint32_t, m));
+    }
 }
 
 __global__ void k_zero_u32(uint32_t* p, int n)
@@ -417,33 +437,71 @@ __global__ void k_zero_u32(uint32_t* p, int n)
 }
 
 // r_c = sqrt(max2_c / max1_c) (1 when either is 0); s1 = max_c(max1_c r_c)/448,
-// s2 = max_c(max2_c / r_c)/448; writes r[c], inv scales and scale = s1*s2.
-__global__ void k_fp8_scales(const uint32_t* mx1, const uint32_t* mx2, float* r, float* sc, int C)
+// s2 = max_c(max2_c / r_c)/448; writes r[c], inv scales and scale = s1*s2.  A
+// thread per channel (one thread for all took 40 us of 196 channels' divisions
+// and roots in a row).
+__global__ __launch_bounds__(256) void k_fp8_scales(const uint32_t* mx1, const uint32_t* mx2, float* r, float* sc,
+                                                    float* scale, int C)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    __shared__ float s_m[2][4];
     float m1 = 0.0f, m2 = 0.0f;
-    for (int c = 0; c < C; ++c) {
+    for (int c = threadIdx.x; c < C; c += 256) {
         const float a = __builtin_bit_cast(float, mx1[c]), b = __builtin_bit_cast(float, mx2[c]);
         const float rc = (a > 0.0f && b > 0.0f) ? sqrtf(b / a) : 1.0f;
         r[c] = rc;
         m1 = fmaxf(m1, a * rc);
         m2 = fmaxf(m2, b / rc);
     }
+    for (int off = 32; off > 0; off >>= 1) {
+        m1 = fmaxf(m1, __shfl_xor(m1, off));
+        m2 = fmaxf(m2, __shfl_xor(m2, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s_m[0][threadIdx.x / 64] = m1;
+        s_m[1][threadIdx.x / 64] = m2;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < 4; ++w) {
+        m1 = fmaxf(m1, s_m[0][w]);
+        m2 = fmaxf(m2, s_m[1][w]);
+    }
     const float s1 = m1 > 0.0f ? m1 / 448.0f : 1.0f;
     const float s2 = m2 > 0.0f ? m2 / 448.0f : 1.0f;
     sc[0] = s1 * s2;
     sc[1] = s1;
     sc[2] = s2;
+    *scale = s1 * s2;
 }
 
-__global__ void k_fp8_quant(const float* f, uint8_t* q, const float* r, const float* sc, int which, int C,
-                            long long HW, long long n)
+// Both tensors (blockIdx.y), 4 neighbouring pixels of a plane per thread, loaded
+// and stored together whatever their alignment; blockIdx.x = plane * chunks + chunk
+__global__ __launch_bounds__(256) void k_fp8_quant(const float* f1, const float* f2, uint8_t* q1, uint8_t* q2,
+                                                   const float* r, const float* sc, int C, long long HW, int chunks)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = (int)((i / HW) % C);
-    const float v = which == 0 ? (f[i] * r[c]) / sc[1] : (f[i] / r[c]) / sc[2];
-    q[i] = f32_to_e4m3(v);
+    typedef float F4U __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint32_t U1 __attribute__((aligned(1)));
+    const long long pl = blockIdx.x / chunks;
+    const long long i = ((long long)(blockIdx.x - pl * chunks) * 256 + threadIdx.x) * 4;
+    if (i >= HW) return;
+    const bool second = blockIdx.y != 0;
+    const float rc = r[pl % C], s = sc[second ? 2 : 1];
+    const float* f = (second ? f2 : f1) + pl * HW + i;
+    uint8_t* q = (second ? q2 : q1) + pl * HW + i;
+    const int n = (int)(HW - i < 4 ? HW - i : 4);
+    float v[4];
+    if (n == 4) {
+        const F4U x = *reinterpret_cast<const F4U*>(f);
+        for (int j = 0; j < 4; ++j) v[j] = x[j];
+    } else {
+        for (int j = 0; j < 4; ++j) v[j] = j < n ? f[j] : 0.0f;
+    }
+    uint32_t pk = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pk |= (uint32_t)f32_to_e4m3((second ? v[j] / rc : v[j] * rc) / s) << (8 * j);
+    if (n == 4) *reinterpret_cast<U1*>(q) = pk;
+    else
+        for (int j = 0; j < n; ++j) q[j] = (uint8_t)(pk >> (8 * j));
 }
 
 }  // namespace vsc
@@ -473,15 +531,13 @@ static int quantize_fp8_pair(const float* f1, const float* f2, uint8_t* q1, uint
     float* r = reinterpret_cast<float*>(mx + 2 * C);
     float* sc = r + C;
     hipLaunchKernelGGL(k_zero_u32, dim3((2 * C + 255) / 256), dim3(256), 0, s, mx, 2 * C);
-    const unsigned gx = (unsigned)std::min<long long>((HW + 255) / 256, 64);
-    hipLaunchKernelGGL(k_chan_absmax, dim3(gx, C, N), dim3(256), 0, s, f1, mx, N, C, HW);
-    hipLaunchKernelGGL(k_chan_absmax, dim3(gx, C, N), dim3(256), 0, s, f2, mx + C, N, C, HW);
-    hipLaunchKernelGGL(k_fp8_scales, dim3(1), dim3(64), 0, s, mx, mx + C, r, sc, C);
-    const unsigned g = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_fp8_quant, dim3(g), dim3(256), 0, s, f1, q1, r, sc, 0, C, HW, n);
-    hipLaunchKernelGGL(k_fp8_quant, dim3(g), dim3(256), 0, s, f2, q2, r, sc, 1, C, HW, n);
+    const unsigned gx = (unsigned)std::min<long long>((HW + 4095) / 4096, 16);
+    hipLaunchKernelGGL(k_chan_absmax, dim3(2 * gx, C, N), dim3(256), 0, s, f1, f2, mx, C, HW);
+    hipLaunchKernelGGL(k_fp8_scales, dim3(1), dim3(256), 0, s, mx, mx + C, r, sc, scale, C);
+    const int chunks = (int)((HW + 1023) / 1024);
+    hipLaunchKernelGGL(k_fp8_quant, dim3((unsigned)((long long)N * C * chunks), 2), dim3(256), 0, s, f1, f2, q1, q2, r, sc, C, HW,
+                       chunks);
     rc = check_launch("vsc_quantize_fp8_pair");
-    if (!rc) rc = check_hip(hipMemcpyAsync(scale, sc, sizeof(float), hipMemcpyDeviceToDevice, s), "vsc_quantize_fp8_pair");
     if (workspace) return rc;
     const int rc2 = check_hip(hipFreeAsync(ws, s), "vsc_quantize_fp8_pair workspace free");
     return rc ? rc : rc2;
