@@ -1,7 +1,7 @@
 // 3x3 convolution over channels-last (NHWC) tensors on MFMA (gfx950): the
 // building block of the flow network (Conv2d layers of pwcnet.py:186-241,
-// 511-535, 614-644; padding = dilation, stride 1 or 2) and of the learned flow
-// upsampler.  FP32 (v_mfma_f32_16x16x4_f32), BF16 and FP16
+// 511-535, 614-644; padding = dilation, stride 1 or 2; k_conv3x3w but for the
+// layers of at most 16 channels) and of the learned flow upsampler (k_conv3x3).  FP32 (v_mfma_f32_16x16x4_f32), BF16 and FP16
 // (v_mfma_f32_16x16x32_{bf16,f16}) operands, FP32 accumulation, bias,
 // LeakyReLU(0.1) / ReLU and a residual add fused into the epilogue.
 //
@@ -22,6 +22,9 @@
 #include "vsc_internal.h"
 
 #include <algorithm>
+#include <cstring>
+#include <iterator>
+#include <vector>
 
 namespace vsc {
 
@@ -38,7 +41,7 @@ template <> struct ConvK<EK_F16> { static constexpr int KC = 32; };
 struct ConvArgs {
     const void* in; int in_cs, in_c0;
     int N, H, W, Cin;
-    const void* wt; const float* bias;
+    const void* wt; const void* wtp; const float* bias;
     void* out; int out_cs, out_c0;
     void* out2; int out2_cs, out2_c0;   // optional second copy of the result, in the input's element kind (Cout <= 16)
     const void* add; int add_cs, add_c0;
@@ -46,14 +49,8 @@ struct ConvArgs {
     int Ho, Wo, Cout;
     int pad, pstep, act;
     int tiles_x, tiles_y;
-    // split over input channels: blockIdx.y = part * ctiles + channel tile; part p
-    // covers chunks [p*cpp, (p+1)*cpp) and writes raw FP32 sums to
-    // partial + p*part_stride (k_conv_finalize adds them in part order)
-    // flush > 0 (FP32, 64-pixel tiles): an unsplit layer that keeps a split's order
-    // of sums: every `flush` chunks the accumulators are added to the total
-    int ctiles, cpp, flush;
-    float* partial;
-    long long part_stride;
+    // packed weights: every `flush` chunks the accumulators are added to a total (0: never)
+    int flush;
 };
 
 template <int EK>
@@ -101,7 +98,7 @@ __device__ inline void conv_load4(const void* src, long long off, float v[4], in
     for (int r = 0; r < 4; ++r) v[r] += (r < nvalid) ? E::ld(p[r]) : 0.0f;
 }
 
-template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX, bool FLUSH>
+template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
 __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 {
     using E = Elem<EK>;
@@ -122,8 +119,7 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 
     const int tid = threadIdx.x, q = tid / 64, lane = tid % 64;
     const int l16 = lane % 16, lg = lane / 16;
-    const int n = blockIdx.z, kp = blockIdx.y / a.ctiles, nt0 = (blockIdx.y % a.ctiles) * NT;
-    const int cbeg = kp * a.cpp * KC, cend = min(a.Cin, (kp + 1) * a.cpp * KC);
+    const int n = blockIdx.z, nt0 = blockIdx.y * NT;
     int t = blockIdx.x;
     const int tx = t % a.tiles_x; t /= a.tiles_x;
     const int ty = t % a.tiles_y; t /= a.tiles_y;
@@ -143,7 +139,7 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
     // 1080p network's level-3 layers 13.5 us a launch, now 12.2)
     float bias[NT / 16][4];
     const float g = a.gate ? *a.gate : 1.0f;
-    const bool with_bias = a.bias && !a.partial;
+    const bool with_bias = a.bias;
 #pragma unroll
     for (int i = 0; i < NT / 16; ++i)
 #pragma unroll
@@ -242,45 +238,16 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d)
-        if (cbeg + d * KC < cend) fetch(cbeg + d * KC, rp[d], rw[d]);
-    [[maybe_unused]] cv_f32x4 total[NT / 16][MR];
-    [[maybe_unused]] int left = a.flush;
-    auto add_up = [&]() {
-#pragma unroll
-        for (int i = 0; i < NT / 16; ++i)
-#pragma unroll
-            for (int m = 0; m < MR; ++m) {
-                total[i][m] += acc[i][m];
-                acc[i][m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            }
-    };
-    if constexpr (FLUSH) {
-#pragma unroll
-        for (int i = 0; i < NT / 16; ++i)
-#pragma unroll
-            for (int m = 0; m < MR; ++m) total[i][m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    for (int c0 = cbeg; c0 < cend; c0 += DEPTH * KC) {
+        if (d * KC < a.Cin) fetch(d * KC, rp[d], rw[d]);
+    for (int c0 = 0; c0 < a.Cin; c0 += DEPTH * KC) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const int cc = c0 + d * KC;
-            if (cc >= cend) break;
+            if (cc >= a.Cin) break;
             stage(rp[d], rw[d]);
-            if (cc + DEPTH * KC < cend) fetch(cc + DEPTH * KC, rp[d], rw[d]);
+            if (cc + DEPTH * KC < a.Cin) fetch(cc + DEPTH * KC, rp[d], rw[d]);
             compute();
-            if constexpr (FLUSH) {
-                if (--left == 0 || cc + KC >= cend) {
-                    add_up();
-                    left = a.flush;
-                }
-            }
         }
-    }
-    if constexpr (FLUSH) {
-#pragma unroll
-        for (int i = 0; i < NT / 16; ++i)
-#pragma unroll
-            for (int m = 0; m < MR; ++m) acc[i][m] = total[i][m];
     }
 
     // epilogue: lane holds output channels nt0 + 16i + 4lg + r of pixel l16 of row q*MR+m
@@ -294,11 +261,6 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
             const int co = nt0 + i * 16 + 4 * lg;
             const int nv = min(4, a.Cout - co);
             if (nv <= 0) continue;
-            if (a.partial) {
-                float* d = a.partial + kp * a.part_stride + pix * a.Cout + co;
-                for (int r = 0; r < nv; ++r) d[r] = acc[i][m][r];
-                continue;
-            }
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -317,96 +279,272 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
     }
 }
 
-// sum of the split partials in part order, then the epilogue of k_conv3x3
-template <int EK, int EKO>
-__global__ void k_conv_finalize(ConvArgs a, int parts)
+// The same layers with packed weights (conv_pack_weights), for chunks of a whole
+// K step (32 channels, FP32 16): the flow network's layers.
+//
+// What bounded k_conv3x3 there is its weights' way from L2: a block's rows of 32
+// channels lie 9*Cin elements apart, which falls on a few of the L2's channels
+// (32 more input channels cost a 120x72x2 -> 128 layer 1.9 us at 17 MB), and
+// every block passed them through LDS besides.  Packed, a tap's weights of 16
+// output channels are 1 KB in the lanes' order: one coalesced load, straight to
+// registers.  So a wave owns 16 output channels of MR rows of 16 pixels, its nine
+// taps' weights stand in registers, and each is replaced by the next chunk's as
+// soon as its products are issued.  Only the input patch goes through LDS, two
+// buffers of it, so a chunk has one barrier, and a patch row's fragment is read
+// once for the taps of all three rows.  The loads are buffer loads that give
+// zeros past the end (the image's outside, the channels' tail) instead of
+// branches, so that the waits count the loads behind them.
+//
+// FLUSH: every `flush` chunks the accumulators are added to a total and cleared:
+// the order of sums of a channel loop split into parts, without the parts' way
+// through memory and the launch that adds them (5 us).
+//
+// Measured, us a layer (k_conv3x3 -> this): BF16 120x72x2 pixels, 128 -> 128
+// channels 16.9 -> 9.7, 256 -> 128 23.1 -> 13.3, 480x288 32 -> 32 24 -> 10.5;
+// FP32 120x72x2 256 -> 128 120 -> 79 (its products alone are 69), 160 -> 64
+// 55.8 -> 30.8, 15x9x2 256 -> 128 49 -> 12.6.  The network of a 1080p frame at
+// half size in BF16 533 -> 386 us, of a 640x360 frame in FP32 786 -> 672 us.
+template <int EK, int EKO, int S, int NT, int MR, bool FLUSH>
+__global__ __launch_bounds__(256) void k_conv3x3w(ConvArgs a)
 {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long total = (long long)a.N * a.Ho * a.Wo * a.Cout;
-    if (e >= total) return;
-    const int co = (int)(e % a.Cout);
-    const long long pix = e / a.Cout;
-    float x = 0.0f;
-    for (int k = 0; k < parts; ++k) x += a.partial[k * a.part_stride + e];
-    if (a.bias) x += a.bias[co];
-    if (a.act == 1) x = x > 0.0f ? x : x * 0.1f;
-    else if (a.act == 2) x = x > 0.0f ? x : 0.0f;
-    if (a.gate) x *= *a.gate;
-    using E = Elem<EKO>;
-    if (a.add) x += E::ld(static_cast<const typename E::T*>(a.add)[pix * a.add_cs + a.add_c0 + co]);
-    static_cast<typename E::T*>(a.out)[pix * a.out_cs + a.out_c0 + co] = E::st(x);
-    if (a.out2) static_cast<typename Elem<EK>::T*>(a.out2)[pix * a.out2_cs + a.out2_c0 + co] = Elem<EK>::st(x);
+    using E = Elem<EK>;
+    using T = typename E::T;
+    constexpr int VEC = E::VEC, KC = ConvK<EK>::KC, KV = 4;
+    static_assert(KC == KV * VEC, "four 16-byte vectors a pixel and chunk");
+    constexpr int WC = NT / 16, RG = 4 / WC;            // channel groups and row groups of the waves
+    constexpr int TH = RG * MR, TW = 16;
+    constexpr int PR = (TH - 1) * S + 3, PC = (TW - 1) * S + 3;
+    constexpr int ROW = KC + (EK == EK_F32 ? 0 : 2) * VEC;
+    constexpr int NP = PR * PC * KV, RP = (NP + 255) / 256;
+    constexpr int XR = (MR - 1) * S + 3;                // patch rows of a wave
+    __shared__ __attribute__((aligned(16))) T sP[2][PR * PC * ROW];
+
+    const int tid = threadIdx.x, lane = tid % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int q = wave / WC, wc = wave % WC;
+    const int l16 = lane % 16, lg = lane / 16;
+    const int n = blockIdx.z, nt0 = blockIdx.y * NT + wc * 16;
+    int t = blockIdx.x;
+    const int tx = t % a.tiles_x; t /= a.tiles_x;
+    const int ty = t % a.tiles_y; t /= a.tiles_y;
+    const int ps = a.pstep, py = t / ps, px = t % ps;
+    const int base_y = py - a.pad + ps * ty * TH * S, base_x = px - a.pad + ps * tx * TW * S;
+    // buffer loads: one past the end (NOWHERE) gives zeros, so no load is in a branch
+    // and the waits count the loads behind them
+    constexpr unsigned NOWHERE = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t in = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(static_cast<const T*>(a.in) + (long long)n * a.H * a.W * a.in_cs + a.in_c0), 0,
+        (int)((a.H * a.W * a.in_cs - a.in_c0) * sizeof(T)), 0x00020000);
+    const int chunks = (a.Cin + KC - 1) / KC, c16 = (a.Cout + 15) / 16;
+    const __amdgpu_buffer_rsrc_t wt = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.wtp), 0, c16 * chunks * 9 * 1024, 0x00020000);
+
+    cv_f32x4 acc[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) acc[m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const float g = a.gate ? *a.gate : 1.0f;
+    const bool with_bias = a.bias;
+    float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (with_bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bias[r] = a.bias[min(nt0 + 4 * lg + r, a.Cout - 1)];
+    }
+
+    const int cv = tid % KV * VEC;
+    unsigned off[RP];
+#pragma unroll
+    for (int k = 0; k < RP; ++k) {
+        const int p = (tid + 256 * k) / KV, r = p / PC, c = p % PC;
+        const int iy = base_y + ps * r, ix = base_x + ps * c;
+        off[k] = p < PR * PC && iy >= 0 && iy < a.H && ix >= 0 && ix < a.W ? ((iy * a.W + ix) * a.in_cs + cv) * sizeof(T) : NOWHERE;
+    }
+    cv_u32x4 rp[RP], w[9];
+    auto fetch = [&](int c0) {
+        const unsigned none = c0 + cv < a.Cin ? 0u : NOWHERE;
+#pragma unroll
+        for (int k = 0; k < RP; ++k)
+            rp[k] = __builtin_bit_cast(cv_u32x4, __builtin_amdgcn_raw_buffer_load_b128(in, off[k] | none, c0 * sizeof(T), 0));
+    };
+    const unsigned wlane = nt0 < a.Cout ? lane * 16u : NOWHERE, wfirst = nt0 < a.Cout ? nt0 / 16 * chunks * 9 * 1024u : 0u;
+    auto load_w = [&](int tap, int chunk) {
+        w[tap] = __builtin_bit_cast(cv_u32x4, __builtin_amdgcn_raw_buffer_load_b128(wt, wlane, wfirst + (chunk * 9 + tap) * 1024, 0));
+    };
+
+    // (the loop's order, for the waits' counts)
+    fetch(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap) load_w(tap, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    [[maybe_unused]] cv_f32x4 total[MR];
+    [[maybe_unused]] int left = a.flush;
+    if constexpr (FLUSH) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m) total[m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    int buf = 0;
+    for (int c0 = 0; c0 < a.Cin; c0 += KC, buf ^= 1) {
+        const bool more = c0 + KC < a.Cin;
+#pragma unroll
+        for (int k = 0; k < RP; ++k) {
+            const int u = tid + 256 * k;
+            if (u < NP) *reinterpret_cast<cv_u32x4*>(&sP[buf][(u / KV) * ROW + cv]) = rp[k];
+        }
+        // the LDS writes alone are waited for: the next chunk's loads stay in flight
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        fetch(c0 + KC);
+        const T* sp = &sP[buf][(q * MR * S * PC + l16 * S) * ROW + lg * VEC];
+        cv_u32x4 x[3][XR];
+        // rows of the tap's column that are not held yet
+        auto frag = [&](int tap) {
+            const int ky = tap / 3, kx = tap % 3;
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                const int r = m * S + ky;
+                if (ky >= S && m < MR - 1) continue;
+                x[kx][r] = *reinterpret_cast<const cv_u32x4*>(sp + (r * PC + kx) * ROW);
+            }
+        };
+        frag(0);
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            if (tap + 1 < 9) frag(tap + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) acc[m] = conv_mfma<EK>(w[tap], x[tap % 3][m * S + tap / 3], acc[m]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_w(tap, more ? c0 / KC + 1 : c0 / KC);
+        }
+        if constexpr (FLUSH) {
+            if (--left == 0 || !more) {
+#pragma unroll
+                for (int m = 0; m < MR; ++m) {
+                    total[m] += acc[m];
+                    acc[m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+                left = a.flush;
+            }
+        }
+    }
+
+    const int co = nt0 + 4 * lg, nv = min(4, a.Cout - co);
+    if (nv <= 0) return;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+        const int oy = py + ps * (ty * TH + q * MR + m), ox = px + ps * (tx * TW + l16);
+        if (oy >= a.Ho || ox >= a.Wo) continue;
+        const long long pix = ((long long)n * a.Ho + oy) * a.Wo + ox;
+        const cv_f32x4 s = FLUSH ? total[m] : acc[m];
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float y = with_bias ? s[r] + bias[r] : s[r];
+            const float low = a.act == 1 ? y * 0.1f : a.act == 2 ? 0.0f : y;
+            y = y > 0.0f ? y : low;
+            v[r] = a.gate ? y * g : y;
+        }
+        if (a.add) conv_load4<EKO>(a.add, pix * a.add_cs + a.add_c0 + co, v, nv);
+        conv_store4<EKO>(a.out, pix * a.out_cs + a.out_c0 + co, v, nv);
+        if constexpr (NT == 16)
+            if (a.out2) conv_store4<EK>(a.out2, pix * a.out2_cs + a.out2_c0 + co, v, nv);
+    }
 }
 
-// Parts a layer's channel loop is split into (1: unsplit), given its blocks per
-// batch item: when the grid leaves most CUs idle (FP32: under 128 blocks per
-// item; 16-bit: under 32, where the partial-sum traffic and the finalize launch
-// cost more than idle CUs down to that size, as measured on 1080p frames) and
-// the caller provided room for the partial sums.  The split depends on one batch
-// item's geometry and the room per item only, so an item's result has the same
-// bits alone and in a batch of any size.
+// Parts whose sums a packed layer of one batch item's `item_blocks` blocks (of
+// the tiles that k_conv3x3 would take) keeps apart: what a split over the idle
+// CUs would give, bounded by kConvPartFloats of partial sums an item.  It
+// depends on one item's geometry only, so an item's result has the same bits
+// alone and in a batch of any size.
+constexpr long long kConvPartFloats = 2LL << 20;
 template <int EK>
 static int conv_parts(const ConvArgs& a, long long item_blocks, int chunks)
 {
-    if (!a.partial || chunks < 2 || item_blocks >= (EK == EK_F32 ? 128 : 32)) return 1;
+    if (chunks < 2 || item_blocks >= (EK == EK_F32 ? 128 : 32)) return 1;
     const long long item_stride = (long long)a.Ho * a.Wo * a.Cout;
     int parts = (int)std::min<long long>(chunks, (256 + item_blocks - 1) / item_blocks);
-    parts = (int)std::min<long long>(parts, a.part_stride / std::max<long long>(item_stride, 1));
+    parts = (int)std::min<long long>(parts, kConvPartFloats / std::max<long long>(item_stride, 1));
     if (parts < 2) return 1;
     const int cpp = (chunks + parts - 1) / parts;
     return (chunks + cpp - 1) / cpp;
 }
 
-// Modelled time (us) of an FP32 layer of 64-pixel tiles, `blocks` blocks of `w`
-// channels before the split, `chunks` chunks in `parts` parts: a chunk costs
-// 0.042 us per channel + 4 of the fullest CU's blocks (its MFMAs) but at least
-// 0.8 us (its way through LDS), a split 5.5 us for the launch that adds the parts
-// (fitted on the layers of a 640x360 frame).
-static double conv_split_cost(long long blocks, int w, int chunks, int parts)
-{
-    const long long full = (blocks * parts + 255) / 256;
-    return ((chunks + parts - 1) / parts) * std::max(0.8, 0.042 * full * (w + 4)) + (parts > 1 ? 5.5 : 0.0);
-}
-
 template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
-static void conv_go(const ConvArgs& a, int split_nt, hipStream_t s)
+static void conv_go(const ConvArgs& a, hipStream_t s)
 {
-    constexpr int KC = KCX;
     const int ps = a.pstep;
     ConvArgs b = a;
     const int hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
     b.tiles_y = (hs + NW * MR - 1) / (NW * MR);
     b.tiles_x = (ws + 15) / 16;
-    b.ctiles = (a.Cout + NT - 1) / NT;
-    const int chunks = (a.Cin + KC - 1) / KC;
-    const long long item_px = (long long)b.tiles_x * b.tiles_y * ps * ps;
-    const long long stride = (long long)a.Ho * a.Wo * a.Cout * a.N;
-    const int parts = conv_parts<EK>(a, item_px * ((a.Cout + split_nt - 1) / split_nt), chunks);
-    b.cpp = (chunks + parts - 1) / parts;
-    if constexpr (EK == EK_F32 && MR == 1) {
-        if (parts > 1 && conv_split_cost(item_px * b.ctiles * a.N, NT, chunks, 1) < conv_split_cost(item_px * b.ctiles * a.N, NT, chunks, parts)) {
-            b.flush = b.cpp;
-            b.cpp = chunks;
-            b.partial = nullptr;
-            dim3 grid(b.tiles_x * b.tiles_y * ps * ps, b.ctiles, a.N);
-            hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, true>), grid, dim3(64 * NW), 0, s, b);
-            return;
+    dim3 grid(b.tiles_x * b.tiles_y * ps * ps, (a.Cout + NT - 1) / NT, a.N);
+    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX>), grid, dim3(64 * NW), 0, s, b);
+}
+
+template <int EK, int EKO, int S, int NT, int MR>
+static void conv_gow(const ConvArgs& a, hipStream_t s)
+{
+    constexpr int TH = 4 / (NT / 16) * MR;
+    ConvArgs b = a;
+    const int ps = a.pstep, hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
+    b.tiles_y = (hs + TH - 1) / TH;
+    b.tiles_x = (ws + 15) / 16;
+    dim3 grid(b.tiles_x * b.tiles_y * ps * ps, (a.Cout + NT - 1) / NT, a.N);
+    if (a.flush) {
+        if constexpr (MR <= 3) hipLaunchKernelGGL((k_conv3x3w<EK, EKO, S, NT, MR, true>), grid, dim3(256), 0, s, b);
+    } else {
+        hipLaunchKernelGGL((k_conv3x3w<EK, EKO, S, NT, MR, false>), grid, dim3(256), 0, s, b);
+    }
+}
+
+// Tile of a packed layer: the (channels, rows of a wave) of least modelled time a
+// chunk, `full` blocks standing on the fullest CU.  FP32: the products bound it,
+// 0.51 us a row and block and 0.06 a block.  16-bit: a block takes 0.26 + 0.045
+// MR us (its loads and its barrier) but at least 0.1 MR beside others and 0.13
+// MR alone.  (Fitted on 26 layers x 15 tiles, within 10% of the best tile on
+// each; 120x72x2, 128 -> 128, BF16: 32 channels x 3 rows 11.0 us, 768 blocks, x 4
+// 11.3, 576 blocks, 64 x 5 9.7, 480 blocks.)
+template <int EK, int EKO, int S>
+static void conv_packed(const ConvArgs& a, hipStream_t s)
+{
+    struct Tile {
+        int nt, mr;
+        void (*go)(const ConvArgs&, hipStream_t);
+    };
+    static const Tile narrow[] = {{16, 1, conv_gow<EK, EKO, S, 16, 1>}, {16, 2, conv_gow<EK, EKO, S, 16, 2>}};
+    static const Tile wide[] = {
+        {64, 1, conv_gow<EK, EK, S, 64, 1>}, {64, 2, conv_gow<EK, EK, S, 64, 2>}, {64, 3, conv_gow<EK, EK, S, 64, 3>},
+        {32, 1, conv_gow<EK, EK, S, 32, 1>}, {32, 2, conv_gow<EK, EK, S, 32, 2>}, {32, 3, conv_gow<EK, EK, S, 32, 3>},
+        {64, 4, conv_gow<EK, EK, S, 64, 4>}, {32, 4, conv_gow<EK, EK, S, 32, 4>}, {64, 5, conv_gow<EK, EK, S, 64, 5>},
+        {64, 6, conv_gow<EK, EK, S, 64, 6>}};
+    const int ps = a.pstep;
+    const long long hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
+    const Tile* first = a.Cout <= 16 ? narrow : wide;
+    const Tile* last = a.Cout <= 16 ? std::end(narrow) : std::end(wide);
+    const Tile* best = nullptr;
+    double least = 1e300;
+    for (const Tile* t = first; t != last; ++t) {
+        if (a.flush && t->mr > 3) continue;
+        if (a.Cout <= 32 && t->nt > 32) continue;
+        const int th = 64 / t->nt * t->mr;
+        const long long blocks = (hs + th - 1) / th * ((ws + 15) / 16) * ps * ps * ((a.Cout + t->nt - 1) / t->nt) * a.N;
+        const double full = (double)((blocks + 255) / 256), m = t->mr;
+        const double cost = EK == EK_F32 ? full * (0.51 * m + 0.06)
+                                         : std::max(std::max(full * (0.26 + 0.045 * m), full * 0.1 * m), 0.13 * m);
+        if (cost < least * 0.999) {
+            least = cost;
+            best = t;
         }
     }
-    b.partial = parts > 1 ? a.partial : nullptr;
-    b.part_stride = stride;
-    dim3 grid(b.tiles_x * b.tiles_y * ps * ps, b.ctiles * parts, a.N);
-    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, false>), grid, dim3(64 * NW), 0, s, b);
-    if (parts > 1)
-        hipLaunchKernelGGL((k_conv_finalize<EK, EKO>), dim3((unsigned)((stride + 255) / 256)), dim3(256), 0, s, b, parts);
+    best->go(a, s);
 }
 
 template <int EK, int EKO, int S, int NT, int KCX>
-static void conv_mr(const ConvArgs& a, int mr, int split_nt, hipStream_t s)
+static void conv_mr(const ConvArgs& a, int mr, hipStream_t s)
 {
-    if (mr == 4) conv_go<EK, EKO, S, NT, (S == 1 ? 4 : 2), 4, KCX>(a, split_nt, s);
-    else if (mr == 2) conv_go<EK, EKO, S, NT, 2, 4, KCX>(a, split_nt, s);
-    else conv_go<EK, EKO, S, NT, 1, 4, KCX>(a, split_nt, s);
+    if (mr == 4) conv_go<EK, EKO, S, NT, (S == 1 ? 4 : 2), 4, KCX>(a, s);
+    else if (mr == 2) conv_go<EK, EKO, S, NT, 2, 4, KCX>(a, s);
+    else conv_go<EK, EKO, S, NT, 1, 4, KCX>(a, s);
 }
 
 // Tile choice.  Channel tile: FP32 layers take the widest tile they fill (64,
@@ -428,44 +566,50 @@ static void conv_pick(const ConvArgs& a, hipStream_t s)
     auto blocks = [&](int mr) { return (px / (64LL * mr)) * ntiles; };
     int mr = (S == 1 && blocks(4) >= 512) ? 4 : (blocks(2) >= (EK == EK_F32 ? 512 : 128) ? 2 : 1);
     if (S == 2 && mr > 2) mr = 2;
+    if constexpr (EK != EK_F16) {
+        if (a.wtp) {
+            ConvArgs b = a;
+            const int chunks = (a.Cin + ConvK<EK>::KC - 1) / ConvK<EK>::KC;
+            const long long hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
+            const long long tiles = (hs + 4 * mr - 1) / (4 * mr) * ((ws + 15) / 16) * ps * ps;
+            const int parts = conv_parts<EK>(a, tiles * ntiles, chunks);
+            b.flush = parts > 1 ? (chunks + parts - 1) / parts : 0;
+            conv_packed<EK, EKO, S>(b, s);
+            return;
+        }
+    }
     constexpr int KC = ConvK<EK>::KC;
     if constexpr (EK == EK_F32) {
         // Layers of 64-pixel tiles: the widest channel tiles are the cheapest a
-        // channel, but on a grid of a few blocks per CU the fullest CU decides
-        // (288 blocks are two on 32 of the 256 CUs), 96 channels leave a quarter
-        // of two 64-channel tiles empty, and narrow tiles can do without a split.
-        // So the width of least modelled time, split or not.  (80x48 pixels, 2
-        // items, 128 -> 128 channels: 46 us with 64 channels, 31 with 16; 256 -> 96:
-        // 52 + 5 with 64 split, 37 with 16 unsplit.)  The order of sums is the
-        // widest tiles' split in every case, so the choice leaves the bits alone.
+        // channel, but on a grid of a few blocks per CU the fullest CU decides, and
+        // 96 channels leave a quarter of two 64-channel tiles empty.  So the width of
+        // least (blocks on the fullest CU) x (channels + 4).
         int nt = NTsel;
         if (mr == 1) {
             const long long item = (((a.Ho + ps - 1) / ps + 3) / 4) * (((a.Wo + ps - 1) / ps + 15) / 16) * (long long)ps * ps;
-            const int chunks = (a.Cin + KC - 1) / KC, parts = conv_parts<EK>(a, item * ntiles, chunks);
-            double best = 1e300;
+            long long best = 1LL << 62;
             for (int w = NTsel; w >= 16; w /= 2) {
-                const long long blocks = item * ((a.Cout + w - 1) / w) * a.N;
-                const double cost = std::min(conv_split_cost(blocks, w, chunks, 1), conv_split_cost(blocks, w, chunks, parts));
-                if (cost < best - 1e-9) {
+                const long long cost = (item * ((a.Cout + w - 1) / w) * a.N + 255) / 256 * (w + 4);
+                if (cost < best) {
                     best = cost;
                     nt = w;
                 }
             }
         }
-        if (nt == 64) conv_mr<EK, EKO, S, 64, KC>(a, mr, NTsel, s);
-        else if (nt == 32) conv_mr<EK, EKO, S, 32, KC>(a, mr, NTsel, s);
-        else conv_mr<EK, EKO, S, 16, KC>(a, mr, NTsel, s);
+        if (nt == 64) conv_mr<EK, EKO, S, 64, KC>(a, mr, s);
+        else if (nt == 32) conv_mr<EK, EKO, S, 32, KC>(a, mr, s);
+        else conv_mr<EK, EKO, S, 16, KC>(a, mr, s);
     } else {
         // layers with 8 or 16 input channels (the image and the first feature
         // level) stage chunks of that width
         if (NTsel == 32) {
-            if (a.Cin <= 8) conv_mr<EK, EKO, S, 32, 8>(a, mr, NTsel, s);
-            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 32, 16>(a, mr, NTsel, s);
-            else conv_mr<EK, EKO, S, 32, KC>(a, mr, NTsel, s);
+            if (a.Cin <= 8) conv_mr<EK, EKO, S, 32, 8>(a, mr, s);
+            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 32, 16>(a, mr, s);
+            else conv_mr<EK, EKO, S, 32, KC>(a, mr, s);
         } else {
-            if (a.Cin <= 8) conv_mr<EK, EKO, S, 16, 8>(a, mr, NTsel, s);
-            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 16, 16>(a, mr, NTsel, s);
-            else conv_mr<EK, EKO, S, 16, KC>(a, mr, NTsel, s);
+            if (a.Cin <= 8) conv_mr<EK, EKO, S, 16, 8>(a, mr, s);
+            else if (a.Cin <= 16) conv_mr<EK, EKO, S, 16, 16>(a, mr, s);
+            else conv_mr<EK, EKO, S, 16, KC>(a, mr, s);
         }
     }
 }
@@ -475,6 +619,36 @@ static void conv_stride(const ConvArgs& a, int stride, hipStream_t s)
 {
     if (stride == 2) conv_pick<EK, EKO, 2>(a, s);
     else conv_pick<EK, EKO, 1>(a, s);
+}
+
+// whole K steps of channels (16-bit layers of 8 or 16 channels put several taps
+// into one instead), an item that a buffer descriptor spans
+bool conv_takes_packed(int ek_in, int ek_out, int cin, int cout, long long item_elements)
+{
+    const int eb = ek_in == EK_F32 ? 4 : 2;
+    return ek_in != EK_F16 && (ek_in == EK_F32 || cin > 16) && (ek_out == ek_in || cout <= 16) && item_elements * eb < (1LL << 31);
+}
+
+static int packed_chunks(int cin, int elem_bytes) { return (cin * elem_bytes + 63) / 64; }
+
+size_t conv_packed_bytes(int cout, int cin, int elem_bytes)
+{
+    return (size_t)((cout + 15) / 16) * packed_chunks(cin, elem_bytes) * 9 * 1024;
+}
+
+void conv_pack_weights(const void* w, void* out, int cout, int cin, int elem_bytes)
+{
+    const int chunks = packed_chunks(cin, elem_bytes), vec = 16 / elem_bytes;
+    char* o = static_cast<char*>(out);
+    for (int ct = 0; ct < (cout + 15) / 16; ++ct)
+        for (int ch = 0; ch < chunks; ++ch)
+            for (int tap = 0; tap < 9; ++tap)
+                for (int lane = 0; lane < 64; ++lane, o += 16) {
+                    const int co = ct * 16 + lane % 16, ci = (ch * 4 + lane / 16) * vec;
+                    const int n = co < cout ? std::max(0, std::min(vec, cin - ci)) : 0;
+                    memset(o, 0, 16);
+                    if (n) memcpy(o, static_cast<const char*>(w) + (((size_t)co * 9 + tap) * cin + ci) * elem_bytes, (size_t)n * elem_bytes);
+                }
 }
 
 int launch_conv3x3(const ConvDesc& d, hipStream_t s)
@@ -507,13 +681,13 @@ int launch_conv3x3(const ConvDesc& d, hipStream_t s)
     ConvArgs a{};
     a.in = d.in.p; a.in_cs = d.in.cs; a.in_c0 = d.in.c0;
     a.N = d.in.n; a.H = d.in.h; a.W = d.in.w; a.Cin = d.in.c;
-    a.wt = d.wt; a.bias = d.bias;
+    a.wt = d.wt; a.wtp = d.wtp; a.bias = d.bias;
+    if (d.wtp && !conv_takes_packed(ek, eko, d.in.c, Cout, (long long)d.in.h * d.in.w * d.in.cs))
+        return set_error(VSC_E_INVALID, "conv3x3: packed weights for a layer that does not take them");
     a.out = d.out.p; a.out_cs = d.out.cs; a.out_c0 = d.out.c0;
     a.out2 = d.out2.p; a.out2_cs = d.out2.cs; a.out2_c0 = d.out2.c0;
     a.add = d.add.p; a.add_cs = d.add.cs; a.add_c0 = d.add.c0;
     a.gate = d.gate;
-    a.partial = d.partial;
-    a.part_stride = (long long)d.partial_cap;   // capacity per item in floats; conv_go turns it into the part stride
     a.Ho = Ho; a.Wo = Wo; a.Cout = Cout;
     a.pad = d.pad; a.pstep = d.dil; a.act = d.act;
     if (ek == EK_F32) conv_stride<EK_F32, EK_F32>(a, d.stride, s);
@@ -545,4 +719,32 @@ extern "C" int vsc_conv3x3_nhwc(const void* in, int in_cs, int in_c0, int N, int
     d.stride = stride; d.dil = dilation; d.pad = pad; d.act = act;
     d.ek_in = elem_kind(dtype); d.ek_out = elem_kind(out_dtype);
     return launch_conv3x3(d, as_stream(stream));
+}
+
+// Diagnostic (no declaration in vsc.h): a layer with packed weights.  wt: host
+// [Cout][3][3][Cin] in the element type, packed and uploaded for the call;
+// the output's pixel stride is its channels, input pixels hold Cin channels.
+extern "C" int vsct_conv3x3_packed(const void* in, int N, int H, int W, int Cin, const void* wt, const float* bias,
+                                   void* out, int Cout, int stride, int dilation, int act, int dtype, int out_dtype,
+                                   vsc_hip_stream stream)
+{
+    using namespace vsc;
+    const int eb = dtype == VSC_F32 ? 4 : 2;
+    std::vector<char> pk(conv_packed_bytes(Cout, Cin, eb));
+    conv_pack_weights(wt, pk.data(), Cout, Cin, eb);
+    void* dev = nullptr;
+    int rc = check_hip(hipMalloc(&dev, pk.size()), "vsct_conv3x3_packed");
+    if (rc) return rc;
+    if (!(rc = check_hip(hipMemcpy(dev, pk.data(), pk.size(), hipMemcpyHostToDevice), "vsct_conv3x3_packed"))) {
+        ConvDesc d{};
+        d.in = Nhwc{const_cast<void*>(in), N, H, W, Cin, Cin, 0};
+        d.out = Nhwc{out, N, (H - 1) / stride + 1, (W - 1) / stride + 1, Cout, Cout, 0};
+        d.wtp = dev; d.bias = bias;
+        d.stride = stride; d.dil = dilation; d.pad = dilation; d.act = act;
+        d.ek_in = elem_kind(dtype); d.ek_out = elem_kind(out_dtype);
+        rc = launch_conv3x3(d, as_stream(stream));
+    }
+    (void)hipDeviceSynchronize();
+    (void)hipFree(dev);
+    return rc;
 }

@@ -34,7 +34,6 @@ constexpr int kDecC = 456;                                  // dec channels: 448
 constexpr int kRefIn0 = 416, kRefInC = 40;
 constexpr int kRefOut[7] = {128, 128, 128, 96, 64, 32, 2};
 constexpr int kRefDil[7] = {1, 2, 4, 8, 16, 1, 1};
-constexpr size_t kPartialFloatsPerItem = (size_t)2 << 20;  // 8 MB of FP32 partial sums per batch item
 
 inline int rup(int x, int m) { return (x + m - 1) / m * m; }
 
@@ -62,7 +61,8 @@ struct Layer {
     std::vector<int> cmap;   // reference input channel -> padded position (conv layers)
     int cin_pad;             // padded input channels of the device weights
     std::vector<float> w, b; // reference layout (host)
-    void* dw = nullptr;      // device weights: conv [cout][3][3][cin_pad] (element kind), upflow FP32 reference layout
+    bool packed = false;     // conv: the device weights are packed (conv_pack_weights)
+    void* dw = nullptr;      // device weights: conv [cout][3][3][cin_pad] or packed (element kind), upflow FP32 reference layout
     float* db = nullptr;     // device bias
 };
 
@@ -86,9 +86,6 @@ struct vsc_flownet {
     float* flow[7] = {};                  // per level [pairs][h][w][2]
     float* refined = nullptr;             // [pairs][h3][w3][2]
     void* rbuf[2] = {nullptr, nullptr};   // refiner ping-pong [pairs][h3][w3][128]
-    float* partial = nullptr;             // split-channel partial sums of the small decoder layers
-    float* partial_x = nullptr;           // the same for the extractor ([frames] items): extraction and
-                                          // decoding may run on two streams at once
     std::vector<void*> owned;
     int last_pairs = 0;
 };
@@ -104,6 +101,8 @@ void add_conv(vsc_flownet* n, int cin, int cout, int stride, int dil, int act, c
     Layer l;
     l.cin = cin; l.cout = cout; l.k = 3; l.stride = stride; l.dil = dil; l.act = act;
     l.cmap = cmap; l.cin_pad = cin_pad;
+    // no tensor of the network has more elements an item than 8 times its input's pixels
+    l.packed = conv_takes_packed(n->ek, n->ek, cin_pad, cout, 8LL * n->Hp * n->Wp);
     n->L.push_back(l);
 }
 
@@ -173,6 +172,12 @@ size_t param_count_of(const vsc_flownet* n)
     return c;
 }
 
+size_t weight_bytes(const vsc_flownet* n, const Layer& l)
+{
+    if (l.k == 4) return l.w.size() * 4;
+    return l.packed ? conv_packed_bytes(l.cout, l.cin_pad, n->eb) : (size_t)l.cout * 9 * l.cin_pad * n->eb;
+}
+
 int upload_params(vsc_flownet* n)
 {
     for (Layer& l : n->L) {
@@ -185,13 +190,20 @@ int upload_params(vsc_flownet* n)
                 for (int ci = 0; ci < l.cin; ++ci)
                     for (int t = 0; t < 9; ++t)
                         p[((size_t)co * 9 + t) * l.cin_pad + l.cmap[ci]] = l.w[((size_t)co * l.cin + ci) * 9 + t];
-            if (n->ek == EK_F32) {
-                if (check_hip(hipMemcpy(l.dw, p.data(), p.size() * 4, hipMemcpyHostToDevice), "flownet upload")) return VSC_E_HIP;
-            } else {
-                std::vector<uint16_t> h(p.size());
+            std::vector<uint16_t> h;
+            const void* src = p.data();
+            if (n->ek != EK_F32) {
+                h.resize(p.size());
                 for (size_t j = 0; j < p.size(); ++j) h[j] = f32_to_bf16(p[j]);
-                if (check_hip(hipMemcpy(l.dw, h.data(), h.size() * 2, hipMemcpyHostToDevice), "flownet upload")) return VSC_E_HIP;
+                src = h.data();
             }
+            std::vector<char> pk;
+            if (l.packed) {
+                pk.resize(weight_bytes(n, l));
+                conv_pack_weights(src, pk.data(), l.cout, l.cin_pad, n->eb);
+                src = pk.data();
+            }
+            if (check_hip(hipMemcpy(l.dw, src, weight_bytes(n, l), hipMemcpyHostToDevice), "flownet upload")) return VSC_E_HIP;
         }
         if (check_hip(hipMemcpy(l.db, l.b.data(), l.b.size() * 4, hipMemcpyHostToDevice), "flownet upload")) return VSC_E_HIP;
     }
@@ -223,8 +235,7 @@ Sizes sizes_of(const vsc_flownet* n)
     z.rbuf = px3 * 128 * eb;
     z.weights = 0;
     for (const Layer& l : n->L)
-        z.weights += (l.k == 4 ? l.w.size() * 4 : (size_t)l.cout * 9 * l.cin_pad * eb) + l.b.size() * 4 + 512;
-    z.weights += kPartialFloatsPerItem * (n->pairs + n->frames) * 4;
+        z.weights += weight_bytes(n, l) + l.b.size() * 4 + 512;
     return z;
 }
 
@@ -268,10 +279,8 @@ int alloc_all(vsc_flownet* n)
     n->refined = static_cast<float*>(dalloc(n, z.refined, rc));
     n->rbuf[0] = dalloc(n, z.rbuf, rc);
     n->rbuf[1] = dalloc(n, z.rbuf, rc);
-    n->partial = static_cast<float*>(dalloc(n, kPartialFloatsPerItem * n->pairs * 4, rc));
-    n->partial_x = static_cast<float*>(dalloc(n, kPartialFloatsPerItem * n->frames * 4, rc));
     for (Layer& l : n->L) {
-        l.dw = dalloc(n, l.k == 4 ? l.w.size() * 4 : (size_t)l.cout * 9 * l.cin_pad * n->eb, rc);
+        l.dw = dalloc(n, weight_bytes(n, l), rc);
         l.db = static_cast<float*>(dalloc(n, l.b.size() * 4, rc));
     }
     return rc;
@@ -282,19 +291,17 @@ void* feat_ptr(vsc_flownet* n, int slot, int lvl)
     return static_cast<char*>(n->feat[lvl]) + (size_t)slot * (n->Hp >> lvl) * (n->Wp >> lvl) * cv_of(n, lvl) * n->eb;
 }
 
-int conv(vsc_flownet* n, const Layer& l, Nhwc in, Nhwc out, Nhwc add, int ek_out, hipStream_t s, Nhwc out2 = Nhwc{},
-         float* partial = nullptr)
+int conv(vsc_flownet* n, const Layer& l, Nhwc in, Nhwc out, Nhwc add, int ek_out, hipStream_t s, Nhwc out2 = Nhwc{})
 {
-    // the device weights are [cout][3][3][cin_pad]: the slices must match them exactly
+    // the device weights hold cin_pad input channels: the slices must match them exactly
     if (in.c != l.cin_pad || out.c != l.cout || (add.p && add.c != l.cout))
         return set_error(VSC_E_INVALID, "flownet: layer slice does not match its weights");
     ConvDesc d{};
     d.in = in; d.out = out; d.add = add; d.out2 = out2;
-    d.wt = l.dw; d.bias = l.db;
+    (l.packed ? d.wtp : d.wt) = l.dw;
+    d.bias = l.db;
     d.stride = l.stride; d.dil = l.dil; d.pad = l.dil; d.act = l.act;
     d.ek_in = n->ek; d.ek_out = ek_out;
-    d.partial = partial ? partial : n->partial;
-    d.partial_cap = kPartialFloatsPerItem;
     return launch_conv3x3(d, s);
 }
 
@@ -322,12 +329,9 @@ int extract(vsc_flownet* n, const uint8_t* const* rgba, int m, int slot, hipStre
         // outputs carry the layer's channel count; as inputs the slices include
         // the zero padding channels up to the 16-byte multiple
         const int co = kFeatC[k];
-        float* px = n->partial_x;
-        if ((rc = conv(n, l[0], x, T(a, m, h, w, co, cv, 0), Nhwc{}, n->ek, s, Nhwc{}, px))) return rc;
-        if ((rc = conv(n, l[1], T(a, m, h, w, cv, cv, 0), T(b, m, h, w, co, cv, 0), Nhwc{}, n->ek, s, Nhwc{}, px)))
-            return rc;
-        if ((rc = conv(n, l[2], T(b, m, h, w, cv, cv, 0), T(c, m, h, w, co, cv, 0), Nhwc{}, n->ek, s, Nhwc{}, px)))
-            return rc;
+        if ((rc = conv(n, l[0], x, T(a, m, h, w, co, cv, 0), Nhwc{}, n->ek, s))) return rc;
+        if ((rc = conv(n, l[1], T(a, m, h, w, cv, cv, 0), T(b, m, h, w, co, cv, 0), Nhwc{}, n->ek, s))) return rc;
+        if ((rc = conv(n, l[2], T(b, m, h, w, cv, cv, 0), T(c, m, h, w, co, cv, 0), Nhwc{}, n->ek, s))) return rc;
         x = T(c, m, h, w, cv, cv, 0);
     }
     return VSC_OK;

@@ -394,14 +394,20 @@ struct ConvDesc {
     Nhwc in, out, add;   // add.p == nullptr: no residual
     Nhwc out2;           // out2.p == nullptr: none; else a second copy of the result in the input's element kind (Cout <= 16)
     const void* wt;      // [Cout][3][3][in.c], element kind of in
+    const void* wtp;     // nullptr, or the weights packed (conv_pack_weights) in place of wt
     const float* bias;   // [Cout] or nullptr
     const float* gate;   // nullptr, or a device scalar multiplying the activated result before `add`
     int stride, dil, pad, act;
     int ek_in, ek_out;
-    float* partial;      // optional FP32 scratch: small layers split their channel loop into it
-    size_t partial_cap;  // scratch capacity in floats per batch item (the scratch holds in.n items' worth)
 };
 int launch_conv3x3(const ConvDesc& d, hipStream_t s);
+// Weights in the order the lanes of k_conv3x3w read them: [16 output channels][K
+// step of input channels][tap][lane][16 bytes], zeros beyond either end.  `w` and
+// `out`: bytes of [Cout][3][3][cin] and conv_packed_bytes of packed elements.
+size_t conv_packed_bytes(int cout, int cin, int elem_bytes);
+// whether a layer may take them; an item: one batch item's pixels times its pixel stride
+bool conv_takes_packed(int ek_in, int ek_out, int cin, int cout, long long item_elements);
+void conv_pack_weights(const void* w, void* out, int cout, int cin, int elem_bytes);
 
 // the flow network with room for `pairs` (1 .. 8) (first, second) pairs per
 // decode (vsc_flownet_create: 2)
