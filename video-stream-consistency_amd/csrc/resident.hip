@@ -14,6 +14,14 @@
 // (DPP), up and down neighbours from the lane's own registers, and from LDS at
 // the waves' first and last rows: one barrier per sweep.
 //
+// Strips.  A level too large for the chip is swept in rounds of up to some tens
+// of sweeps; in a round, strips of rows are resident one after the other, each
+// with as many rows beyond its own as the round has sweeps (those rows' values
+// go wrong from the cut inwards, a row a sweep, and are not kept).  O and U go
+// through memory once a round.  A 3840x2160 frame of 150 and 75 sweeps: 2553 us
+// against 3787 with the blocked solver on level 0, a 2560x1440 one 1211 against
+// 1595, one of 2000x1125 898 against 985.
+//
 // The image's edges cost no branches: a wave shift brings 0 into lanes 0 and
 // 63, so a tile flush with the image's left or right edge sees the missing
 // neighbour as +0 (which changes no nonzero sum), the first wave's upper and
@@ -48,10 +56,11 @@ namespace vsc {
 namespace {
 
 // control words of a stream (device memory, all zero at rest)
-enum { CTL_ABORT = 0, CTL_EXIT = 16, CTL_TICKET = 32, CTL_FEXIT = 48, CTL_FLAGS = 64, CTL_STRIDE = 16 };
-constexpr int RES_MAX_TILES = 1024;
+enum { CTL_ABORT = 0, CTL_EXIT = 16, CTL_TICKET = 32, CTL_FEXIT = 48, CTL_FLAGS = 64, CTL_STRIDE = 16, CTL_FSTRIDE = 4 };
+constexpr int RES_MAX_TILES = 1024, FIN_MAX_TILES = 4096;
 constexpr int RES_NW = 8;   // waves of a block
-static_assert((CTL_FLAGS + RES_MAX_TILES * CTL_STRIDE) * 4 <= RESIDENT_CTL_BYTES, "control block size");
+static_assert((CTL_FLAGS + RES_MAX_TILES * CTL_STRIDE) * 4 <= RESIDENT_CTL_BYTES &&
+              (CTL_FLAGS + FIN_MAX_TILES * CTL_FSTRIDE) * 4 <= RESIDENT_CTL_BYTES, "control block size");
 // 100 MHz ticks: 3 ms, several times the longest kernel of a frame
 constexpr long long RES_WAIT_TICKS = 300000;
 
@@ -64,8 +73,12 @@ struct ResArgs {
     const float* A;       // reference order: the adapted processed frame
     const float* Oin;
     float* Oout;
+    const float* Uin;     // null: zero (the level's first sweeps)
+    float* Uout;          // null: not kept (its last ones)
     float* X[2][2];       // exchange planes: [set][0] holds O, [set][1] holds U
-    int W, H, iters, h, nx, ny, per_xcd;
+    long long plane;      // elements of a channel's plane (of all but X)
+    int own0, own1;       // rows that are the launch's to write
+    int W, H, iters, h, nx, ny, per_xcd;   // H: rows of the region that the launch sweeps
     float step, mom;
     unsigned* ctl;
 };
@@ -148,7 +161,7 @@ __global__ __launch_bounds__(64 * NW, (8 / NW) * NW / 4) void k_consist_resident
     unsigned* flags = a.ctl + CTL_FLAGS;
 
     if (tid == 0) s_go = ld_agent(a.ctl + CTL_ABORT) == 0u;   // given up already?
-    const long long plane = (long long)a.W * a.H;
+    const long long plane = (long long)a.W * a.H;              // of X; what a launch reaches of the other planes
     const int row0 = wv * R;                                   // the wave's first row in the tile
     const int base = (gy0 + row0) * a.W + gx0 + PX * lane;     // element offset of the lane's first pixel
     __syncthreads();
@@ -157,8 +170,8 @@ __global__ __launch_bounds__(64 * NW, (8 / NW) * NW / 4) void k_consist_resident
         V o[R], u[R], q[R], ad[FMA ? 1 : R];   // FMA form: ad unused
         {
             // (buffer accesses: one offset register for all rows) k first, through registers that o, q and u take afterwards
-            const __amdgpu_buffer_rsrc_t O_ = plane_rsrc(a.Oin + c * plane, plane), Q_ = plane_rsrc(a.Q + c * plane, plane);
-            const __amdgpu_buffer_rsrc_t K_ = plane_rsrc(a.K + c * plane, plane), A_ = plane_rsrc(a.A + c * plane, plane);
+            const __amdgpu_buffer_rsrc_t O_ = plane_rsrc(a.Oin + c * a.plane, plane), Q_ = plane_rsrc(a.Q + c * a.plane, plane);
+            const __amdgpu_buffer_rsrc_t K_ = plane_rsrc(a.K + c * a.plane, plane), A_ = plane_rsrc(a.A + c * a.plane, plane);
 #pragma unroll
             for (int r = 0; r < R; ++r)
                 *reinterpret_cast<V*>(&sK[row0 + r][PX * lane]) = load_px<PX, 0>(K_, base * 4, r * a.W * 4);
@@ -169,6 +182,11 @@ __global__ __launch_bounds__(64 * NW, (8 / NW) * NW / 4) void k_consist_resident
                 q[r] = load_px<PX, 0>(Q_, base * 4, r * a.W * 4);
                 if constexpr (!FMA) ad[r] = load_px<PX, 0>(A_, base * 4, r * a.W * 4);
                 u[r] = V{};
+            }
+            if (a.Uin) {
+                const __amdgpu_buffer_rsrc_t U_ = plane_rsrc(a.Uin + c * a.plane, plane);
+#pragma unroll
+                for (int r = 0; r < R; ++r) u[r] = load_px<PX, 0>(U_, base * 4, r * a.W * 4);
             }
         }
         // columns and rows whose values are exact after h sweeps
@@ -355,13 +373,15 @@ __global__ __launch_bounds__(64 * NW, (8 / NW) * NW / 4) void k_consist_resident
             }
         }
         if (go) {
-            const __amdgpu_buffer_rsrc_t Oo = plane_rsrc(a.Oout + c * plane, plane);
+            const __amdgpu_buffer_rsrc_t Oo = plane_rsrc(a.Oout + c * a.plane, plane);
+            const __amdgpu_buffer_rsrc_t Uo = plane_rsrc(a.Uout + c * a.plane, plane);
             if (lane_exact) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const int y = row0 + r;
-                    if (y < ye0 || y >= ye1) continue;
+                    if (y < ye0 || y >= ye1 || gy0 + y < a.own0 || gy0 + y >= a.own1) continue;
                     store_px<PX, 0>(o[r], Oo, base * 4, r * a.W * 4);
+                    if (a.Uout) store_px<PX, 0>(u[r], Uo, base * 4, r * a.W * 4);
                 }
             }
         }
@@ -384,7 +404,7 @@ struct FinishArgs {
     const float* A;
     float* O[2];
     float* U[2];
-    int W, H, iters, halo, nx, ny, phases;
+    int W, H, iters, halo, nx, ny, phases, base;   // base: the level's sweeps before these
     float step, mom;
     unsigned* ctl;
     unsigned* note;       // host word: a resident launch was given up
@@ -409,7 +429,7 @@ __global__ __launch_bounds__(SB_TW * SB_STRIPS) void k_consist_finish(FinishArgs
             if (tid < 25) {   // the 5 x 5 tiles around: the last tile of a row overlaps two before it
                 const int dx = tid % 5 - 2, dy = tid / 5 - 2;
                 if (tx + dx >= 0 && tx + dx < a.nx && ty + dy >= 0 && ty + dy < a.ny)
-                    while (ld_agent(flags + (tile + dy * a.nx + dx) * CTL_STRIDE) < (unsigned)ph) __builtin_amdgcn_s_sleep(8);
+                    while (ld_agent(flags + (tile + dy * a.nx + dx) * CTL_FSTRIDE) < (unsigned)ph) __builtin_amdgcn_s_sleep(8);
             }
             __syncthreads();
             if (tid < 64) __threadfence();   // drops this CU's and this XCD's stale lines
@@ -417,11 +437,11 @@ __global__ __launch_bounds__(SB_TW * SB_STRIPS) void k_consist_finish(FinishArgs
         }
         const int first = ph * a.halo, n = min(a.halo, a.iters - first);
         consist_tile<R, SB_STRIPS, FMA>(a.K, a.A, a.Q, a.O[ph & 1], a.O[(ph + 1) & 1], a.U[ph & 1], a.U[(ph + 1) & 1],
-                                        a.W, a.H, n, first, a.step, a.mom, a.halo, a.nx, a.ny, 1, tile, sO);
+                                        a.W, a.H, n, a.base + first, a.step, a.mom, a.halo, a.nx, a.ny, 1, tile, sO);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tid < 64) __threadfence();       // writes this XCD's lines back
-        if (tid == 0) st_agent(flags + tile * CTL_STRIDE, (unsigned)(ph + 1));
+        if (tid == 0) st_agent(flags + tile * CTL_FSTRIDE, (unsigned)(ph + 1));
         // keeps this branch apart from the next turn's: merged by the compiler, thread 0 would leave the others' loop
         __syncthreads();
     }
@@ -429,7 +449,7 @@ __global__ __launch_bounds__(SB_TW * SB_STRIPS) void k_consist_finish(FinishArgs
     if (tid == 0) s_t = atomicAdd(a.ctl + CTL_FEXIT, 1u) == gridDim.x - 1u;
     __syncthreads();
     if (s_t) {
-        for (int i = tid; i < ntiles; i += SB_TW * SB_STRIPS) st_agent(flags + i * CTL_STRIDE, 0u);
+        for (int i = tid; i < ntiles; i += SB_TW * SB_STRIPS) st_agent(flags + i * CTL_FSTRIDE, 0u);
         if (tid == 0) {
             st_agent(a.ctl + CTL_TICKET, 0u);
             st_agent(a.ctl + CTL_FEXIT, 0u);
@@ -502,54 +522,95 @@ bool plan_resident(int W, int H, int iters, int cus, int fma, ResidentPlan* out)
             const double cost = phases * (1.6 + 0.2 * k.r) + iters * (0.25 + (fma ? 0.0253 : 0.042) * k.px * k.r);
             if (cost < best) {
                 best = cost;
-                *out = ResidentPlan{v, h, nx, ny};
+                *out = ResidentPlan{v, h, nx, ny, 1, 1, H};
             }
         }
     }
     return best < 1e299;
 }
 
+// halo and phases of the ticket form for a round of `iters` sweeps: odd, so that
+// it ends in the planes that the resident form writes
+static void finish_phases(int W, int H, int iters, int fma, int* halo, int* phases)
+{
+    const BlockedPlan bp = plan_consist_blocked(W, H, iters, fma);
+    for (int k = (iters + bp.halo - 1) / bp.halo;; ++k) {
+        *halo = (iters + k - 1) / k;
+        *phases = (iters + *halo - 1) / *halo;
+        if (*phases % 2 == 1) break;
+    }
+}
+static int finish_tiles(int W, int H, int halo, int fma)
+{
+    return 3 * tile_count(W, SB_TW, halo) * tile_count(H, SB_STRIPS * (fma ? SB_R_FMA : SB_R), halo);
+}
+
+// The rounds, strips and tile shape of least modelled time for a level that does
+// not fit at once.  A launch costs what plan_resident says and its way in and
+// out, at 7.5 TB/s and 3 us; it has to beat the blocked solver's 0.88 us
+// (reference order 1.15) a sweep and million values.  The exchange planes, four
+// of a region's size, lie in A and P (reference order: P alone, A being read), or
+// one in each of U, U, P and A when a single round leaves U alone.
+bool plan_resident_strips(int W, int H, int iters, int cus, int fma, ResidentPlan* out)
+{
+    if (iters < 1 || W > 65535 || H > 65535) return false;
+    const double px = 3.0 * W * H;
+    double best = 0.95 * iters * px * (fma ? 0.88e-6 : 1.15e-6);
+    bool found = false;
+    for (int rounds = 1; rounds <= 8 && rounds <= iters; ++rounds) {
+        const int sweeps = (iters + rounds - 1) / rounds;
+        if ((iters + sweeps - 1) / sweeps != rounds) continue;
+        for (int strips = 2; strips <= 12; ++strips) {
+            const int own = (H + strips - 1) / strips, rows = std::min(H, own + 2 * sweeps);
+            if ((fma ? (rounds == 1 ? 1 : 2) : 4) * rows > H || (long long)W * rows >= (1LL << 28)) continue;
+            for (int v = 0; v < (int)(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
+                const Variant& k = kVariants[v];
+                if (k.fma != fma || k.px < 4) continue;   // large levels fill the chip with large tiles
+                for (int h = 4; h <= 16; h += 4) {
+                    const int nx = res_count(W, 64 * k.px, h, 4), ny = res_count(rows, RES_NW * k.r, h, 1);
+                    const long long tiles = 3LL * nx * ny;
+                    if (tiles == 0 || tiles > cus || tiles > RES_MAX_TILES) continue;
+                    const double io = (tiles * 512.0 * k.px * k.r * (fma ? 16 : 20) + 24.0 * W * own) / 7.5e6 + 3.0;
+                    const double one = (sweeps + h - 1) / h * (1.6 + 0.2 * k.r) + sweeps * (0.25 + (fma ? 0.0253 : 0.042) * k.px * k.r);
+                    if (rounds * strips * (one + io) < best) {
+                        best = rounds * strips * (one + io);
+                        *out = ResidentPlan{v, h, nx, ny, rounds, strips, rows};
+                        found = true;
+                    }
+                }
+            }
+        }
+    }
+    if (!found) return false;
+    for (int r = 0, first = 0; r < out->rounds; ++r) {   // the ticket form has room for every round
+        const int n = std::min((iters + out->rounds - 1) / out->rounds, iters - first);
+        int halo, phases;
+        finish_phases(W, H, n, fma, &halo, &phases);
+        if (finish_tiles(W, H, halo, fma) > FIN_MAX_TILES) return false;
+        first += n;
+    }
+    return true;
+}
+
 int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_t s)
 {
     const int fma = kVariants[plan.variant].fma;
-    // the ticket form's phases: odd, so that it ends in O[1] as the resident form does
-    const BlockedPlan bp = plan_consist_blocked(l.W, l.H, l.iters, fma);
+    const long long plane = (long long)l.W * l.H;
     FinishArgs f{};
-    for (int k = (l.iters + bp.halo - 1) / bp.halo;; ++k) {
-        f.halo = (l.iters + k - 1) / k;
-        f.phases = (l.iters + f.halo - 1) / f.halo;
-        if (f.phases % 2 == 1) break;
-    }
     f.K = l.K;
     f.Q = l.Q;
     f.A = l.A;
     f.W = l.W;
     f.H = l.H;
-    f.iters = l.iters;
     f.step = l.step;
     f.mom = l.mom;
     f.ctl = l.ctl;
     f.note = l.note;
-    f.nx = tile_count(l.W, SB_TW, f.halo);
-    f.ny = tile_count(l.H, SB_STRIPS * (fma ? SB_R_FMA : SB_R), f.halo);
-    if (3 * f.nx * f.ny > RES_MAX_TILES) return set_error(VSC_E_INVALID, "resident solver: too many tiles");
     ResArgs a{};
-    a.K = l.K;
-    a.Q = l.Q;
     a.A = l.A;
-    a.Oin = l.O[0];
-    a.Oout = l.O[1];
-    a.X[0][0] = l.U[0];
-    a.X[0][1] = l.U[1];
-    a.X[1][0] = l.O[1];
-    a.X[1][1] = l.P;
-    for (int i = 0; i < 2; ++i) {
-        f.O[i] = l.O[i];
-        f.U[i] = l.U[i];
-    }
+    a.plane = plane;
     a.W = l.W;
-    a.H = l.H;
-    a.iters = l.iters;
+    a.H = plan.rows;
     a.h = plan.h;
     a.nx = plan.nx;
     a.ny = plan.ny;
@@ -557,6 +618,20 @@ int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_
     a.step = l.step;
     a.mom = l.mom;
     a.ctl = l.ctl;
+    if (plan.strips > 1) {
+        const long long region = 3LL * l.W * plan.rows;
+        const bool alone = fma && plan.rounds == 1;
+        float* second = fma ? const_cast<float*>(l.A) : l.P + 2 * region;
+        a.X[0][0] = l.P;
+        a.X[0][1] = alone ? l.U[0] : l.P + region;
+        a.X[1][0] = second;
+        a.X[1][1] = alone ? l.U[1] : second + region;
+    } else {
+        a.X[0][0] = l.U[0];
+        a.X[0][1] = l.U[1];
+        a.X[1][0] = l.O[1];
+        a.X[1][1] = l.P;
+    }
     // after the resident launch before it on this device, whatever its stream
     int dev = 0, rc;
     if ((rc = check_hip(hipGetDevice(&dev), "resident solver"))) return rc;
@@ -570,9 +645,38 @@ int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_
     }
     // algorithmic bytes: read O and the per-pixel constants and write O once
     const int slot = prof_start(PROF_CONSIST_BLOCKED, (fma ? 4.0 : 5.0) * 3 * 4 * (double)l.W * l.H, s);
-    kVariants[plan.variant].go(a, s);
-    if (fma) hipLaunchKernelGGL((k_consist_finish<SB_R_FMA, true>), dim3(256), dim3(SB_TW * SB_STRIPS), 0, s, f);
-    else hipLaunchKernelGGL((k_consist_finish<SB_R, false>), dim3(256), dim3(SB_TW * SB_STRIPS), 0, s, f);
+    const int sweeps = (l.iters + plan.rounds - 1) / plan.rounds, own = (l.H + plan.strips - 1) / plan.strips;
+    for (int r = 0, first = 0; r < plan.rounds; ++r, first += sweeps) {
+        const int from = r & 1, n = std::min(sweeps, l.iters - first);
+        a.iters = n;
+        for (int k = 0; k < plan.strips; ++k) {
+            const int y0 = std::min(k * own, l.H), y1 = std::min(y0 + own, l.H);
+            if (y0 == y1) break;
+            const int top = std::max(0, std::min(y0 - sweeps, l.H - plan.rows));   // the region's first row
+            const long long at = (long long)top * l.W;
+            a.K = l.K + at;
+            a.Q = l.Q + at;
+            if (!fma) a.A = l.A + at;
+            a.Oin = l.O[from] + at;
+            a.Oout = l.O[from ^ 1] + at;
+            a.Uin = r > 0 ? l.U[from] + at : nullptr;
+            a.Uout = r + 1 < plan.rounds ? l.U[from ^ 1] + at : nullptr;
+            a.own0 = y0 - top;
+            a.own1 = y1 - top;
+            kVariants[plan.variant].go(a, s);
+        }
+        finish_phases(l.W, l.H, n, fma, &f.halo, &f.phases);
+        f.nx = tile_count(l.W, SB_TW, f.halo);
+        f.ny = tile_count(l.H, SB_STRIPS * (fma ? SB_R_FMA : SB_R), f.halo);
+        f.iters = n;
+        f.base = first;
+        for (int i = 0; i < 2; ++i) {
+            f.O[i] = l.O[from ^ i];
+            f.U[i] = l.U[from ^ i];
+        }
+        if (fma) hipLaunchKernelGGL((k_consist_finish<SB_R_FMA, true>), dim3(256), dim3(SB_TW * SB_STRIPS), 0, s, f);
+        else hipLaunchKernelGGL((k_consist_finish<SB_R, false>), dim3(256), dim3(SB_TW * SB_STRIPS), 0, s, f);
+    }
     prof_stop(slot, s);
     if ((rc = check_launch("consist_resident"))) return rc;
     return check_hip(hipEventRecord(turn.ev, s), "resident solver");
@@ -593,5 +697,20 @@ extern "C" int vsct_resident_plan(int W, int H, int iters, int cus, int fma, int
     for (int i = 0; i < 5; ++i) out[i] = v[i];
     for (int i = 0; i < p.nx; ++i) xs[i] = res_start(i, p.nx, W, tw, 4);
     for (int i = 0; i < p.ny; ++i) ys[i] = res_start(i, p.ny, H, th, 1);
+    return 1;
+}
+
+// Diagnostic (no declaration in vsc.h): the same for a level swept in strips;
+// out also holds the rounds, the strips and a region's rows.
+extern "C" int vsct_resident_strips(int W, int H, int iters, int cus, int fma, int* out, int* xs, int* ys)
+{
+    using namespace vsc;
+    ResidentPlan p;
+    if (!plan_resident_strips(W, H, iters, cus, fma, &p)) return 0;
+    const int tw = 64 * kVariants[p.variant].px, th = RES_NW * kVariants[p.variant].r;
+    const int v[8] = {tw, th, p.h, p.nx, p.ny, p.rounds, p.strips, p.rows};
+    for (int i = 0; i < 8; ++i) out[i] = v[i];
+    for (int i = 0; i < p.nx; ++i) xs[i] = res_start(i, p.nx, W, tw, 4);
+    for (int i = 0; i < p.ny; ++i) ys[i] = res_start(i, p.ny, p.rows, th, 1);
     return 1;
 }

@@ -36,6 +36,12 @@ struct vsc_stream {
     volatile unsigned* note = nullptr;
     int cus = 0, skip = 0, backoff = 0;
     bool shared = false;
+    // the levels' resident plans of the last frame's form and sweeps
+    struct {
+        int iters = -1, fma = -1;
+        bool ok = false;
+        vsc::ResidentPlan plan{};
+    } planned[VSC_MAX_LEVELS];
     // staged (per-stage reference sequence) images, allocated on first use
     void* staged_block = nullptr;
     float* st[32] = {};
@@ -330,14 +336,14 @@ bool resident_frame(vsc_stream* s, const vsc_params& p, hipStream_t st)
 }
 
 // The buffer of O[j] in which level j starts.  The blocked solver starts in 0
-// and swaps at every launch; a resident level 0 starts where its one swap ends
-// in the same buffer, so that the two forms may alternate between frames and
+// and swaps at every launch; a resident level 0 (swaps: its rounds) starts where
+// it ends in the same buffer, so that the two forms may alternate between frames and
 // in captured graphs.
-int level_start(const vsc_stream* s, int j, int iters, int fma, bool resident)
+int level_start(const vsc_stream* s, int j, int iters, int fma, int swaps)
 {
-    if (!resident || j > 0) return 0;
+    if (!swaps || j > 0) return 0;
     const int halo = plan_consist_blocked(s->lw[0], s->lh[0], iters, fma).halo;
-    return ((iters + halo - 1) / halo & 1) ^ 1;
+    return ((iters + halo - 1) / halo ^ swaps) & 1;
 }
 
 // Pyramid solve, levels L-1 .. 0 (videostabilizer.cpp:219-227): a level that
@@ -350,7 +356,7 @@ int solve_pyramid(vsc_stream* s, int L, const vsc_params& p, int fma, const Resi
     for (int j = L - 1; j >= 0; --j) {
         const int w = s->lw[j], h = s->lh[j];
         const int iters = p.num_iter / (j + 1);
-        int rc, cur = level_start(s, j, iters, fma, resident[j]);
+        int rc, cur = level_start(s, j, iters, fma, resident[j] ? res[j].rounds : 0);
         if (j != L - 1) {
             rc = launch_bilinear(pl(s->O[j + 1][*final_idx], s->lw[j + 1], s->lh[j + 1]), pl(s->O[j][cur], w, h), st);
             if (rc) return rc;
@@ -359,7 +365,7 @@ int solve_pyramid(vsc_stream* s, int L, const vsc_params& p, int fma, const Resi
             ResidentLevel l{s->L[j], s->Wt[j], s->A[j], {s->O[j][cur], s->O[j][cur ^ 1]}, {s->U[j][0], s->U[j][1]},
                             s->P[j], w, h, iters, p.step_size, p.mom_fac, s->ctl, const_cast<unsigned*>(s->note)};
             if ((rc = launch_resident(l, res[j], st))) return rc;
-            *final_idx = cur ^ 1;
+            *final_idx = (cur ^ res[j].rounds) & 1;
             continue;
         }
         const BlockedPlan plan = plan_consist_blocked(w, h, iters, fma);
@@ -444,10 +450,21 @@ int frame_fused(vsc_stream* s, const vsc_frame_in* in, const vsc_params& p, uint
     ResidentPlan rplan[VSC_MAX_LEVELS];
     bool resident[VSC_MAX_LEVELS] = {};
     if (resident_frame(s, p, st))
-        for (int j = 0; j < L; ++j) resident[j] = plan_resident(s->lw[j], s->lh[j], p.num_iter / (j + 1), s->cus, fma, &rplan[j]);
+        for (int j = 0; j < L; ++j) {
+            auto& k = s->planned[j];
+            const int iters = p.num_iter / (j + 1);
+            if (k.iters != iters || k.fma != fma) {
+                k.ok = plan_resident(s->lw[j], s->lh[j], iters, s->cus, fma, &k.plan) ||
+                       plan_resident_strips(s->lw[j], s->lh[j], iters, s->cus, fma, &k.plan);
+                k.iters = iters;
+                k.fma = fma;
+            }
+            resident[j] = k.ok;
+            rplan[j] = k.plan;
+        }
     if (L == 1) {
         // single level: the solution starts at the processed frame (videostabilizer.cpp:209)
-        const int start = level_start(s, 0, p.num_iter, fma, resident[0]);
+        const int start = level_start(s, 0, p.num_iter, fma, resident[0] ? rplan[0].rounds : 0);
         if ((rc = launch_copy_view(pl(s->P[0], W, H), pl(s->O[0][start], W, H), st))) return rc;
     }
     int fin = 0;

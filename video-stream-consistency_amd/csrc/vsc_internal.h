@@ -240,12 +240,13 @@ int launch_consist_blocked(const float* lapP, const float* A, const float* Wt, c
 int launch_fma_consts(float* L, const float* A, float* Wt, int W, int H, float step, hipStream_t s);
 // One pyramid level solved with its tiles resident on the chip (resident.hip);
 // K, Q, A: k, q and unused (FMA form) or lapP, w, A (reference order).  O[0]
-// holds the initial solution, O[1] receives the result; U and P are scratch of
-// a level's size; ctl: RESIDENT_CTL_BYTES of device memory of the stream's
+// holds the initial solution, O[rounds & 1] receives the result; U, P and, in the
+// FMA form, A are scratch of a level's size; ctl: RESIDENT_CTL_BYTES of device memory of the stream's
 // own, zero at rest.
 constexpr size_t RESIDENT_CTL_BYTES = 66 << 10;
 struct ResidentPlan {
     int variant, h, nx, ny;
+    int rounds, strips, rows;   // 1, 1, H when the level fits at once; rows: of a strip's region
 };
 struct ResidentLevel {
     const float* K;
@@ -261,6 +262,8 @@ struct ResidentLevel {
 };
 // false when no tiling of the level fits `cus` compute units at once
 bool plan_resident(int W, int H, int iters, int cus, int fma, ResidentPlan* out);
+// a level that does not: false where the blocked solver is the faster one
+bool plan_resident_strips(int W, int H, int iters, int cus, int fma, ResidentPlan* out);
 int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_t s);
 // a stream whose frames run beside other work on purpose (overlapped pipelines,
 // the server): its solver leaves CUs free between launches (blocked form only)
