@@ -1,3 +1,4 @@
+import gc
 import importlib
 import os
 import sys
@@ -12,6 +13,13 @@ if ROOT not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP kernels through the C ABI)")
+
+
+def pytest_runtest_setup(item):
+    # objects that earlier tests left in reference cycles give their device memory back here, not in
+    # the middle of a test's graph capture (a free while a stream is captured invalidates the capture)
+    if item.get_closest_marker("gpu"):
+        gc.collect()
 
 
 @pytest.fixture(scope="session")
