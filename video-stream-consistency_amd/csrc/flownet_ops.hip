@@ -65,7 +65,7 @@ __device__ inline fo_f32x4 corr_mma(const fo_u32x4& a, const fo_u32x4& b, fo_f32
 template <int EK, bool BFMM, int DG>
 __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
 {
-    static_assert(DG == 9 || DG == 3, "all displacements, or a third of them");
+    static_assert(DG == 9 || DG == 3 || DG == 1, "all displacements, a third of them or one");
     static_assert(!BFMM || EK == EK_F32, "BF16 products of FP32 storage only");
     using E = Elem<EK>;
     using T = typename E::T;
@@ -99,32 +99,37 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
 #pragma unroll
         for (int t = 0; t < 2; ++t) acc[d][t] = fo_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
+    // Staging: a thread's vectors keep their pixels and channel offset for the whole
+    // call.  Buffer loads give zeros outside the image and past the channels (offset
+    // NOWHERE), so that no load is in a branch and the waits leave the chunks behind
+    // in flight.
     constexpr int DEPTH = DG == 9 ? 1 : 2;
+    constexpr unsigned NOWHERE = 0x80000000u;
+    const __amdgpu_buffer_rsrc_t F1 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(f1), 0, (int)((((long long)a.H * a.W - 1) * a.cs1 + a.C) * sizeof(T)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t F2 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(f2), 0, (int)((((long long)a.H * a.W - 1) * a.cs2 + a.C) * sizeof(T)), 0x00020000);
+    // units of the f1 tile first, in whole rows of threads (NA is a multiple of 512)
+    static_assert(NA % 512 == 0, "a thread's unit k is of one tile for all threads");
+    const int cv = tid % KV * VEC;
+    unsigned off[RU];
     fo_u32x4 regs[DEPTH][RU];
-    auto fetch = [&](int c0, fo_u32x4 (&rg)[RU]) {
 #pragma unroll
-        for (int k = 0; k < RU; ++k) {
-            const int u = tid + 512 * k;
-            fo_u32x4 v = fo_u32x4{0u, 0u, 0u, 0u};
-            if (u < NA) {
-                const int p = u / KV, cv = u % KV, r = p / RP, x = p % RP;
-                const int gh = h0 + r, gw = w0 + x, ch = c0 + cv * VEC;
-                if (gh < a.H && gw < a.W && ch < a.C) {
-                    v = *reinterpret_cast<const fo_u32x4*>(f1 + ((long long)gh * a.W + gw) * a.cs1 + ch);
-                    // the decoder's concatenation takes f1 beside the cost volume
-                    // (pwcnet.py:578): every block stages its own pixels' f1 once
-                    if (copy_f1)
-                        *reinterpret_cast<fo_u32x4*>(static_cast<T*>(a.out) +
-                                                     (((long long)n * a.H + gh) * a.W + gw) * a.ocs + a.f1_c0 + ch) = v;
-                }
-            } else if (u < NU) {
-                const int ub = u - NA, p = ub / KV, cv = ub % KV, r = p / BP, x = p % BP;
-                const int gh = h0 - HALO + d0 + r, gw = w0 - HALO + x, ch = c0 + cv * VEC;
-                if (gh >= 0 && gh < a.H && gw >= 0 && gw < a.W && ch < a.C)
-                    v = *reinterpret_cast<const fo_u32x4*>(f2 + ((long long)gh * a.W + gw) * a.cs2 + ch);
-            }
-            rg[k] = v;
+    for (int k = 0; k < RU; ++k) {
+        const int u = tid + 512 * k;
+        if (u < NA) {
+            const int p = u / KV, gh = h0 + p / RP, gw = w0 + p % RP;
+            off[k] = gh < a.H && gw < a.W ? (unsigned)(((gh * a.W + gw) * a.cs1 + cv) * sizeof(T)) : NOWHERE;
+        } else {
+            const int p = (u - NA) / KV, gh = h0 - HALO + d0 + p / BP, gw = w0 - HALO + p % BP;
+            off[k] = u < NU && gh >= 0 && gh < a.H && gw >= 0 && gw < a.W ? (unsigned)(((gh * a.W + gw) * a.cs2 + cv) * sizeof(T)) : NOWHERE;
         }
+    }
+    auto fetch = [&](int c0, fo_u32x4 (&rg)[RU]) {
+        const unsigned none = c0 + cv < a.C ? 0u : NOWHERE;
+#pragma unroll
+        for (int k = 0; k < RU; ++k)
+            rg[k] = __builtin_bit_cast(fo_u32x4, __builtin_amdgcn_raw_buffer_load_b128(512 * k < NA ? F1 : F2, off[k] | none, c0 * sizeof(T), 0));
     };
 
     auto chunk = [&](int c0, fo_u32x4 (&rg)[RU]) {
@@ -133,6 +138,13 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
         for (int k = 0; k < RU; ++k) {
             const int u = tid + 512 * k;
             if (u >= NU) continue;
+            // the decoder's concatenation takes f1 beside the cost volume
+            // (pwcnet.py:578): every block stages its own pixels' f1 once
+            if (512 * k < NA && copy_f1 && off[k] != NOWHERE && c0 + cv < a.C) {
+                const int p = u / KV;
+                *reinterpret_cast<fo_u32x4*>(static_cast<T*>(a.out) +
+                                             (((long long)n * a.H + h0 + p / RP) * a.W + w0 + p % RP) * a.ocs + a.f1_c0 + c0 + cv) = rg[k];
+            }
             M* dst = u < NA ? &sA[(u / KV) * ROW + (u % KV) * VEC] : &sB[((u - NA) / KV) * ROW + ((u - NA) % KV) * VEC];
             if constexpr (BFMM) {
                 // 4 FP32 channels -> 4 BF16 (round to nearest even)
@@ -146,7 +158,7 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
             }
         }
         __syncthreads();
-        if (c0 + DEPTH * KC < a.C) fetch(c0 + DEPTH * KC, rg);
+        fetch(c0 + DEPTH * KC, rg);
         const fo_u32x4 fa = *reinterpret_cast<const fo_u32x4*>(&sA[(qr * RP + 16 * seg + l16) * ROW + lg * (KC / 4)]);
 #pragma unroll
         for (int d = 0; d < DG; ++d) {
@@ -159,8 +171,10 @@ __global__ __launch_bounds__(512) void k_corr_nhwc(CorrArgs a)
         }
     };
 #pragma unroll
-    for (int i = 0; i < DEPTH; ++i)
-        if (i * KC < a.C) fetch(i * KC, regs[i]);
+    for (int i = 0; i < DEPTH; ++i) {
+        fetch(i * KC, regs[i]);
+        __builtin_amdgcn_sched_barrier(0);   // the loop's order, for the waits' counts
+    }
     for (int c0 = 0; c0 < a.C; c0 += DEPTH * KC) {
 #pragma unroll
         for (int i = 0; i < DEPTH; ++i)
@@ -224,14 +238,21 @@ int launch_corr_nhwc(int ek, const void* const* f1, const void* const* f2, int c
     for (int i = 0; i < N; ++i) { a.f1[i] = f1[i]; a.f2[i] = f2[i]; }
     a.cs1 = cs1; a.cs2 = cs2; a.C = C; a.H = H; a.W = W; a.out = out; a.ocs = ocs;
     a.f1_c0 = f1_c0;
+    if ((long long)H * W * std::max(cs1, cs2) * (ek == EK_F32 ? 4 : 2) >= (1LL << 31))
+        return set_error(VSC_E_INVALID, "corr nhwc: tensor too large");
     if (f1_c0 >= 0 && f1_c0 + C > ocs) return set_error(VSC_E_INVALID, "corr nhwc: f1 copy outside the pixel");
-    // thirds of the displacements while whole blocks would not give every CU two
-    const bool thirds = (long long)((W + 31) / 32) * ((H + 3) / 4) * N < 512;
-    dim3 grid((W + 31) / 32, (H + 3) / 4, thirds ? 3 * N : N);
-    auto go = [&](auto whole, auto third) { hipLaunchKernelGGL(thirds ? third : whole, grid, dim3(512), 0, s, a); };
-    if (ek == EK_BF16) go(k_corr_nhwc<EK_BF16, false, 9>, k_corr_nhwc<EK_BF16, false, 3>);
-    else if (bf16_products) go(k_corr_nhwc<EK_F32, true, 9>, k_corr_nhwc<EK_F32, true, 3>);
-    else go(k_corr_nhwc<EK_F32, false, 9>, k_corr_nhwc<EK_F32, false, 3>);
+    // one displacement row a block while all those blocks fit the chip at once (FP32
+    // 10x6x196: 21.7 us in thirds, 11 in ninths; a 640x360 frame's FP32 network 663
+    // and 648 us), thirds while whole blocks would not give every CU two
+    const long long tiles = (long long)((W + 31) / 32) * ((H + 3) / 4) * N;
+    const int groups = 9 * tiles <= 256 ? 9 : tiles < 512 ? 3 : 1;
+    dim3 grid((W + 31) / 32, (H + 3) / 4, groups * N);
+    auto go = [&](auto whole, auto third, auto ninth) {
+        hipLaunchKernelGGL(groups == 1 ? whole : groups == 3 ? third : ninth, grid, dim3(512), 0, s, a);
+    };
+    if (ek == EK_BF16) go(k_corr_nhwc<EK_BF16, false, 9>, k_corr_nhwc<EK_BF16, false, 3>, k_corr_nhwc<EK_BF16, false, 1>);
+    else if (bf16_products) go(k_corr_nhwc<EK_F32, true, 9>, k_corr_nhwc<EK_F32, true, 3>, k_corr_nhwc<EK_F32, true, 1>);
+    else go(k_corr_nhwc<EK_F32, false, 9>, k_corr_nhwc<EK_F32, false, 3>, k_corr_nhwc<EK_F32, false, 1>);
     return check_launch("corr nhwc");
 }
 
@@ -409,37 +430,50 @@ __device__ inline void resize_tap(int dst, int in, int out, int& i0, int& i1, fl
     lam = src - (float)i0;
 }
 
+template <int EK> __device__ inline uint32_t bits_of(float v)
+{
+    if constexpr (EK == EK_F32) return __builtin_bit_cast(uint32_t, v);
+    else return (uint32_t)Elem<EK>::st(v);
+}
+
 template <int EK>
 __global__ void k_preprocess(const uint8_t* __restrict__ rgba, int W, int H, int Wd, int Hd, int Wp, int Hp,
-                             void* out, int ocs)
+                             void* out)
 {
-    using E = Elem<EK>;
+    // b / 255 of every byte (a division a thread instead of twelve)
+    __shared__ float s_unit[256];
+    s_unit[threadIdx.x] = (float)threadIdx.x / 255.0f;
+    __syncthreads();
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y;
     if (x >= Wp || y >= Hp) return;
     int x0, x1, y0, y1;
     float lx, ly;
     resize_tap(x, Wd, Wp, x0, x1, lx);
     resize_tap(y, Hd, Hp, y0, y1, ly);
-    auto src = [&](int xd, int yd, int c) {
+    typedef uint32_t Px __attribute__((aligned(1)));
+    auto src = [&](int xd, int yd) {
         const int xs = Wd == W ? xd : min(W - 1, (int)(((float)xd + 0.5f) * ((float)W / (float)Wd)));
         const int ys = Hd == H ? yd : min(H - 1, (int)(((float)yd + 0.5f) * ((float)H / (float)Hd)));
-        return (float)rgba[((long long)ys * W + xs) * 4 + c] / 255.0f;
+        return *reinterpret_cast<const Px*>(rgba + ((long long)ys * W + xs) * 4);
     };
-    typename E::T* o = static_cast<typename E::T*>(out) + ((long long)y * Wp + x) * ocs;
-    for (int c = 0; c < 3; ++c) {
-        const float v = (1.0f - ly) * ((1.0f - lx) * src(x0, y0, c) + lx * src(x1, y0, c)) +
-                        ly * ((1.0f - lx) * src(x0, y1, c) + lx * src(x1, y1, c));
-        o[c] = E::st(v);
-    }
-    for (int c = 3; c < ocs; ++c) o[c] = E::st(0.0f);
+    const uint32_t p00 = src(x0, y0), p10 = src(x1, y0), p01 = src(x0, y1), p11 = src(x1, y1);
+    auto value = [&](int c) {
+        auto unit = [&](uint32_t p) { return s_unit[p >> (8 * c) & 255u]; };
+        return (1.0f - ly) * ((1.0f - lx) * unit(p00) + lx * unit(p10)) + ly * ((1.0f - lx) * unit(p01) + lx * unit(p11));
+    };
+    // three channels and zeros, 16 bytes a pixel
+    const uint32_t r = bits_of<EK>(value(0)), g = bits_of<EK>(value(1)), b = bits_of<EK>(value(2));
+    const fo_u32x4 v = EK == EK_F32 ? fo_u32x4{r, g, b, 0u} : fo_u32x4{r | g << 16, b, 0u, 0u};
+    reinterpret_cast<fo_u32x4*>(out)[(long long)y * Wp + x] = v;
 }
 
 int launch_preprocess(int ek, const uint8_t* rgba, int W, int H, int Wd, int Hd, int Wp, int Hp, void* out, int ocs,
                       hipStream_t s)
 {
+    if (ocs * (ek == EK_F32 ? 4 : 2) != 16) return set_error(VSC_E_INVALID, "preprocess: pixels of 16 bytes");
     dim3 grid((Wp + 255) / 256, Hp);
-    if (ek == EK_BF16) hipLaunchKernelGGL(k_preprocess<EK_BF16>, grid, dim3(256), 0, s, rgba, W, H, Wd, Hd, Wp, Hp, out, ocs);
-    else hipLaunchKernelGGL(k_preprocess<EK_F32>, grid, dim3(256), 0, s, rgba, W, H, Wd, Hd, Wp, Hp, out, ocs);
+    if (ek == EK_BF16) hipLaunchKernelGGL(k_preprocess<EK_BF16>, grid, dim3(256), 0, s, rgba, W, H, Wd, Hd, Wp, Hp, out);
+    else hipLaunchKernelGGL(k_preprocess<EK_F32>, grid, dim3(256), 0, s, rgba, W, H, Wd, Hd, Wp, Hp, out);
     return check_launch("preprocess");
 }
 
@@ -467,23 +501,23 @@ __global__ void k_flow_final(const float* __restrict__ flows, int h, int w, int 
     // align_corners = True upsample of the level flow, evaluated at (X, Y) of the Hp x Wp grid
     const float sx = w > 1 ? (float)(w - 1) / (float)(Wp - 1) : 0.0f;
     const float sy = h > 1 ? (float)(h - 1) / (float)(Hp - 1) : 0.0f;
-    auto up = [&](int X, int Y, int c) {
+    typedef float F2 __attribute__((ext_vector_type(2)));
+    typedef float F2U __attribute__((ext_vector_type(2), aligned(4)));
+    const F2* fl2 = reinterpret_cast<const F2*>(fl);
+    auto up = [&](int X, int Y) {
         const float fxs = (float)X * sx, fys = (float)Y * sy;
         const int i0 = min((int)fxs, w - 1), j0 = min((int)fys, h - 1);
         const int i1 = min(i0 + 1, w - 1), j1 = min(j0 + 1, h - 1);
         const float ax = fxs - (float)i0, ay = fys - (float)j0;
-        const float v00 = fl[((long long)j0 * w + i0) * 2 + c] * 20.0f, v10 = fl[((long long)j0 * w + i1) * 2 + c] * 20.0f;
-        const float v01 = fl[((long long)j1 * w + i0) * 2 + c] * 20.0f, v11 = fl[((long long)j1 * w + i1) * 2 + c] * 20.0f;
+        const F2 v00 = fl2[j0 * w + i0] * 20.0f, v10 = fl2[j0 * w + i1] * 20.0f;
+        const F2 v01 = fl2[j1 * w + i0] * 20.0f, v11 = fl2[j1 * w + i1] * 20.0f;
         return (1.0f - ay) * ((1.0f - ax) * v00 + ax * v10) + ay * ((1.0f - ax) * v01 + ax * v11);
     };
     const float su = swap_scale ? (float)Wd / (float)Wp : (float)Hd / (float)Hp;
     const float sv = swap_scale ? (float)Hd / (float)Hp : (float)Wd / (float)Wp;
     float* o = out + ((long long)y * Wd + x) * out_ch;
-    for (int c = 0; c < 2; ++c) {
-        const float v = (1.0f - ly) * ((1.0f - lx) * up(x0, y0, c) + lx * up(x1, y0, c)) +
-                        ly * ((1.0f - lx) * up(x0, y1, c) + lx * up(x1, y1, c));
-        o[c] = v * (c == 0 ? su : sv);
-    }
+    const F2 v = (1.0f - ly) * ((1.0f - lx) * up(x0, y0) + lx * up(x1, y0)) + ly * ((1.0f - lx) * up(x0, y1) + lx * up(x1, y1));
+    *reinterpret_cast<F2U*>(o) = F2U{v.x * su, v.y * sv};
     if (out_ch == 3) o[2] = 0.0f;
 }
 
