@@ -470,8 +470,10 @@ int frame_fused(vsc_stream* s, const vsc_frame_in* in, const vsc_params& p, uint
     int fin = 0;
     if ((rc = solve_pyramid(s, L, p, fma, rplan, resident, st, &fin))) return rc;
     const View res = pl(s->O[0][fin], W, H);
-    if (out_rgba && (rc = launch_to_rgba(res, out_rgba, st))) return rc;
-    if (out_float && (rc = launch_copy_view(res, View{out_float, W, H, 3, 1, 3}, st))) return rc;
+    if (out_rgba && out_float) rc = launch_outputs(res.d, W, H, out_rgba, out_float, st);
+    else if (out_rgba) rc = launch_to_rgba(res, out_rgba, st);
+    else if (out_float) rc = launch_copy_view(res, View{out_float, W, H, 3, 1, 3}, st);
+    if (rc) return rc;
     s->last_idx = fin;
     return VSC_OK;
 }

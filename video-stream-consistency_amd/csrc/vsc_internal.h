@@ -269,6 +269,8 @@ int launch_resident(const ResidentLevel& l, const ResidentPlan& plan, hipStream_
 // the server): its solver leaves CUs free between launches (blocked form only)
 void stream_set_shared(vsc_stream* s);
 int launch_to_rgba(View in, uint8_t* out, hipStream_t s);
+// a planar frame as RGBA8 and as an HWC float frame
+int launch_outputs(const float* planar, int W, int H, uint8_t* rgba, float* frame, hipStream_t s);
 int launch_rgba_to_view(const uint8_t* in, View out, hipStream_t s);
 int launch_copy_view(View in, View out, hipStream_t s);
 
