@@ -46,6 +46,7 @@ struct ConvArgs {
     void* out2; int out2_cs, out2_c0;   // optional second copy of the result, in the input's element kind (Cout <= 16)
     const void* add; int add_cs, add_c0;
     const float* gate;
+    const float* mask;                   // optional (FP32, the output's layout): the result is 0 where it is not above 0
     int Ho, Wo, Cout;
     int pad, pstep, act;
     int tiles_x, tiles_y;
@@ -269,6 +270,13 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
                 if (a.act == 1) x = x > 0.0f ? x : x * 0.1f;
                 else if (a.act == 2) x = x > 0.0f ? x : 0.0f;
                 v[r] = a.gate ? x * g : x;
+            }
+            if constexpr (EKO == EK_F32) {
+                if (a.mask) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (r < nv && !(a.mask[pix * a.out_cs + a.out_c0 + co + r] > 0.0f)) v[r] = 0.0f;
+                }
             }
             if (a.add) conv_load4<EKO>(a.add, pix * a.add_cs + a.add_c0 + co, v, nv);
             conv_store4<EKO>(a.out, pix * a.out_cs + a.out_c0 + co, v, nv);
@@ -688,6 +696,8 @@ int launch_conv3x3(const ConvDesc& d, hipStream_t s)
     a.out2 = d.out2.p; a.out2_cs = d.out2.cs; a.out2_c0 = d.out2.c0;
     a.add = d.add.p; a.add_cs = d.add.cs; a.add_c0 = d.add.c0;
     a.gate = d.gate;
+    a.mask = d.mask;
+    if (d.mask && (eko != EK_F32 || d.wtp || d.add.p)) return set_error(VSC_E_INVALID, "conv3x3: a mask goes with FP32 outputs, plain weights and no residual");
     a.Ho = Ho; a.Wo = Wo; a.Cout = Cout;
     a.pad = d.pad; a.pstep = d.dil; a.act = d.act;
     if (ek == EK_F32) conv_stride<EK_F32, EK_F32>(a, d.stride, s);

@@ -46,7 +46,7 @@ constexpr int T_W2 = 0, T_W3 = 16 * 9 * 16, T_N = T_W3 + 16 * 9 * 4;
 
 struct vsc_upsampler {
     float* p = nullptr;       // U_NP master params
-    float* g = nullptr;       // gradients
+    float* g = nullptr;       // gradients, then the loss kernel's sums (with the workspace)
     float* m = nullptr;       // Adam moments
     float* v = nullptr;
     uint16_t* w16 = nullptr;  // FP16 inference weights
@@ -55,7 +55,7 @@ struct vsc_upsampler {
     // training workspace (grown on demand)
     size_t ws_px = 0, ws_part = 0;
     float *x = nullptr, *base = nullptr, *a1 = nullptr, *a2 = nullptr, *out = nullptr;
-    float *dout = nullptr, *d2 = nullptr, *d1 = nullptr, *part = nullptr, *loss = nullptr;
+    float *dout = nullptr, *d2 = nullptr, *d1 = nullptr, *part = nullptr;
 };
 
 namespace vsc {
@@ -114,12 +114,6 @@ __global__ void k_charb(const float* __restrict__ out, const float* __restrict__
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-__global__ void k_relu_bw(float* d, const float* a, long long n)
-{
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n && !(a[i] > 0.0f)) d[i] = 0.0f;
 }
 
 // weight and bias gradients of a 3x3 conv (stride 1, pad 1) over a 16 x 16
@@ -700,9 +694,10 @@ void master_to_ref(const std::vector<float>& m, float* r)
 }
 
 int conv(const void* in, int cin, const void* wt, const float* bias, void* out, int out_cs, int cout, int act,
-         const void* add, int add_cs, const float* gate, int ek, int eko, int N, int H, int W, hipStream_t s)
+         const void* add, int add_cs, const float* gate, int ek, int eko, int N, int H, int W, hipStream_t s, const float* mask = nullptr)
 {
     ConvDesc d{};
+    d.mask = mask;
     d.in = Nhwc{const_cast<void*>(in), N, H, W, cin, cin, 0};
     d.out = Nhwc{out, N, H, W, cout, out_cs, 0};
     d.add = Nhwc{const_cast<void*>(add), N, H, W, cout, add_cs, 0};
@@ -715,10 +710,10 @@ int conv(const void* in, int cin, const void* wt, const float* bias, void* out, 
 int grow(vsc_upsampler* u, size_t px, size_t part)
 {
     if (px <= u->ws_px && part <= u->ws_part) return VSC_OK;
-    float** bufs[] = {&u->x, &u->base, &u->a1, &u->a2, &u->out, &u->dout, &u->d2, &u->d1, &u->part, &u->loss};
+    float** bufs[] = {&u->x, &u->base, &u->a1, &u->a2, &u->out, &u->dout, &u->d2, &u->d1, &u->part, &u->g};
     if (hipDeviceSynchronize() != hipSuccess) return set_error(VSC_E_HIP, "upsampler: sync");
     for (float** b : bufs) { (void)hipFree(*b); *b = nullptr; }
-    const size_t sz[] = {px * 4, px * 2, px * 16, px * 16, px * 2, px * 4, px * 16, px * 16, part, px / 256 + 2};
+    const size_t sz[] = {px * 4, px * 2, px * 16, px * 16, px * 2, px * 4, px * 16, px * 16, part, U_NP + px / 256 + 2};
     for (int i = 0; i < 10; ++i)
         if (hipMalloc(reinterpret_cast<void**>(bufs[i]), sz[i] * 4) != hipSuccess) {
             u->ws_px = u->ws_part = 0;
@@ -729,9 +724,10 @@ int grow(vsc_upsampler* u, size_t px, size_t part)
     return VSC_OK;
 }
 
-// forward (FP32) and backward into u->g; optional loss (host, synchronises)
+// forward (FP32) and backward into u->g; optional loss and gradients (host; one
+// copy for both, synchronises)
 int fwd_bwd(vsc_upsampler* u, int B, const float* lo, int lw, int lh, const uint8_t* rgba, const float* gt, int W,
-            int H, float scale, float* loss_host, hipStream_t s)
+            int H, float scale, float* loss_host, std::vector<float>* grads, hipStream_t s)
 {
     const size_t px = (size_t)B * W * H;
     const int tx = (W + 15) / 16, ty = (H + 15) / 16;
@@ -747,7 +743,7 @@ int fwd_bwd(vsc_upsampler* u, int B, const float* lo, int lw, int lh, const uint
     if ((rc = conv(u->a2, 16, u->p + U_W3, u->p + U_B3, u->out, 2, 2, 0, u->base, 2, nullptr, EK_F32, EK_F32, B, H, W, s))) return rc;
     // loss and dOut
     const unsigned lb = (unsigned)((px + 255) / 256);
-    hipLaunchKernelGGL(k_charb, dim3(lb), dim3(256), 0, s, u->out, gt, u->dout, u->loss, (long long)px, 1e-3f,
+    hipLaunchKernelGGL(k_charb, dim3(lb), dim3(256), 0, s, u->out, gt, u->dout, u->g + U_NP, (long long)px, 1e-3f,
                        1.0f / (float)px);
     if ((rc = check_launch("upsampler loss"))) return rc;
     const int nb = B * tx * ty;
@@ -756,28 +752,28 @@ int fwd_bwd(vsc_upsampler* u, int B, const float* lo, int lw, int lh, const uint
     hipLaunchKernelGGL((k_conv_bw_w<16, 2, 4>), gw, dim3(256), 0, s, u->a2, u->dout, H, W, tx, ty, u->part);
     hipLaunchKernelGGL(k_reduce_rows, dim3((2 * 9 * 16 + 2 + 31) / 32), dim3(1024), 0, s, u->part, nb, 2 * 9 * 16 + 2,
                        u->g + U_W3);
-    if ((rc = conv(u->dout, 4, u->wT + T_W3, nullptr, u->d2, 16, 16, 0, nullptr, 0, nullptr, EK_F32, EK_F32, B, H, W, s))) return rc;
-    hipLaunchKernelGGL(k_relu_bw, dim3((unsigned)((px * 16 + 255) / 256)), dim3(256), 0, s, u->d2, u->a2, (long long)px * 16);
+    if ((rc = conv(u->dout, 4, u->wT + T_W3, nullptr, u->d2, 16, 16, 0, nullptr, 0, nullptr, EK_F32, EK_F32, B, H, W, s, u->a2))) return rc;
     // layer 2
     hipLaunchKernelGGL((k_conv_bw_w<16, 16, 16>), gw, dim3(256), 0, s, u->a1, u->d2, H, W, tx, ty, u->part);
     hipLaunchKernelGGL(k_reduce_rows, dim3((16 * 9 * 16 + 16 + 31) / 32), dim3(1024), 0, s, u->part, nb,
                        16 * 9 * 16 + 16, u->g + U_W2);
-    if ((rc = conv(u->d2, 16, u->wT + T_W2, nullptr, u->d1, 16, 16, 0, nullptr, 0, nullptr, EK_F32, EK_F32, B, H, W, s))) return rc;
-    hipLaunchKernelGGL(k_relu_bw, dim3((unsigned)((px * 16 + 255) / 256)), dim3(256), 0, s, u->d1, u->a1, (long long)px * 16);
+    if ((rc = conv(u->d2, 16, u->wT + T_W2, nullptr, u->d1, 16, 16, 0, nullptr, 0, nullptr, EK_F32, EK_F32, B, H, W, s, u->a1))) return rc;
     // layer 1
     hipLaunchKernelGGL((k_conv_bw_w<U_C1, 16, 16>), gw, dim3(256), 0, s, u->x, u->d1, H, W, tx, ty, u->part);
     hipLaunchKernelGGL(k_reduce_rows, dim3((16 * 9 * U_C1 + 16 + 31) / 32), dim3(1024), 0, s, u->part, nb,
                        16 * 9 * U_C1 + 16, u->g + U_W1);
     if ((rc = check_launch("upsampler backward"))) return rc;
+    if (!loss_host && !grads) return VSC_OK;
+    std::vector<float> back(U_NP + lb);
+    if (check_hip(hipMemcpyAsync(back.data(), u->g, back.size() * 4, hipMemcpyDeviceToHost, s), "upsampler loss") ||
+        check_hip(hipStreamSynchronize(s), "upsampler loss"))
+        return VSC_E_HIP;
     if (loss_host) {
-        std::vector<float> parts(lb);
-        if (check_hip(hipMemcpyAsync(parts.data(), u->loss, lb * 4, hipMemcpyDeviceToHost, s), "upsampler loss") ||
-            check_hip(hipStreamSynchronize(s), "upsampler loss"))
-            return VSC_E_HIP;
         double t = 0.0;
-        for (float x : parts) t += x;
+        for (unsigned i = 0; i < lb; ++i) t += back[U_NP + i];
         *loss_host = (float)(t / (double)px);
     }
+    if (grads) grads->assign(back.begin(), back.begin() + U_NP);
     return VSC_OK;
 }
 
@@ -803,9 +799,9 @@ extern "C" int vsc_upsampler_create(unsigned long long seed, vsc_upsampler** out
     *out = nullptr;
     vsc_upsampler* u = new (std::nothrow) vsc_upsampler();
     if (!u) return set_error(VSC_E_NOMEM, "vsc_upsampler_create: host memory");
-    void** bufs[] = {(void**)&u->p, (void**)&u->g, (void**)&u->m, (void**)&u->v, (void**)&u->w16, (void**)&u->wT};
-    const size_t sz[] = {U_NP * 4, U_NP * 4, U_NP * 4, U_NP * 4, H_N * 2, T_N * 4};
-    for (int i = 0; i < 6; ++i)
+    void** bufs[] = {(void**)&u->p, (void**)&u->m, (void**)&u->v, (void**)&u->w16, (void**)&u->wT};
+    const size_t sz[] = {U_NP * 4, U_NP * 4, U_NP * 4, H_N * 2, T_N * 4};
+    for (int i = 0; i < 5; ++i)
         if (hipMalloc(bufs[i], sz[i]) != hipSuccess || hipMemset(*bufs[i], 0, sz[i]) != hipSuccess) {
             vsc_upsampler_destroy(u);
             return set_error(VSC_E_NOMEM, "vsc_upsampler_create: device allocation failed");
@@ -832,7 +828,7 @@ extern "C" int vsc_upsampler_create(unsigned long long seed, vsc_upsampler** out
 extern "C" int vsc_upsampler_destroy(vsc_upsampler* u)
 {
     if (!u) return VSC_OK;
-    void* bufs[] = {u->p, u->g, u->m, u->v, u->w16, u->wT, u->x, u->base, u->a1, u->a2, u->out, u->dout, u->d2, u->d1, u->part, u->loss};
+    void* bufs[] = {u->p, u->g, u->m, u->v, u->w16, u->wT, u->x, u->base, u->a1, u->a2, u->out, u->dout, u->d2, u->d1, u->part};
     for (void* b : bufs) (void)hipFree(b);
     delete u;
     return VSC_OK;
@@ -920,12 +916,9 @@ extern "C" int vsc_upsampler_loss_grad(vsc_upsampler* u, int batch, const float*
     int rc = check_train_args(u, batch, flow_lo, lo_w, lo_h, rgba, flow_gt, width, height);
     if (rc) return rc;
     hipStream_t s = as_stream(stream);
-    if ((rc = fwd_bwd(u, batch, flow_lo, lo_w, lo_h, rgba, flow_gt, width, height, scale, loss, s))) return rc;
+    std::vector<float> g;
+    if ((rc = fwd_bwd(u, batch, flow_lo, lo_w, lo_h, rgba, flow_gt, width, height, scale, loss, grad_host ? &g : nullptr, s))) return rc;
     if (grad_host) {
-        std::vector<float> g(U_NP);
-        if (check_hip(hipMemcpyAsync(g.data(), u->g, U_NP * 4, hipMemcpyDeviceToHost, s), "vsc_upsampler_loss_grad") ||
-            check_hip(hipStreamSynchronize(s), "vsc_upsampler_loss_grad"))
-            return VSC_E_HIP;
         master_to_ref(g, grad_host);
     }
     return VSC_OK;
@@ -939,7 +932,7 @@ extern "C" int vsc_upsampler_train_step(vsc_upsampler* u, int batch, const float
     if (rc) return rc;
     if (!(lr > 0.0f)) return set_error(VSC_E_INVALID, "vsc_upsampler_train_step: lr must be positive");
     hipStream_t s = as_stream(stream);
-    if ((rc = fwd_bwd(u, batch, flow_lo, lo_w, lo_h, rgba, flow_gt, width, height, scale, loss, s))) return rc;
+    if ((rc = fwd_bwd(u, batch, flow_lo, lo_w, lo_h, rgba, flow_gt, width, height, scale, loss, nullptr, s))) return rc;
     u->step += 1;
     const float b1 = 0.9f, b2 = 0.999f;
     const float bc1 = 1.0f - (float)std::pow(0.9, u->step), bc2 = 1.0f - (float)std::pow(0.999, u->step);

@@ -402,6 +402,7 @@ struct ConvDesc {
     const void* wtp;     // nullptr, or the weights packed (conv_pack_weights) in place of wt
     const float* bias;   // [Cout] or nullptr
     const float* gate;   // nullptr, or a device scalar multiplying the activated result before `add`
+    const float* mask;   // nullptr, or FP32 values in out's layout: the result is 0 where they are not above 0
     int stride, dil, pad, act;
     int ek_in, ek_out;
 };
