@@ -26,7 +26,7 @@ namespace vsc {
 // The loads are 16 bytes wide whatever the alignment; a slot over the right edge
 // is read further left and shifted.  (One pixel a load with its own index
 // arithmetic took 4 us a chunk: 17x30x196 28.4 us, now 12.9; 480x272x32 34.9 us,
-// now 24.1, its multiplications and additions alone about 20.)  This staging
+// now 24.1, its multiplications and additions alone 17.)  This staging
 // replaces the reference's channels-last rearrange kernels and their per-call
 // cudaMalloc (correlation_cuda.cu:32-95,365-370).  Output rows are written 4*QX
 // bytes a lane, again whatever the alignment (479x271x32: 115 us with 4-byte
