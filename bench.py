@@ -774,10 +774,10 @@ def stabilize_run(args, vsc, dev, O, P, F, B, mode, steps, with_profile=False):
         if n_solver:
             ach = by_solver / (ms_solver * 1e-3) / 1e9
             r["solver"] = {
-                "kernel": "k_consist_blocked (temporally blocked consistency solver)",
+                "kernel": "k_consist_resident (consistency solver, a level resident on the chip)",
                 "bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4),
-                "traffic": traffic_from_profile("k_consist_blocked", "stabilize"),
+                "traffic": traffic_from_profile("k_consist_resident", "stabilize"),
                 "launches": n_solver, "avg_launch_us": round(1000.0 * ms_solver / n_solver, 3),
                 "ms_per_frame": round(ms_solver / nprof, 4),
                 "algorithmic_bytes_per_launch": round(by_solver / n_solver),
