@@ -27,7 +27,9 @@ def _give_up(vsc, st):
 
 @pytest.mark.parametrize("mode", [0, 2])
 @pytest.mark.parametrize("W,H,levels,iters", [(128, 48, 1, 20), (129, 49, 1, 19), (131, 65, 2, 33), (256, 64, 1, 8),
-                                              (258, 98, 2, 75), (515, 201, 3, 100), (640, 360, 2, 150), (1282, 718, 2, 41)])
+                                              (258, 98, 2, 75), (515, 201, 3, 100), (640, 360, 2, 150), (1282, 718, 2, 41),
+                                              # one pixel a lane: levels one tile large, a pixel larger, flush on both sides
+                                              (64, 64, 1, 21), (65, 67, 1, 40), (130, 66, 2, 150), (199, 113, 2, 33), (321, 181, 1, 26)])
 def test_routes_agree(cuda, mode, W, H, levels, iters):
     """Tile edges and remainders (levels one tile large, one pixel larger, odd
     ones), whole and part phases, one to three levels, both solver forms."""

@@ -35,8 +35,8 @@ def _axis(L, T, h, starts):
 @pytest.mark.parametrize("fma", [0, 1])
 @pytest.mark.parametrize("cus", [256, 64, 32])
 def test_tilings_cover_and_exchange(vsc, fma, cus):
-    sizes = [(W, H) for W in (127, 128, 129, 131, 255, 256, 257, 300, 480, 640, 853, 960, 1281, 1571, 1920)
-             for H in (47, 48, 49, 63, 64, 101, 129, 180, 270, 361, 540, 719, 784, 1080)]
+    sizes = [(W, H) for W in (64, 65, 99, 127, 128, 129, 131, 255, 256, 257, 300, 480, 640, 853, 960, 1281, 1571, 1920)
+             for H in (32, 33, 45, 47, 48, 49, 63, 64, 101, 129, 180, 270, 361, 540, 719, 784, 1080)]
     found = 0
     for W, H in sizes:
         for iters in (1, 2, 7, 20, 75, 149, 150, 304):
@@ -53,5 +53,5 @@ def test_tilings_cover_and_exchange(vsc, fma, cus):
             _axis(H, th, h, ys)
     assert found > 100
     # a level narrower or lower than every tile, or one that does not fit the chip, has none
-    assert _plan(vsc, 127, 500, 150, cus, fma) is None and _plan(vsc, 500, 47, 150, cus, fma) is None
+    assert _plan(vsc, 63, 500, 150, cus, fma) is None and _plan(vsc, 500, 31, 150, cus, fma) is None
     assert _plan(vsc, 3840, 2160, 150, cus, fma) is None and _plan(vsc, 640, 360, 0, cus, fma) is None

@@ -103,6 +103,10 @@ template <> struct Quad<2> {
     typedef float T __attribute__((ext_vector_type(2), aligned(4)));
     typedef uint32_t B __attribute__((ext_vector_type(2)));
 };
+template <> struct Quad<1> {
+    typedef float T __attribute__((ext_vector_type(1), aligned(4)));
+    typedef uint32_t B;
+};
 
 // A lane's pixels to and from an exchange plane, coherent across the device
 // (sc1: past the XCD's own L2).  NOWHERE lies past every
@@ -113,14 +117,16 @@ __device__ __forceinline__ void store_px(const typename Quad<PX>::T& v, const __
 {
     using B = typename Quad<PX>::B;
     if constexpr (PX == 4) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(B, v), x, at, row, AUX);
-    else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B, v), x, at, row, AUX);
+    else if constexpr (PX == 2) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B, v), x, at, row, AUX);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(B, v), x, at, row, AUX);
 }
 template <int PX, int AUX = AUX_AGENT>
 __device__ __forceinline__ typename Quad<PX>::T load_px(const __amdgpu_buffer_rsrc_t& x, int at, int row)
 {
     using V = typename Quad<PX>::T;
     if constexpr (PX == 4) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(x, at, row, AUX));
-    else return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(x, at, row, AUX));
+    else if constexpr (PX == 2) return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(x, at, row, AUX));
+    else return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(x, at, row, AUX));
 }
 
 // buffer descriptor of a plane of `n` floats
@@ -225,8 +231,8 @@ __global__ __launch_bounds__(64 * NW, (8 / NW) * NW / 4) void k_consist_resident
         const int w_up = top ? DUMP : 2 * wv - 1, w_dn = low ? DUMP : 2 * wv;
         auto row_update = [&](int r, const V& vk, V& prev, const V& up, const V& dn) {
             const V cur = o[r];
-            const float lf = from_left(cur[PX - 1]), rt = from_right(cur[0]);
             const float rm = right63 ? 0.0f : cur[PX - 1];
+            const float lf = from_left(cur[PX - 1]), rt = from_right(PX == 1 ? rm : cur[0]);
 #pragma unroll
             for (int p = 0; p < PX; ++p) {
                 const float rv = p == PX - 1 ? rt : p == PX - 2 ? rm : cur[p + 1 < PX ? p + 1 : 0];
@@ -469,7 +475,10 @@ void go_resident(const ResArgs& a, hipStream_t s)
 }
 
 // tile shapes: 64*px x RES_NW*r pixels.  The FMA form holds three registers a
-// pixel (o, u, q), the reference order four, so its tiles end at r = 12.
+// pixel (o, u, q), the reference order four, so its tiles end at r = 12.  One
+// pixel a lane is for small levels, whose sweeps are bound by their latency: more
+// and smaller tiles (frames of 640x360 in reference order 250 us with two and
+// more, 232 with one; 320x180 246 and 184; 200x113, FMA form, 251 and 192).
 struct Variant {
     int px, r, fma;
     void (*go)(const ResArgs&, hipStream_t);
@@ -482,6 +491,10 @@ const Variant kVariants[] = {
     {2, 8, 0, go_resident<2, 8, false>},   {2, 10, 0, go_resident<2, 10, false>}, {2, 12, 0, go_resident<2, 12, false>},
     {2, 16, 0, go_resident<2, 16, false>}, {4, 6, 0, go_resident<4, 6, false>},  {4, 8, 0, go_resident<4, 8, false>},
     {4, 10, 0, go_resident<4, 10, false>}, {4, 12, 0, go_resident<4, 12, false>},
+    {1, 4, 1, go_resident<1, 4, true>},    {1, 4, 0, go_resident<1, 4, false>},
+    {1, 6, 1, go_resident<1, 6, true>},    {1, 8, 1, go_resident<1, 8, true>},   {1, 10, 1, go_resident<1, 10, true>},
+    {1, 12, 1, go_resident<1, 12, true>},  {1, 6, 0, go_resident<1, 6, false>},  {1, 8, 0, go_resident<1, 8, false>},
+    {1, 10, 0, go_resident<1, 10, false>}, {1, 12, 0, go_resident<1, 12, false>},
 };
 
 // the end of the last resident launch of each device
