@@ -505,13 +505,20 @@ struct Turn {
 };
 Turn turns[RES_MAX_DEVICES];
 
-// tiles along an axis, 0 if the axis does not take tiles of T pixels
+// tiles along an axis, 0 if the axis does not take tiles of T pixels.  A tile
+// waits for the tiles beside it and for no other, so no other's pixels may hold a
+// part of its exact ones: it would publish or store them with nothing that orders
+// this after that tile's loads of them.  Where the tiles overlap by much (three on
+// an axis a little longer than two), h is refused.
 int res_count(int L, int T, int h, int q)
 {
     if (L < T || T < 4 * h + 4 * q) return 0;
     if (L == T) return 1;
     const int O = T - 2 * h;                    // the most two neighbours may be apart (a multiple of q)
-    return 1 + (L - T + O - 1) / O;
+    const int n = 1 + (L - T + O - 1) / O;
+    for (int i = 0; i + 2 < n; ++i)
+        if (res_start(i + 2, n, L, T, q) < res_start(i, n, L, T, q) + T - h) return 0;
+    return n;
 }
 
 }  // namespace
