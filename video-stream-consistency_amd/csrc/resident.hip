@@ -16,8 +16,9 @@
 //
 // Strips.  A level too large for the chip is swept in rounds of up to some tens
 // of sweeps; in a round, strips of rows are resident one after the other, each
-// with as many rows beyond its own as the round has sweeps (those rows' values
-// go wrong from the cut inwards, a row a sweep, and are not kept).  O and U go
+// with as many rows above its own as the round has sweeps, and one more below
+// (their values go wrong from the cut inwards, a row a sweep, below two with the
+// first: the row above the last has no lower neighbour; they are not kept).  O and U go
 // through memory once a round.  A 3840x2160 frame of 150 and 75 sweeps: 2553 us
 // against 3787 with the blocked solver on level 0, a 2560x1440 one 1211 against
 // 1595, one of 2000x1125 898 against 985.
@@ -581,7 +582,7 @@ bool plan_resident_strips(int W, int H, int iters, int cus, int fma, ResidentPla
         const int sweeps = (iters + rounds - 1) / rounds;
         if ((iters + sweeps - 1) / sweeps != rounds) continue;
         for (int strips = 2; strips <= 12; ++strips) {
-            const int own = (H + strips - 1) / strips, rows = std::min(H, own + 2 * sweeps);
+            const int own = (H + strips - 1) / strips, rows = std::min(H, own + 2 * sweeps + 1);
             if ((fma ? (rounds == 1 ? 1 : 2) : 4) * rows > H || (long long)W * rows >= (1LL << 28)) continue;
             for (int v = 0; v < (int)(sizeof(kVariants) / sizeof(kVariants[0])); ++v) {
                 const Variant& k = kVariants[v];
