@@ -459,22 +459,43 @@ __global__ __launch_bounds__(256) void k_conv3x3w(ConvArgs a)
     }
 }
 
-// Parts whose sums a packed layer of one batch item's `item_blocks` blocks (of
-// the tiles that k_conv3x3 would take) keeps apart: what a split over the idle
-// CUs would give, bounded by kConvPartFloats of partial sums an item.  It
-// depends on one item's geometry only, so an item's result has the same bits
-// alone and in a batch of any size.
-constexpr long long kConvPartFloats = 2LL << 20;
+// The channel tile of k_conv3x3, and the rows of a wave of its pixel tile for
+// `items` batch items (conv_pick says why).
 template <int EK>
-static int conv_parts(const ConvArgs& a, long long item_blocks, int chunks)
+static int conv_nt(const ConvArgs& a)
 {
-    if (chunks < 2 || item_blocks >= (EK == EK_F32 ? 128 : 32)) return 1;
+    if (EK == EK_F32 && a.Cout > 32) return 64;
+    return a.Cout > 16 ? 32 : 16;
+}
+template <int EK, int S>
+static int conv_rows(const ConvArgs& a, int items)
+{
+    const int ps = a.pstep, nt = conv_nt<EK>(a);
+    const long long px = (long long)((a.Ho + ps - 1) / ps) * ps * ((a.Wo + ps - 1) / ps) * ps * items;
+    const long long ntiles = (a.Cout + nt - 1) / nt;
+    auto blocks = [&](int mr) { return (px / (64LL * mr)) * ntiles; };
+    const int mr = (S == 1 && blocks(4) >= 512) ? 4 : (blocks(2) >= (EK == EK_F32 ? 512 : 128) ? 2 : 1);
+    return S == 2 && mr > 2 ? 2 : mr;
+}
+
+// Chunks whose sums a packed layer keeps apart (ConvArgs::flush): what a split of
+// the channel loop over the CUs that one batch item's blocks of k_conv3x3 leave idle
+// would give, bounded by kConvPartFloats of partial sums an item.  One item's
+// geometry alone decides, the pixel tile's rows included, so an item's result has
+// the same bits alone and in a batch of any size.
+constexpr long long kConvPartFloats = 2LL << 20;
+template <int EK, int S>
+static int conv_flush(const ConvArgs& a)
+{
+    const int chunks = (a.Cin + ConvK<EK>::KC - 1) / ConvK<EK>::KC, ps = a.pstep, mr = conv_rows<EK, S>(a, 1), nt = conv_nt<EK>(a);
+    const long long hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
+    const long long item_blocks = (hs + 4 * mr - 1) / (4 * mr) * ((ws + 15) / 16) * ps * ps * ((a.Cout + nt - 1) / nt);
+    if (chunks < 2 || item_blocks >= (EK == EK_F32 ? 128 : 32)) return 0;
     const long long item_stride = (long long)a.Ho * a.Wo * a.Cout;
     int parts = (int)std::min<long long>(chunks, (256 + item_blocks - 1) / item_blocks);
     parts = (int)std::min<long long>(parts, kConvPartFloats / std::max<long long>(item_stride, 1));
-    if (parts < 2) return 1;
-    const int cpp = (chunks + parts - 1) / parts;
-    return (chunks + cpp - 1) / cpp;
+    if (parts < 2) return 0;
+    return (chunks + parts - 1) / parts;
 }
 
 template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
@@ -567,21 +588,11 @@ static void conv_mr(const ConvArgs& a, int mr, hipStream_t s)
 template <int EK, int EKO, int S>
 static void conv_pick(const ConvArgs& a, hipStream_t s)
 {
-    const int ps = a.pstep;
-    const long long px = (long long)((a.Ho + ps - 1) / ps) * ps * ((a.Wo + ps - 1) / ps) * ps * a.N;
-    const int NTsel = EK == EK_F32 ? (a.Cout > 32 ? 64 : (a.Cout > 16 ? 32 : 16)) : (a.Cout > 16 ? 32 : 16);
-    const long long ntiles = (a.Cout + NTsel - 1) / NTsel;
-    auto blocks = [&](int mr) { return (px / (64LL * mr)) * ntiles; };
-    int mr = (S == 1 && blocks(4) >= 512) ? 4 : (blocks(2) >= (EK == EK_F32 ? 512 : 128) ? 2 : 1);
-    if (S == 2 && mr > 2) mr = 2;
+    const int ps = a.pstep, NTsel = conv_nt<EK>(a), mr = conv_rows<EK, S>(a, a.N);
     if constexpr (EK != EK_F16) {
         if (a.wtp) {
             ConvArgs b = a;
-            const int chunks = (a.Cin + ConvK<EK>::KC - 1) / ConvK<EK>::KC;
-            const long long hs = (a.Ho + ps - 1) / ps, ws = (a.Wo + ps - 1) / ps;
-            const long long tiles = (hs + 4 * mr - 1) / (4 * mr) * ((ws + 15) / 16) * ps * ps;
-            const int parts = conv_parts<EK>(a, tiles * ntiles, chunks);
-            b.flush = parts > 1 ? (chunks + parts - 1) / parts : 0;
+            b.flush = conv_flush<EK, S>(a);
             conv_packed<EK, EKO, S>(b, s);
             return;
         }
@@ -757,4 +768,17 @@ extern "C" int vsct_conv3x3_packed(const void* in, int N, int H, int W, int Cin,
     (void)hipDeviceSynchronize();
     (void)hipFree(dev);
     return rc;
+}
+
+// Diagnostic (no declaration in vsc.h): the chunks whose sums a packed layer keeps
+// apart, 0 when it has one sum.
+extern "C" int vsct_conv_flush(int N, int H, int W, int Cin, int Cout, int stride, int dilation, int dtype)
+{
+    using namespace vsc;
+    ConvArgs a{};
+    a.N = N; a.H = H; a.W = W; a.Cin = Cin;
+    a.Ho = (H - 1) / stride + 1; a.Wo = (W - 1) / stride + 1; a.Cout = Cout;
+    a.pstep = dilation;
+    if (dtype == VSC_F32) return stride == 2 ? conv_flush<EK_F32, 2>(a) : conv_flush<EK_F32, 1>(a);
+    return stride == 2 ? conv_flush<EK_BF16, 2>(a) : conv_flush<EK_BF16, 1>(a);
 }
