@@ -308,6 +308,31 @@ int prepare_flows(vsc_stream* s, const vsc_frame_in* in, View* fwd, View* bwd, h
     return rc;
 }
 
+// Whether a stream is not captured and has every CU.  A query that fails says no
+// and leaves no error behind for the next launch's check (the legacy stream cannot
+// be asked while a blocking stream is captured).  The handles that stand for a
+// default stream without naming one are not asked: not every runtime resolves them
+// in a query.
+bool whole_device(hipStream_t st, int cus)
+{
+    if (st == hipStreamLegacy || st == hipStreamPerThread) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (cap != hipStreamCaptureStatusNone) return false;
+    if (!st) return true;
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    int n = 0;
+    for (uint32_t m : mask) n += __builtin_popcount(m);
+    return n == 0 || n >= cus;
+}
+
 // Whether this frame's levels may use the resident solver: not beside other
 // work on purpose, not under capture (its launches take turns across streams),
 // not on a stream that leaves CUs out, and not for some frames after the device
@@ -324,15 +349,7 @@ bool resident_frame(vsc_stream* s, const vsc_params& p, hipStream_t st)
         --s->skip;
         return false;
     }
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
-    uint32_t mask[32] = {};
-    if (st && hipExtStreamGetCUMask(st, 32, mask) == hipSuccess) {
-        int n = 0;
-        for (uint32_t m : mask) n += __builtin_popcount(m);
-        if (n > 0 && n < s->cus) return false;
-    }
-    return true;
+    return whole_device(st, s->cus);
 }
 
 // The buffer of O[j] in which level j starts.  The blocked solver starts in 0
