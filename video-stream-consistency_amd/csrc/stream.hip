@@ -36,6 +36,14 @@ struct vsc_stream {
     volatile unsigned* note = nullptr;
     int cus = 0, skip = 0, backoff = 0;
     bool shared = false;
+    int resident_levels = 0;   // of the last frame
+    // the HIP stream of its frames, and the end of the last one that was marked
+    // (beside_others)
+    hipStream_t on = nullptr;
+    hipEvent_t done = nullptr;
+    bool ran = false, under_way = false;
+    int dev = -1, hold = 0;
+    vsc_stream *next = nullptr, *prev = nullptr;   // of the device's
     // the levels' resident plans of the last frame's form and sweeps
     struct {
         int iters = -1, fma = -1;
@@ -111,6 +119,94 @@ struct Notes {
 };
 Notes notes;
 
+// The stabilizers of a device.
+constexpr int MAX_DEVICES = 64;
+struct Device {
+    std::mutex m;
+    vsc_stream* first = nullptr;
+};
+Device devices[MAX_DEVICES];
+
+void enlist(vsc_stream* s, int dev)
+{
+    if (dev < 0 || dev >= MAX_DEVICES) return;
+    Device& d = devices[dev];
+    std::lock_guard<std::mutex> hold(d.m);
+    s->dev = dev;
+    s->next = d.first;
+    if (d.first) d.first->prev = s;
+    d.first = s;
+}
+
+void delist(vsc_stream* s)
+{
+    if (s->dev < 0) return;
+    Device& d = devices[s->dev];
+    std::lock_guard<std::mutex> hold(d.m);
+    (s->prev ? s->prev->next : d.first) = s->next;
+    if (s->next) s->next->prev = s->prev;
+    if (s->done) (void)hipEventDestroy(s->done);
+}
+
+// Whether a frame of another stabilizer is under way on another HIP stream.  The
+// answer yes holds for 64 frames more: stabilizers that run side by side do not
+// ask for each frame, nor take a resident one whenever the other is between two.
+bool beside_others(vsc_stream* s, hipStream_t st)
+{
+    if (s->dev < 0) return false;
+    Device& d = devices[s->dev];
+    std::lock_guard<std::mutex> lock(d.m);
+    if (s->hold > 0) {
+        --s->hold;
+        return true;
+    }
+    for (vsc_stream* o = d.first; o; o = o->next) {
+        if (o == s || !o->under_way || o->on == st) continue;
+        const hipError_t e = hipEventQuery(o->done);
+        if (e != hipSuccess) (void)hipGetLastError();
+        if (e == hipErrorNotReady) {
+            s->hold = 64;
+            return true;
+        }
+        o->under_way = false;
+    }
+    return false;
+}
+
+// Marks a frame's end for the others' beside_others: only where another
+// stabilizer, whose frames could be resident, runs on another HIP stream.
+void frame_enqueued(vsc_stream* s, hipStream_t st)
+{
+    if (s->dev < 0) return;
+    Device& d = devices[s->dev];
+    std::lock_guard<std::mutex> lock(d.m);
+    s->on = st;
+    s->ran = true;
+    const vsc_stream* o = d.first;
+    while (o && (o == s || !o->ran || o->shared || o->on == st)) o = o->next;
+    if (!o || st == hipStreamLegacy || st == hipStreamPerThread) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        (s->done || hipEventCreateWithFlags(&s->done, hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess) &&
+        hipEventRecord(s->done, st) == hipSuccess)
+        s->under_way = true;
+    else
+        (void)hipGetLastError();
+}
+
+// Whether a frame keeps the resident solver beside other stabilizers' frames.
+// Resident launches take turns and leave a small frame's idle CUs idle; the
+// blocked solver's fill the chip from several HIP streams.  Frames a second of
+// three stabilizers, resident in turn | blocked side by side: FMA form 320x180
+// 5720 | 10613, 640x360 4841 | 6502, 960x540 3938 | 4745, 1120x630 3385 | 3227,
+// 1920x1080 2013 | 1181; reference order 320x180 5144 | 8093, 560x316 4665 |
+// 5484, 640x360 4232 | 3334, 1280x720 2330 | 1904, and 1920x1080, whose level 0 is
+// blocked in both, 960 | 985.
+bool worth_beside(const vsc_stream* s, const bool* resident, int fma)
+{
+    return resident[0] && (long long)s->W * s->H >= (fma ? 600000 : 200000);
+}
+
 }  // namespace
 
 extern "C" size_t vsc_stream_footprint(int width, int height, int flow_width, int flow_height)
@@ -168,7 +264,7 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
         return set_error(VSC_E_INVALID, "vsc_stream_create: internal error: carve does not match the footprint");
     }
     // without these the blocked solver runs alone
-    int dev = 0;
+    int dev = -1;
     static const std::vector<unsigned> zeros(RESIDENT_CTL_BYTES / 4, 0u);
     unsigned* ctl = reinterpret_cast<unsigned*>(static_cast<char*>(s->block) + s->bytes);
     if (hipGetDevice(&dev) == hipSuccess &&
@@ -179,6 +275,7 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
     } else {
         (void)hipGetLastError();
     }
+    enlist(s, dev);
     *out = s;
     return VSC_OK;
 }
@@ -193,6 +290,7 @@ extern "C" int vsc_stream_destroy(vsc_stream* s)
         if (!rc) rc = rc2;
     }
     if (s->note) notes.give(s->note);   // hipFree has waited for the device
+    delist(s);
     delete s;
     return rc;
 }
@@ -479,6 +577,9 @@ int frame_fused(vsc_stream* s, const vsc_frame_in* in, const vsc_params& p, uint
             resident[j] = k.ok;
             rplan[j] = k.plan;
         }
+    const int nres = (int)std::count(resident, resident + L, true);
+    s->resident_levels = nres > 0 && !worth_beside(s, resident, fma) && beside_others(s, st) ? 0 : nres;
+    if (s->resident_levels == 0) std::fill(resident, resident + L, false);
     if (L == 1) {
         // single level: the solution starts at the processed frame (videostabilizer.cpp:209)
         const int start = level_start(s, 0, p.num_iter, fma, resident[0] ? rplan[0].rounds : 0);
@@ -492,6 +593,7 @@ int frame_fused(vsc_stream* s, const vsc_frame_in* in, const vsc_params& p, uint
     else if (out_float) rc = launch_copy_view(res, View{out_float, W, H, 3, 1, 3}, st);
     if (rc) return rc;
     s->last_idx = fin;
+    frame_enqueued(s, st);
     return VSC_OK;
 }
 
@@ -684,6 +786,10 @@ extern "C" int vsct_resident_give_up(vsc_stream* s, vsc_hip_stream stream)
     if (check_hip(hipMemcpyAsync(s->ctl, &one, 4, hipMemcpyHostToDevice, as_stream(stream)), "vsct_resident_give_up")) return 0;
     return check_hip(hipStreamSynchronize(as_stream(stream)), "vsct_resident_give_up") ? 0 : 1;
 }
+
+// Diagnostic (no declaration in vsc.h): the levels of the stream's last fused
+// frame that the resident solver took.
+extern "C" int vsct_resident_levels(const vsc_stream* s) { return s ? s->resident_levels : 0; }
 
 extern "C" int vsc_stab_frame(vsc_stream* s, const vsc_frame_in* in, const vsc_params* params, uint8_t* out_rgba,
                               float* out_float, int mode, vsc_hip_stream stream)
