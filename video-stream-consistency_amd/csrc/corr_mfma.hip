@@ -80,9 +80,10 @@ __device__ inline uint2 nchw_px8(const uint32_t (&raw)[8], int j)
     return make_uint2(__builtin_amdgcn_perm(t23, t01, 0x05040100u), __builtin_amdgcn_perm(t67, t45, 0x05040100u));
 }
 
-template <int KIND, int MD, bool LEGACY, int DG>
+template <int KIND, int MD, bool LEGACY, int DG, bool RUNS>
 __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, const void* __restrict__ f2v,
-                                               float* __restrict__ out, int C, int H, int W, const float* scale)
+                                               float* __restrict__ out, int C, int H, int W, const float* scale,
+                                               int per_xcd, int blocks)
 {
     constexpr int EB = (KIND == CM_FP8) ? 1 : 2;          // bytes per element
     constexpr int ST = CmLayout<EB>::STRIDE;              // LDS pixel stride in elements
@@ -103,8 +104,24 @@ __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, con
     E (*sB)[BC][ST] = reinterpret_cast<E (*)[BC][ST]>(lds + A_BYTES);
     float (*stage)[PL][SP] = reinterpret_cast<float (*)[PL][SP]>(lds);
 
-    const int tiles = gridDim.x / G, dg = blockIdx.x / tiles;
-    const int n = blockIdx.z, h0 = blockIdx.y * CM_ROWS, w0 = blockIdx.x % tiles * CM_PX;
+    int dg, n, h0, w0;
+    if constexpr (RUNS) {   // runs of neighbouring tiles on an XCD, a tile's groups together
+        int t = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+        if (t >= blocks) return;
+        const int tiles = (W + CM_PX - 1) / CM_PX, rows = (H + CM_ROWS - 1) / CM_ROWS;
+        dg = t % G;
+        t /= G;
+        w0 = t % tiles * CM_PX;
+        t /= tiles;
+        h0 = t % rows * CM_ROWS;
+        n = t / rows;
+    } else {
+        const int tiles = gridDim.x / G;
+        dg = blockIdx.x / tiles;
+        w0 = blockIdx.x % tiles * CM_PX;
+        h0 = blockIdx.y * CM_ROWS;
+        n = blockIdx.z;
+    }
     const long long HW = (long long)H * W;
     const E* f1 = static_cast<const E*>(f1v) + (long long)n * C * HW;
     const E* f2 = static_cast<const E*>(f2v) + (long long)n * C * HW;
@@ -267,37 +284,71 @@ __device__ __forceinline__ void corr_mfma_tile(const void* __restrict__ f1v, con
 // FP8, whose staging holds less) with 3 or fewer vertical displacements a
 // block, two with more (480x272x32, FP8: 24.6 us at 4, 21.2 at 6, 19.5 at 8;
 // BF16: 32.6, 26.0, 35.0 with spills).
-template <int KIND, int MD, bool LEGACY, int DG>
+template <int KIND, int MD, bool LEGACY, int DG, bool RUNS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(DG > 3 ? 4 : KIND == CM_FP8 ? 8 : 6)))
 void k_corr_mfma(const void* __restrict__ f1, const void* __restrict__ f2, float* __restrict__ out, int C, int H, int W,
-                 const float* scale)
+                 const float* scale, int per_xcd, int blocks)
 {
-    corr_mfma_tile<KIND, MD, LEGACY, DG>(f1, f2, out, C, H, W, scale);
+    corr_mfma_tile<KIND, MD, LEGACY, DG, RUNS>(f1, f2, out, C, H, W, scale, per_xcd, blocks);
 }
 
-template <int KIND, int MD, int DG>
+template <int KIND, int MD, int DG, bool RUNS>
 static void launch_mfma_dg(const void* f1, const void* f2, float* out, int N, int C, int H, int W, bool legacy,
                            const float* scale, hipStream_t s)
 {
     dim3 grid((W + CM_PX - 1) / CM_PX * ((2 * MD + 1) / DG), (H + CM_ROWS - 1) / CM_ROWS, N);
-    if (legacy) hipLaunchKernelGGL((k_corr_mfma<KIND, MD, true, DG>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale);
-    else hipLaunchKernelGGL((k_corr_mfma<KIND, MD, false, DG>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale);
+    const int blocks = (int)(grid.x * grid.y * grid.z), per_xcd = (blocks + 7) / 8;
+    if (RUNS) grid = dim3(8 * per_xcd);
+    if (legacy)
+        hipLaunchKernelGGL((k_corr_mfma<KIND, MD, true, DG, RUNS>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale, per_xcd, blocks);
+    else
+        hipLaunchKernelGGL((k_corr_mfma<KIND, MD, false, DG, RUNS>), grid, dim3(512), 0, s, f1, f2, out, C, H, W, scale, per_xcd, blocks);
 }
 
-// Vertical displacements per block: all nine need 72 sums a lane, so one or two
-// blocks stood on a CU, each a chain of loads, products, staging and stores;
-// thirds stage half as much again but overlap three or four blocks (BF16,
-// 240x136x64: 16.7 us with nine, 13.3 with three; 213x119x64: 15.9, 13.9).  One
-// a block while all of them still fit the chip at once (30x17x196: 10.6 us with
-// one, 13.1 with three, 25.1 with nine; 121x68x96, 612 blocks of one: 10.5, 8.4, 15.2).
+// Vertical displacements per block, and the blocks' order (md = 4; T: tiles of
+// 32 x 4 pixels; us in BF16 | FP8 and pixels x channels).
+//
+// One a block while all of those still fit the chip at once: 30x17x196, T = 5,
+// 10.6 with one, 13.1 with three, 25.1 with nine.
+//
+// Above that a block with all nine needs 72 sums a lane, so two stand on a CU,
+// each a chain of loads, products, staging and stores; thirds stage half as much
+// again but overlap three or four: 240x136x64, T = 272, 16.1 | 13.2 with nine, 14.7
+// | 10.7 with three; 400x200x128, 650, 43.2 | 32.0 and 37.5 | 23.2.  Nine where they
+// fill their rounds of 512: 320x180x128, 450, 25.4 and 28.9 (FP8, whose thirds stand
+// four on a CU, 18.8 and 18.8); 480x272x64, 1020, 32.6 and 35.8 (FP8 25.2 and 24.8);
+// FP8 only with one chunk: 480x272x32 19.2 and 20.7.
+//
+// Blocks go to the XCDs in runs of neighbouring tiles, a tile's thirds together,
+// so that its f2 rows come from that XCD's L2 after the first, and the parts of a
+// line of output at two tiles' border meet there: 320x180x128 38.0 | 24.0 in rows
+// of blocks, 28.9 | 18.8 so; 213x119x64 14.3 and 11.9; 477x272x32 36.9 | 35.9 and 30.3
+// | 27.0.  Rows of whole lines (W a multiple of 16) with up to 16 channels are bound
+// by their stores and the faster in rows of blocks (320x192x8 with nine 12.3 | 11.1,
+// 12.8 | 11.8 in runs; FP8's thirds up to 32, 384x200x32 14.0 and 14.6), and a grid of
+// 8 or 16 tiles across keeps a column on an XCD in rows too (240x136x64 14.1 | 10.4 and
+// 14.7 | 10.7; from T = 384 runs are no slower).  Rows that are not take thirds, whose
+// stores meet sooner (476x272x32 26.0 | 21.6, with nine 35.1 | 27.9; 1916x1080x8 340 |
+// 346 and 411 | 389).
 template <int KIND, int MD>
 static void launch_mfma(const void* f1, const void* f2, float* out, int N, int C, int H, int W, bool legacy,
                         const float* scale, hipStream_t s)
 {
     constexpr int P = 2 * MD + 1;
-    const long long tiles = (long long)((W + CM_PX - 1) / CM_PX) * ((H + CM_ROWS - 1) / CM_ROWS) * N;
-    if (MD == 4 && tiles * P <= 256) launch_mfma_dg<KIND, MD, MD == 4 ? 1 : P>(f1, f2, out, N, C, H, W, legacy, scale, s);
-    else launch_mfma_dg<KIND, MD, P % 3 == 0 ? 3 : P>(f1, f2, out, N, C, H, W, legacy, scale, s);
+    const long long T = (long long)((W + CM_PX - 1) / CM_PX) * ((H + CM_ROWS - 1) / CM_ROWS) * N;
+    auto go = [&](auto launch) { launch(f1, f2, out, N, C, H, W, legacy, scale, s); };
+    if constexpr (MD != 4) {
+        if (T * P <= 512) go(launch_mfma_dg<KIND, MD, 1, false>);
+        else go(launch_mfma_dg<KIND, MD, P, false>);
+    } else {
+        const bool lines = W % 16 == 0, nine = lines && T >= 0.85 * 512 * ((T + 511) / 512) && (KIND != CM_FP8 || C <= CM_KC);
+        const bool near = lines && (W + CM_PX - 1) / CM_PX % 8 == 0 && T < 384;
+        // (the blocks' numbers and their threads fit 32 bits)
+        const bool runs = (!lines || C > (nine || KIND != CM_FP8 ? 16 : CM_KC)) && !near && T < (1 << 20);
+        if (T * P <= 256) go(launch_mfma_dg<KIND, MD, 1, false>);
+        else if (nine) go(runs ? launch_mfma_dg<KIND, MD, P, true> : launch_mfma_dg<KIND, MD, P, false>);
+        else go(runs ? launch_mfma_dg<KIND, MD, 3, true> : launch_mfma_dg<KIND, MD, 3, false>);
+    }
 }
 
 template <int KIND>
