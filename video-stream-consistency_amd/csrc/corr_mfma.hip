@@ -329,7 +329,9 @@ static void launch_mfma_dg(const void* f1, const void* f2, float* out, int N, in
 // 8 or 16 tiles across keeps a column on an XCD in rows too (240x136x64 14.1 | 10.4 and
 // 14.7 | 10.7; from T = 384 runs are no slower).  Rows that are not take thirds, whose
 // stores meet sooner (476x272x32 26.0 | 21.6, with nine 35.1 | 27.9; 1916x1080x8 340 |
-// 346 and 411 | 389).
+// 346 and 411 | 389), but for maps of one group of pixels (4x2000x32 13.0 | 11.9 in
+// rows, 14.7 | 13.0 in runs of thirds; 3x2000x196, read pixel by pixel, 44.5 in runs with
+// nine, 51.8 with three).
 template <int KIND, int MD>
 static void launch_mfma(const void* f1, const void* f2, float* out, int N, int C, int H, int W, bool legacy,
                         const float* scale, hipStream_t s)
@@ -338,13 +340,13 @@ static void launch_mfma(const void* f1, const void* f2, float* out, int N, int C
     const long long T = (long long)((W + CM_PX - 1) / CM_PX) * ((H + CM_ROWS - 1) / CM_ROWS) * N;
     auto go = [&](auto launch) { launch(f1, f2, out, N, C, H, W, legacy, scale, s); };
     if constexpr (MD != 4) {
-        if (T * P <= 512) go(launch_mfma_dg<KIND, MD, 1, false>);
+        if (MD >= 2 && T * P <= 512) go(launch_mfma_dg<KIND, MD, 1, false>);
         else go(launch_mfma_dg<KIND, MD, P, false>);
     } else {
-        const bool lines = W % 16 == 0, nine = lines && T >= 0.85 * 512 * ((T + 511) / 512) && (KIND != CM_FP8 || C <= CM_KC);
-        const bool near = lines && (W + CM_PX - 1) / CM_PX % 8 == 0 && T < 384;
+        const bool lines = W % 16 == 0 || W <= 4, nine = lines && T >= 0.85 * 512 * ((T + 511) / 512) && (KIND != CM_FP8 || C <= CM_KC);
+        const bool near = W == 4 || (lines && (W + CM_PX - 1) / CM_PX % 8 == 0 && T < 384);
         // (the blocks' numbers and their threads fit 32 bits)
-        const bool runs = (!lines || C > (nine || KIND != CM_FP8 ? 16 : CM_KC)) && !near && T < (1 << 20);
+        const bool runs = (!lines || W < 4 || C > (nine || KIND != CM_FP8 ? 16 : CM_KC)) && !near && T < (1 << 20);
         if (T * P <= 256) go(launch_mfma_dg<KIND, MD, 1, false>);
         else if (nine) go(runs ? launch_mfma_dg<KIND, MD, P, true> : launch_mfma_dg<KIND, MD, P, false>);
         else go(runs ? launch_mfma_dg<KIND, MD, 3, true> : launch_mfma_dg<KIND, MD, 3, false>);
