@@ -203,7 +203,11 @@ static void launch_corr_f32(const float* f1, const float* f2, float* out, int N,
                             hipStream_t s)
 {
     constexpr int P = 2 * MD + 1;
-    const long long T = (long long)((W + 31) / 32) * ((H + CF_TH - 1) / CF_TH) * N;
+    const long long rows = (long long)((H + CF_TH - 1) / CF_TH) * N;
+    long long T = (W + 31) / 32 * rows;
+    // a map of one or two 8-pixel tiles across counts those, a quarter each (4x500x196, 63
+    // tiles of 32 or 16 of 8: 32.8 us as the former, 14.0 as the latter)
+    if (W <= 16 && T <= 120) T = ((W + 7) / 8 * rows + 3) / 4;
     if constexpr (MD == 4) {
         if (36 * T <= 256) launch_corr_f32_q<MD, 1, 1, 3, 64>(f1, f2, out, N, C, H, W, legacy, s);
         else if (12 * T <= 256) launch_corr_f32_q<MD, 1, 3, 3, 40>(f1, f2, out, N, C, H, W, legacy, s);
