@@ -528,14 +528,16 @@ __global__ __launch_bounds__(256) void k_fp8_scales(const uint32_t* mx1, const u
 }
 
 // Both tensors (blockIdx.y), 4 neighbouring pixels of a plane per thread, loaded
-// and stored together whatever their alignment; blockIdx.x = plane * chunks + chunk
+// and stored together whatever their alignment; blockIdx.x = (plane - first) * chunks + chunk
 __global__ __launch_bounds__(256) void k_fp8_quant(const float* f1, const float* f2, uint8_t* q1, uint8_t* q2,
-                                                   const float* r, const float* sc, int C, long long HW, int chunks)
+                                                   const float* r, const float* sc, int C, long long HW, int chunks,
+                                                   long long first)
 {
     typedef float F4U __attribute__((ext_vector_type(4), aligned(4)));
     typedef uint32_t U1 __attribute__((aligned(1)));
-    const long long pl = blockIdx.x / chunks;
-    const long long i = ((long long)(blockIdx.x - pl * chunks) * 256 + threadIdx.x) * 4;
+    const unsigned slot = blockIdx.x / chunks;
+    const long long pl = first + slot;
+    const long long i = ((long long)(blockIdx.x - slot * chunks) * 256 + threadIdx.x) * 4;
     if (i >= HW) return;
     const bool second = blockIdx.y != 0;
     const float rc = r[pl % C], s = sc[second ? 2 : 1];
@@ -573,7 +575,7 @@ static int quantize_fp8_pair(const float* f1, const float* f2, uint8_t* q1, uint
 {
     if (!f1 || !f2 || !q1 || !q2 || !scale) return set_error(VSC_E_INVALID, "vsc_quantize_fp8_pair: null pointer");
     if (N < 1 || C < 1 || H < 1 || W < 1) return set_error(VSC_E_INVALID, "vsc_quantize_fp8_pair: empty tensor");
-    const long long HW = (long long)H * W, n = (long long)N * C * HW;
+    const long long HW = (long long)H * W, planes = (long long)N * C;
     // workspace: 2*C maxima + C equalisation factors + 3 scales
     void* ws = workspace;
     int rc;
@@ -587,9 +589,12 @@ static int quantize_fp8_pair(const float* f1, const float* f2, uint8_t* q1, uint
     const unsigned gx = (unsigned)std::min<long long>((HW + 4095) / 4096, 16);
     hipLaunchKernelGGL(k_chan_absmax, dim3(2 * gx, C, N), dim3(256), 0, s, f1, f2, mx, C, HW);
     hipLaunchKernelGGL(k_fp8_scales, dim3(1), dim3(256), 0, s, mx, mx + C, r, sc, scale, C);
+    // (a launch holds fewer than 2^32 threads along a dimension: many small planes take several)
     const int chunks = (int)((HW + 1023) / 1024);
-    hipLaunchKernelGGL(k_fp8_quant, dim3((unsigned)((long long)N * C * chunks), 2), dim3(256), 0, s, f1, f2, q1, q2, r, sc, C, HW,
-                       chunks);
+    const long long most = std::max(1LL, (1LL << 23) / chunks);
+    for (long long first = 0; first < planes; first += most)
+        hipLaunchKernelGGL(k_fp8_quant, dim3((unsigned)(std::min(most, planes - first) * chunks), 2), dim3(256), 0, s, f1, f2, q1, q2,
+                           r, sc, C, HW, chunks, first);
     rc = check_launch("vsc_quantize_fp8_pair");
     if (workspace) return rc;
     const int rc2 = check_hip(hipFreeAsync(ws, s), "vsc_quantize_fp8_pair workspace free");
