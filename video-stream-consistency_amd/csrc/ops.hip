@@ -3,6 +3,7 @@
 // shape contract of src/ort_custom_ops.
 #include "vsc_internal.h"
 
+#include <algorithm>
 #include <string>
 
 namespace vsc {
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(256) void k_corr_generic(const T* __restrict__ f1, 
     const int P = 2 * md + 1;
     const long long HW = (long long)H * W;
     const long long total = (long long)N * P * P * HW;
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long i = ((long long)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= total) return;
     const int w = (int)(i % W);
     const int h = (int)((i / W) % H);
@@ -170,6 +171,17 @@ __global__ __launch_bounds__(256) void k_corr_generic(const T* __restrict__ f1, 
         for (int c = 0; c < C; ++c) acc += a[c * HW] * b[c * HW];
     }
     out[i] = LEGACY ? acc / (T)C : acc;
+}
+
+template <typename T>
+static void launch_corr_generic(const T* f1, const T* f2, T* out, int N, int C, int H, int W, int md, bool legacy, hipStream_t s)
+{
+    // (a launch holds fewer than 2^32 threads along a dimension)
+    const long long blocks = ((long long)N * (2 * md + 1) * (2 * md + 1) * H * W + 255) / 256;
+    const unsigned across = (unsigned)(blocks < (1 << 22) ? blocks : 1 << 22);
+    const dim3 grid(across, (unsigned)((blocks + across - 1) / across));
+    if (legacy) hipLaunchKernelGGL((k_corr_generic<T, true>), grid, dim3(256), 0, s, f1, f2, out, N, C, H, W, md);
+    else hipLaunchKernelGGL((k_corr_generic<T, false>), grid, dim3(256), 0, s, f1, f2, out, N, C, H, W, md);
 }
 
 template <int MD, int QX, int DG, int XS, int CCT>
@@ -244,14 +256,14 @@ template <> struct Pair2<double> { typedef double V __attribute__((ext_vector_ty
 // A block takes 2^BITS columns, or 2^narrow of a map that is no wider (BITS = 0).
 template <typename T, bool PAIR, int BITS>
 __global__ __launch_bounds__(256) void k_warp(const T* __restrict__ in, const T* __restrict__ flow, T* __restrict__ out,
-                                              int C, int H, int W, int narrow)
+                                              int C, int H, int W, int narrow, int first)
 {
     const int bits = BITS ? BITS : narrow;
     const int tiles = (W + (1 << bits) - 1) >> bits;
     const int x = (blockIdx.x % tiles << bits) + (threadIdx.x & ((1 << bits) - 1));
     const int y = blockIdx.y * (256 >> bits) + (threadIdx.x >> bits);
     const int n = blockIdx.z;
-    const int c0 = blockIdx.x / tiles * WG_CH;
+    const int c0 = first + blockIdx.x / tiles * WG_CH;
     const int c1 = min(C, c0 + WG_CH);
     if (x >= W || y >= H) return;
     const long long HW = (long long)H * W;
@@ -345,8 +357,14 @@ static void launch_warp(const T* in, const T* flow, T* out, int N, int C, int H,
     int bits = 2;
     while (bits < 6 && (1 << bits) < W) ++bits;
     const int cols = 1 << bits, rows = 256 >> bits;
-    const dim3 grid((W + cols - 1) / cols * ((C + WG_CH - 1) / WG_CH), (H + rows - 1) / rows, N);
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, flow, out, C, H, W, bits); };
+    const int tiles = (W + cols - 1) / cols;
+    // (a launch holds fewer than 2^32 threads along a dimension: the channels in several where they need more)
+    const int most = std::max(1, (1 << 23) / tiles) * WG_CH;
+    auto go = [&](auto kernel) {
+        for (int first = 0; first < C; first += most)
+            hipLaunchKernelGGL(kernel, dim3(tiles * ((std::min(most, C - first) + WG_CH - 1) / WG_CH), (H + rows - 1) / rows, N),
+                               dim3(256), 0, s, in, flow, out, C, H, W, bits, first);
+    };
     if (W > 32) go(k_warp<T, true, 6>);
     else if (W > 1) go(k_warp<T, true, 0>);
     else go(k_warp<T, false, 0>);
@@ -378,25 +396,13 @@ int correlation_forward(const void* f1, const void* f2, void* out, int N, int C,
             case 2: launch_corr_f32<2>(a, b, o, N, C, H, W, legacy, s); break;
             case 3: launch_corr_f32<3>(a, b, o, N, C, H, W, legacy, s); break;
             case 4: launch_corr_f32<4>(a, b, o, N, C, H, W, legacy, s); break;
-            default: {
-                const long long total = (long long)N * (2 * md + 1) * (2 * md + 1) * H * W;
-                const dim3 g((unsigned)((total + 255) / 256));
-                if (legacy) hipLaunchKernelGGL((k_corr_generic<float, true>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
-                else hipLaunchKernelGGL((k_corr_generic<float, false>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
-            }
+            default: launch_corr_generic(a, b, o, N, C, H, W, md, legacy, s);
         }
         return check_launch("correlation f32");
     }
     if (in_dtype == VSC_F64) {
-        const long long total = (long long)N * (2 * md + 1) * (2 * md + 1) * H * W;
-        const dim3 g((unsigned)((total + 255) / 256));
-        const double* a = static_cast<const double*>(f1);
-        const double* b = static_cast<const double*>(f2);
-        double* o = static_cast<double*>(out);
-        if (legacy)
-            hipLaunchKernelGGL((k_corr_generic<double, true>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
-        else
-            hipLaunchKernelGGL((k_corr_generic<double, false>), g, dim3(256), 0, s, a, b, o, N, C, H, W, md);
+        launch_corr_generic(static_cast<const double*>(f1), static_cast<const double*>(f2), static_cast<double*>(out), N, C, H, W, md,
+                            legacy, s);
         return check_launch("correlation f64");
     }
     if (in_dtype == VSC_BF16 || in_dtype == VSC_F16 || in_dtype == VSC_FP8E4M3) {
