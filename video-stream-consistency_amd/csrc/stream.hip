@@ -10,7 +10,6 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <vector>
 
 using namespace vsc;
 
@@ -79,7 +78,7 @@ size_t footprint(int W, int H, int fw, int fh, int* nlev_out = nullptr)
 {
     int lw[VSC_MAX_LEVELS], lh[VSC_MAX_LEVELS];
     const int n = level_dims(W, H, lw, lh);
-    size_t bytes = 0;
+    size_t bytes = RESIDENT_CTL_BYTES;   // the resident solver's control words, behind the pieces
     for (int j = 0; j < n; ++j) bytes += 8 * piece_bytes((size_t)3 * lw[j] * lh[j]);
     if (fw != W || fh != H) bytes += 2 * piece_bytes((size_t)3 * W * H);
     if (nlev_out) *nlev_out = n;
@@ -231,8 +230,7 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
     s->fh = flow_height;
     s->bytes = footprint(width, height, flow_width, flow_height, &s->nlev);
     level_dims(width, height, s->lw, s->lh);
-    // (the solver's control words stand behind the carved pieces)
-    int rc = check_hip(hipMalloc(&s->block, s->bytes + RESIDENT_CTL_BYTES), "vsc_stream_create");
+    int rc = check_hip(hipMalloc(&s->block, s->bytes), "vsc_stream_create");
     if (rc) {
         delete s;
         return rc;
@@ -258,6 +256,8 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
         s->flow_up[0] = take((size_t)3 * width * height);
         s->flow_up[1] = take((size_t)3 * width * height);
     }
+    unsigned* ctl = reinterpret_cast<unsigned*>(p);
+    p += RESIDENT_CTL_BYTES;
     if ((size_t)(p - static_cast<char*>(s->block)) != s->bytes) {
         (void)hipFree(s->block);
         delete s;
@@ -265,11 +265,10 @@ extern "C" int vsc_stream_create(int width, int height, int flow_width, int flow
     }
     // without these the blocked solver runs alone
     int dev = -1;
-    static const std::vector<unsigned> zeros(RESIDENT_CTL_BYTES / 4, 0u);
-    unsigned* ctl = reinterpret_cast<unsigned*>(static_cast<char*>(s->block) + s->bytes);
+    static const unsigned zeros[RESIDENT_CTL_BYTES / 4] = {};
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipMemcpy(ctl, zeros.data(), RESIDENT_CTL_BYTES, hipMemcpyHostToDevice) == hipSuccess) {
+        hipMemcpy(ctl, zeros, RESIDENT_CTL_BYTES, hipMemcpyHostToDevice) == hipSuccess) {
         s->ctl = ctl;
         s->note = notes.take();
     } else {
