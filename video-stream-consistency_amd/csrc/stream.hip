@@ -13,6 +13,30 @@
 
 using namespace vsc;
 
+// Frames that the blocked solver takes after a resident launch that the device
+// could not hold at once: 64, doubled with each further one up to 4096, halved
+// after as many resident frames without one, so that a rare one costs 64 again.
+struct Pause {
+    int left = 0, length = 0, good = 0;
+    bool resident(bool given_up)
+    {
+        if (given_up) {
+            length = std::min(4096, std::max(64, 2 * length));
+            left = length;
+            good = 0;
+        }
+        if (left > 0) {
+            --left;
+            return false;
+        }
+        if (length > 0 && ++good >= length) {
+            length = length > 64 ? length / 2 : 0;
+            good = 0;
+        }
+        return true;
+    }
+};
+
 struct vsc_stream {
     int W = 0, H = 0, fw = 0, fh = 0;
     int nlev = 0;                      // pyramid levels allocated (<= VSC_MAX_LEVELS)
@@ -29,11 +53,12 @@ struct vsc_stream {
     void* block = nullptr;
     size_t bytes = 0;
     // resident solver (resident.hip): control words, the host word that tells
-    // of a launch the device could not hold at once, and how many frames the
-    // blocked solver takes after one
+    // of a launch the device could not hold at once, and the frames that the blocked
+    // solver takes after one
     unsigned* ctl = nullptr;
     volatile unsigned* note = nullptr;
-    int cus = 0, skip = 0, backoff = 0;
+    int cus = 0;
+    Pause pause;
     bool shared = false;
     int resident_levels = 0;   // of the last frame
     // the HIP stream of its frames, and the end of the last one that was marked
@@ -433,19 +458,13 @@ bool whole_device(hipStream_t st, int cus)
 // Whether this frame's levels may use the resident solver: not beside other
 // work on purpose, not under capture (its launches take turns across streams),
 // not on a stream that leaves CUs out, and not for some frames after the device
-// could not hold a launch at once (64, doubled each time up to 4096).
+// could not hold a launch at once.
 bool resident_frame(vsc_stream* s, const vsc_params& p, hipStream_t st)
 {
     if (!s->note || s->shared || !std::isfinite(p.mom_fac)) return false;
-    if (*s->note) {
-        *s->note = 0u;
-        s->backoff = std::min(4096, std::max(64, 2 * s->backoff));
-        s->skip = s->backoff;
-    }
-    if (s->skip > 0) {
-        --s->skip;
-        return false;
-    }
+    const bool given_up = *s->note != 0u;
+    if (given_up) *s->note = 0u;
+    if (!s->pause.resident(given_up)) return false;
     return whole_device(st, s->cus);
 }
 
@@ -784,6 +803,14 @@ extern "C" int vsct_resident_give_up(vsc_stream* s, vsc_hip_stream stream)
     static const unsigned one = 1u;
     if (check_hip(hipMemcpyAsync(s->ctl, &one, 4, hipMemcpyHostToDevice, as_stream(stream)), "vsct_resident_give_up")) return 0;
     return check_hip(hipStreamSynchronize(as_stream(stream)), "vsct_resident_give_up") ? 0 : 1;
+}
+
+// Diagnostic (no declaration in vsc.h): n frames of a new stream, given_up[i]
+// whether a launch was given up before frame i; resident[i]: what the frame takes.
+extern "C" void vsct_resident_pause(const unsigned char* given_up, int n, unsigned char* resident)
+{
+    Pause p;
+    for (int i = 0; i < n; ++i) resident[i] = p.resident(given_up[i] != 0);
 }
 
 // Diagnostic (no declaration in vsc.h): the levels of the stream's last fused
