@@ -429,9 +429,10 @@ extern "C" int vsc_correlation_forward_noalloc(const void* f1, const void* f2, v
                             ? 0
                             : corr_mfma_workspace_bytes(N, C, H, W, in_dtype);
     if (need > VSC_CORRELATION_STATIC_SCRATCH)
-        return set_error(VSC_E_INVALID, "vsc_correlation_forward_noalloc: the operands need " + std::to_string(need) +
-                                            " bytes of scratch, more than the static " +
-                                            std::to_string((size_t)VSC_CORRELATION_STATIC_SCRATCH));
+        return set_error(VSC_E_INVALID,
+                         "vsc_correlation_forward_noalloc: operands of a width that is no multiple of 4, or unaligned, are taken up "
+                         "to a vsc_correlation_workspace_size() of " + std::to_string((size_t)VSC_CORRELATION_STATIC_SCRATCH) +
+                         ", these have " + std::to_string(need) + " (no scratch is used: vsc_correlation_forward takes any)");
     return correlation_forward(f1, f2, out, N, C, H, W, max_displacement, legacy, in_dtype, chan_scale, stream);
 }
 
@@ -449,7 +450,7 @@ extern "C" int vsc_correlation_forward_ws(const void* f1, const void* f2, void* 
         corr_mfma_asks_workspace(f1, f2, W, in_dtype) ? vsc_correlation_workspace_size(N, C, H, W, in_dtype) : 0;
     if (need && (!workspace || workspace_bytes < need))
         return set_error(VSC_E_INVALID, "vsc_correlation_forward_ws: workspace missing or smaller than "
-                                        "vsc_correlation_workspace_size()");
+                                        "vsc_correlation_workspace_size() (vsc_correlation_forward takes the operands without one)");
     return correlation_forward(f1, f2, out, N, C, H, W, max_displacement, legacy, in_dtype, chan_scale, stream);
 }
 
