@@ -99,7 +99,7 @@ __device__ inline void conv_load4(const void* src, long long off, float v[4], in
     for (int r = 0; r < 4; ++r) v[r] += (r < nvalid) ? E::ld(p[r]) : 0.0f;
 }
 
-template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX>
+template <int EK, int EKO, int S, int NT, int MR, int NW, int KCX, bool EARLY>
 __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 {
     using E = Elem<EK>;
@@ -135,19 +135,21 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 #pragma unroll
         for (int m = 0; m < MR; ++m) acc[i][m] = cv_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // the epilogue's per-channel values, read before the products (after them
-    // the read was one more round trip to memory on every launch's tail: the
-    // 1080p network's level-3 layers 13.5 us a launch, now 12.2)
-    float bias[NT / 16][4];
+    // the epilogue's per-channel values, read before the products unless not EARLY
+    // (after them the read is one more round trip to memory on every launch's tail:
+    // 240x136x2, 64 -> 64, BF16, 17.0 us, 14.9 so)
+    [[maybe_unused]] float bias[NT / 16][4];
     const float g = a.gate ? *a.gate : 1.0f;
     const bool with_bias = a.bias;
+    if constexpr (EARLY) {
 #pragma unroll
-    for (int i = 0; i < NT / 16; ++i)
+        for (int i = 0; i < NT / 16; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int co = nt0 + i * 16 + 4 * lg + r;
-            bias[i][r] = with_bias ? a.bias[min(co, a.Cout - 1)] : 0.0f;
-        }
+            for (int r = 0; r < 4; ++r) {
+                const int co = nt0 + i * 16 + 4 * lg + r;
+                bias[i][r] = with_bias ? a.bias[min(co, a.Cout - 1)] : 0.0f;
+            }
+    }
 
     // input channel chunks are staged through registers DEPTH chunks ahead of
     // the chunk in LDS, so the global loads of a chunk overlap the MFMAs of the
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float x = acc[i][m][r];
-                if (with_bias && r < nv) x += bias[i][r];
+                if (with_bias && r < nv) x += EARLY ? bias[i][r] : a.bias[co + r];
                 if (a.act == 1) x = x > 0.0f ? x : x * 0.1f;
                 else if (a.act == 2) x = x > 0.0f ? x : 0.0f;
                 v[r] = a.gate ? x * g : x;
@@ -507,7 +509,18 @@ static void conv_go(const ConvArgs& a, hipStream_t s)
     b.tiles_y = (hs + NW * MR - 1) / (NW * MR);
     b.tiles_x = (ws + 15) / 16;
     dim3 grid(b.tiles_x * b.tiles_y * ps * ps, (a.Cout + NT - 1) / NT, a.N);
-    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX>), grid, dim3(64 * NW), 0, s, b);
+    // The registers of an early bias cost several FP32 tiles a block of their CU: not
+    // without a bias (400x200, stride 2, 32 -> 32, two items, 14.9 us, 14.0 without), nor
+    // where three blocks a CU instead of four need a round more (480x272, 32 -> 32, 1020
+    // blocks: 37.3 us with three, 31.3 with four; 320x256, 640 blocks: 20.8 and 22.1).
+    if constexpr (EK == EK_F32 && NT <= 32) {
+        const long long n = (long long)grid.x * grid.y * grid.z;
+        if (!a.bias || (NT == 32 && MR == 3 - S && (n + 1023) / 1024 < (n + 767) / 768)) {
+            hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, false>), grid, dim3(64 * NW), 0, s, b);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_conv3x3<EK, EKO, S, NT, MR, NW, KCX, true>), grid, dim3(64 * NW), 0, s, b);
 }
 
 template <int EK, int EKO, int S, int NT, int MR>
