@@ -235,7 +235,21 @@ int vsc_float_to_rgba(vsc_image in, uint8_t* rgba, vsc_hip_stream stream);
  * the Qt frame lists.  Owns the device-resident, double-buffered state (the
  * previous stabilized frame and every intermediate image); nothing is
  * allocated per frame.  One vsc_stream may be driven by one host thread at a
- * time; different streams are independent.                                 */
+ * time; the results of different streams are independent of each other.
+ *
+ * Their timing is not quite.  A frame's solver keeps its levels resident on the
+ * chip where that is the faster form.  Such launches need all of their blocks on
+ * the device at once, so those of one process and device take turns, whatever
+ * HIP streams they are on; frames too small to fill the chip (below 600000
+ * pixels, 200000 in reference order) leave that form to run side by side when
+ * another vsc_stream's frame is under way on another HIP stream, and for 64
+ * frames after.  Kernels of another process may hold the device's CUs: a
+ * resident launch waits at most 3 ms at a time, the frame is then completed without
+ * it, and the stream does without the resident form for 64 frames, twice as many
+ * at each further time (up to 4096), half as many again after as many frames
+ * that went well.  Frames under stream capture, of pipelines with overlap = 1 and
+ * of servers, and those on hipStreamLegacy, hipStreamPerThread or a stream with a
+ * CU mask never take it.  Every form gives the same bits.                      */
 typedef struct vsc_stream vsc_stream;
 
 /* flow_width/flow_height: resolution the flows arrive at (== width/height,
@@ -270,7 +284,7 @@ typedef struct {
     int flow_channels;
 } vsc_frame_in;
 
-#define VSC_FRAME_FUSED 0     /* fused front pass + temporally blocked solver */
+#define VSC_FRAME_FUSED 0     /* fused front pass + resident or temporally blocked solver */
 #define VSC_FRAME_STAGED 1    /* one launch per reference stage (parity aid) */
 #define VSC_FRAME_FMA 2       /* as FUSED, solver update in FMA form: per-pixel
                                  constants q = cnt + w, k = step*(lapP - w*A) and
@@ -324,8 +338,8 @@ int vsc_conv3x3_nhwc(const void* in, int in_cs, int in_c0, int N, int H, int W, 
  * frames by nearest sampling to round(W/f) x round(H/f) before the network;
  * the flow is then produced at that size (flowmodel.cpp:126-133).
  * dtype: VSC_F32 (plain form) or VSC_BF16 (BF16 storage and MFMA operands,
- * FP32 accumulation).  The extractor and the decoders have scratch of their
- * own: an extraction and a decode may run at once on two streams when the
+ * FP32 accumulation).  The extractor and the decoders share no buffer but the
+ * slots: an extraction and a decode may run at once on two streams when the
  * extraction writes none of the slots the decode reads (two extractions, or
  * two decodes, of one network may not).                                    */
 typedef struct vsc_flownet vsc_flownet;
@@ -445,7 +459,10 @@ typedef struct {
                                    frames' features of a call while the previous call decodes.  Frame t's
                                    outputs are then ordered on the caller's stream by the call for
                                    frame t+1 (or vsc_pipeline_sync), and the window frames of call t
-                                   must stay unchanged until then.  Same results as 0. */
+                                   must stay unchanged until then.  Same results as 0.  A frame alone
+                                   on its device (0) uses the resident solver, overlapped ones the
+                                   blocked one: measure both (1080p, BF16 network at downscale 2: one
+                                   frame a call with 0 is as fast as two a call with 1, without its lag) */
     int flow_batch;             /* B, 1..4: the most frames whose flows vsc_pipeline_frames computes in
                                    one batched network decode (the reference's batchSize: FlowModel::run
                                    over B frame pairs every B frames, videostabilizer.cpp:65-71,177,

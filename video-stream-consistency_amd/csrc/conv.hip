@@ -153,8 +153,8 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(ConvArgs a)
 
     // input channel chunks are staged through registers DEPTH chunks ahead of
     // the chunk in LDS, so the global loads of a chunk overlap the MFMAs of the
-    // DEPTH chunks before it (deeper staging measured slower: 2 and 3 chunks
-    // ahead cost the 1080p BF16 network 3% and 18%)
+    // DEPTH chunks before it (deeper staging measured slower: with all of the flow
+    // network on this kernel 2 and 3 chunks ahead cost its 1080p BF16 form 3% and 18%)
     constexpr int DEPTH = 1;
     cv_u32x4 rp[DEPTH][RP], rw[DEPTH][RW];
     auto fetch = [&](int c0, cv_u32x4 (&P)[RP], cv_u32x4 (&Wr)[RW]) {
@@ -589,11 +589,13 @@ static void conv_mr(const ConvArgs& a, int mr, hipStream_t s)
     else conv_go<EK, EKO, S, NT, 1, 4, KCX>(a, s);
 }
 
-// Tile choice.  Channel tile: FP32 layers take the widest tile they fill (64,
-// 32 or 16 output channels); 16-bit layers take 32 (16 when the layer has at
-// most 16): twice the blocks of 64-channel tiles on the small grids of the
-// coarse levels and half the weights staged per block (1080p frames: 556 vs
-// 521 frames/s on one stream, 670 vs 656 frame-pipelined).  Pixel tile:
+// Tile choice of k_conv3x3; packed layers choose theirs by modelled time
+// (conv_packed) and take only the grouping of their sums from here (conv_flush).
+// Channel tile: FP32 layers take the widest tile they fill (64, 32 or 16 output
+// channels); 16-bit layers take 32 (16 when the layer has at most 16): twice the
+// blocks of 64-channel tiles on small grids and half the weights staged per block
+// (with all of the flow network on this kernel 1080p frames ran at 556 frames/s,
+// with 64-channel tiles at 521).  Pixel tile:
 // 256 pixels from two blocks per CU; 128 pixels from two blocks per CU (FP32)
 // or from half a block per CU (16-bit: its MFMAs are 16x faster, so the weights
 // every block re-reads dominate, and halving that traffic pays for the idle
