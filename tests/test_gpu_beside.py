@@ -71,3 +71,48 @@ def test_stabilizers_on_one_stream_stay_resident(cuda):
     torch.cuda.synchronize()
     a.st.close()
     b.st.close()
+
+
+@pytest.mark.parametrize("threads", [False, True])
+@pytest.mark.parametrize("capture_mode", [0, 1, 2])
+def test_asking_for_others_leaves_a_capture_whole(cuda, capture_mode, threads):
+    """The frames' marks and queries while a third stream is captured, by the thread
+    that captures and by another."""
+    import ctypes
+    import threading
+    import torch
+    vsc = importlib.import_module("video-stream-consistency_amd")
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    a = Stab(vsc, cuda, 1920, 1080, 2, torch.cuda.Stream())
+    b = Stab(vsc, cuda, 320, 180, 2, torch.cuda.Stream())
+    ref = Stab(vsc, cuda, 320, 180, 2, b.stream)
+    torch.cuda.synchronize()
+    for s in (a, b):
+        s.frame()
+    torch.cuda.synchronize()
+    c, graph = torch.cuda.Stream(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(ctypes.c_void_p(c.cuda_stream), capture_mode) == 0
+
+    def frames():
+        for _ in range(10):
+            a.frame()
+            b.frame()
+
+    try:
+        if threads:
+            t = threading.Thread(target=frames)
+            t.start()
+            t.join()
+        else:
+            frames()
+    finally:
+        end = hip.hipStreamEndCapture(ctypes.c_void_p(c.cuda_stream), ctypes.byref(graph))
+        hip.hipGraphDestroy(graph)
+    assert end == 0
+    torch.cuda.synchronize()
+    for _ in range(11):
+        ref.frame()
+        torch.cuda.synchronize()
+    assert torch.equal(b.out, ref.out)
+    for s in (a, b, ref):
+        s.st.close()

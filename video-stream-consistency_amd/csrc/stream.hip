@@ -184,17 +184,21 @@ bool beside_others(vsc_stream* s, hipStream_t st)
         --s->hold;
         return true;
     }
-    for (vsc_stream* o = d.first; o; o = o->next) {
+    // (in a thread whose mode is not relaxed the query would end a capture under way elsewhere)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    for (vsc_stream* o = d.first; o && !s->hold; o = o->next) {
         if (o == s || !o->under_way || o->on == st) continue;
         const hipError_t e = hipEventQuery(o->done);
         if (e != hipSuccess) (void)hipGetLastError();
-        if (e == hipErrorNotReady) {
-            s->hold = 64;
-            return true;
-        }
-        o->under_way = false;
+        if (e == hipErrorNotReady) s->hold = 64;
+        else o->under_way = false;
     }
-    return false;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return s->hold > 0;
 }
 
 // Marks a frame's end for the others' beside_others: only where another
